@@ -20,11 +20,21 @@
 // division by the sum (softmax) or by the standard deviation (layer norm) is
 // one IEEE reciprocal per row times a multiply per element (<= 1.5 ulp).
 // The CPU kernels divide per element; both stay far inside the 1e-4 parity
-// bound.  Rows whose width is not a multiple of 4, or wider
-// than 8192, go through a looped wave-per-row kernel that re-reads the row.
+// bound.
+//
+// Rows whose width is not a multiple of 4 (a 50257-word vocabulary), or whose
+// tensors start off a 16-byte boundary, take the same kernels in their ODD
+// form: the row still moves as 16-byte vectors, now at 4-byte alignment
+// (which global loads and stores allow), and its last cols % 4 elements sit
+// one each in the first threads.  Bound by HBM like the aligned rows:
+// [1024, 50257] cross entropy 35 us and its backward 85 us (4.9 TB/s; 79 us
+// at 50256 columns), against 565 and 788 us for a wave per row re-reading it
+// in 4-byte loads; [4096, 8191] softmax 47 us (46 at 8192).  Only rows too
+// wide for the registers (53248 columns) are read more than once.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
+#include <type_traits>
 
 #include "launch.hpp"
 #include "wave.h"
@@ -36,8 +46,86 @@ namespace {
 
 constexpr int kRowsPerBlock = 4;  // one row per wave, 4 waves per block
 
+typedef float cl_f4u __attribute__((ext_vector_type(4), aligned(4)));
+
+// Vector c of a row: ODD rows start at any 4-byte address.
+template <bool ODD>
+__device__ __forceinline__ cl_f4 row_load(const float *row, int c) {
+    if constexpr (ODD) return __builtin_nontemporal_load(reinterpret_cast<const cl_f4u *>(row) + c);
+    else return __builtin_nontemporal_load(reinterpret_cast<const cl_f4 *>(row) + c);
+}
+
+template <bool ODD>
+__device__ __forceinline__ void row_store(float *row, int c, cl_f4 v) {
+    if constexpr (ODD) __builtin_nontemporal_store((cl_f4u)v, reinterpret_cast<cl_f4u *>(row) + c);
+    else __builtin_nontemporal_store(v, reinterpret_cast<cl_f4 *>(row) + c);
+}
+
 __device__ __forceinline__ float fast_exp(float x) {
     return __builtin_amdgcn_exp2f(x * 1.44269504088896341f);
+}
+
+// exp(x) for x <= 0 to about 1.5 ulp: the rounding of x * log2(e) and the
+// part of log2(e) past f32 go back in as a first-order factor.  Below -200
+// (the result is 0 in f32 either way) x is held there, so -inf and the
+// lowest f32 give 0 and not inf - inf; a NaN stays one.
+__device__ __forceinline__ float close_exp(float x) {
+    x = x < -200.0f ? -200.0f : x;
+    const float t = x * 0x1.715476p+0f;
+    const float lo = __builtin_fmaf(x, 0x1.4ae0cp-26f, __builtin_fmaf(x, 0x1.715476p+0f, -t));
+    const float p = __builtin_amdgcn_exp2f(t);
+    return __builtin_fmaf(p, lo * 0.693147180559945f, p);
+}
+
+// The softmax's exponential and final division.  Aligned rows: the hardware
+// 2^x and a multiply by the row's reciprocal.  ODD rows: close_exp and the
+// IEEE quotient (the reciprocal times e, corrected by one FMA remainder), no
+// less precise than the expf and the division a row of any other width used
+// to get; the extra operations hide behind HBM.
+template <bool ODD>
+__device__ __forceinline__ float row_exp(float x) {
+    if constexpr (ODD) return close_exp(x);
+    else return fast_exp(x);
+}
+
+template <bool ODD>
+__device__ __forceinline__ float row_div(float e, float s, float inv) {
+    const float q = e * inv;
+    if constexpr (ODD) return __builtin_fmaf(__builtin_fmaf(-q, s, e), inv, q);
+    else return q;
+}
+
+template <bool ODD>
+__device__ __forceinline__ cl_f4 row_exp4(cl_f4 v, float m) {
+    return (cl_f4){row_exp<ODD>(v.x - m), row_exp<ODD>(v.y - m), row_exp<ODD>(v.z - m),
+                   row_exp<ODD>(v.w - m)};
+}
+
+template <bool ODD>
+__device__ __forceinline__ cl_f4 row_div4(cl_f4 e, float s, float inv) {
+    return (cl_f4){row_div<ODD>(e.x, s, inv), row_div<ODD>(e.y, s, inv), row_div<ODD>(e.z, s, inv),
+                   row_div<ODD>(e.w, s, inv)};
+}
+
+// d / sd of the layer norm, rsd = 1 / sd: a multiply, in ODD rows corrected
+// to the quotient by one FMA remainder (what their division gave).  sdc is sd,
+// or 0 where sd overflowed and rsd is 0, so that the remainder stays finite.
+template <bool ODD>
+__device__ __forceinline__ float row_norm(float d, float sdc, float rsd) {
+    const float q = d * rsd;
+    if constexpr (ODD) return __builtin_fmaf(__builtin_fmaf(-q, sdc, d), rsd, q);
+    else return q;
+}
+
+template <bool ODD>
+__device__ __forceinline__ cl_f4 row_norm4(cl_f4 d, float sdc, float rsd) {
+    return (cl_f4){row_norm<ODD>(d.x, sdc, rsd), row_norm<ODD>(d.y, sdc, rsd),
+                   row_norm<ODD>(d.z, sdc, rsd), row_norm<ODD>(d.w, sdc, rsd)};
+}
+
+// exp of a whole vector, the hardware form (the losses).
+__device__ __forceinline__ cl_f4 fast_exp4(cl_f4 v, float m) {
+    return (cl_f4){fast_exp(v.x - m), fast_exp(v.y - m), fast_exp(v.z - m), fast_exp(v.w - m)};
 }
 
 // x / y correctly rounded, for a y shared by many x, from r = 1 / y (IEEE):
@@ -51,7 +139,7 @@ __device__ __forceinline__ float div_exact(float x, float y, float r) {
     return __builtin_isfinite(q0) ? q1 : q0;
 }
 
-template <int VPT>
+template <int VPT, bool ODD>
 __global__ void __launch_bounds__(256) softmax_wave_kernel(const float *__restrict__ x,
                                                            float *__restrict__ y, int rows,
                                                            int cols) {
@@ -59,16 +147,18 @@ __global__ void __launch_bounds__(256) softmax_wave_kernel(const float *__restri
     const long row = (long)blockIdx.x * kRowsPerBlock + (threadIdx.x >> 6);
     if (row >= rows) return;
     const int nvec = cols >> 2;
-    const cl_f4 *xr = reinterpret_cast<const cl_f4 *>(x + row * (long)cols);
-    cl_f4 *yr = reinterpret_cast<cl_f4 *>(y + row * (long)cols);
+    const float *xr = x + row * (long)cols;
+    float *yr = y + row * (long)cols;
+    const bool has_tail = ODD && lane < (cols & 3);  // lane holds element 4 nvec + lane too
     cl_f4 v[VPT];
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
         const int c = lane + 64 * i;
-        v[i] = c < nvec ? __builtin_nontemporal_load(xr + c)
+        v[i] = c < nvec ? row_load<ODD>(xr, c)
                         : (cl_f4){-INFINITY, -INFINITY, -INFINITY, -INFINITY};
     }
-    float m = -INFINITY;
+    float e = has_tail ? xr[4 * nvec + lane] : -INFINITY;
+    float m = ODD ? e : -INFINITY;
 #pragma unroll
     for (int i = 0; i < VPT; ++i) m = fmaxf(m, hmax4(v[i]));
     m = wave_max(m);
@@ -76,17 +166,22 @@ __global__ void __launch_bounds__(256) softmax_wave_kernel(const float *__restri
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
         if (lane + 64 * i < nvec) {
-            v[i] = (cl_f4){fast_exp(v[i].x - m), fast_exp(v[i].y - m), fast_exp(v[i].z - m),
-                           fast_exp(v[i].w - m)};
+            v[i] = row_exp4<ODD>(v[i], m);
             s += hsum4(v[i]);
         }
     }
-    const float inv = 1.0f / wave_sum(s);
+    if (has_tail) {
+        e = row_exp<ODD>(e - m);
+        s += e;
+    }
+    s = wave_sum(s);
+    const float inv = 1.0f / s;
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
         const int c = lane + 64 * i;
-        if (c < nvec) __builtin_nontemporal_store(v[i] * inv, yr + c);
+        if (c < nvec) row_store<ODD>(yr, c, row_div4<ODD>(v[i], s, inv));
     }
+    if (has_tail) yr[4 * nvec + lane] = row_div<ODD>(e, s, inv);
 }
 
 // gamma and beta are staged in LDS once per workgroup (2 * cols floats):
@@ -94,7 +189,7 @@ __global__ void __launch_bounds__(256) softmax_wave_kernel(const float *__restri
 // costs as much traffic as the rows themselves (at 4096 columns the pair is
 // 32 KiB, the size of the vector L1).  The row's own loads are issued first
 // so the staging overlaps them.
-template <int VPT>
+template <int VPT, bool ODD>
 __global__ void __launch_bounds__(256) layer_norm_wave_kernel(const float *__restrict__ x,
                                                               const float *__restrict__ gamma,
                                                               const float *__restrict__ beta,
@@ -105,25 +200,34 @@ __global__ void __launch_bounds__(256) layer_norm_wave_kernel(const float *__res
     const long row = (long)blockIdx.x * kRowsPerBlock + (threadIdx.x >> 6);
     const bool live = row < rows;
     const int nvec = cols >> 2;
-    const cl_f4 *xr = reinterpret_cast<const cl_f4 *>(x + (live ? row : 0) * (long)cols);
+    const float *xr = x + (live ? row : 0) * (long)cols;
+    const bool has_tail = ODD && live && lane < (cols & 3);
     cl_f4 v[VPT];
     float s = 0.0f;
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
         const int c = lane + 64 * i;
-        v[i] = (live && c < nvec) ? __builtin_nontemporal_load(xr + c) : (cl_f4){0.f, 0.f, 0.f, 0.f};
+        v[i] = (live && c < nvec) ? row_load<ODD>(xr, c) : (cl_f4){0.f, 0.f, 0.f, 0.f};
     }
-    const cl_f4 *g4 = reinterpret_cast<const cl_f4 *>(gamma);
-    const cl_f4 *b4 = reinterpret_cast<const cl_f4 *>(beta);
+    float e = 0.0f, eg = 0.0f, eb = 0.0f;  // the tail element, its gamma and beta
+    if (has_tail) {
+        e = xr[4 * nvec + lane];
+        eg = gamma[4 * nvec + lane];
+        eb = beta[4 * nvec + lane];
+    }
+    using gvec = typename std::conditional<ODD, cl_f4u, cl_f4>::type;
+    const gvec *g4 = reinterpret_cast<const gvec *>(gamma);
+    const gvec *b4 = reinterpret_cast<const gvec *>(beta);
     for (int c = threadIdx.x; c < nvec; c += 256) {
         s_gb[c] = g4[c];
         s_gb[nvec + c] = b4[c];
     }
     __syncthreads();
     if (!live) return;
-    cl_f4 *yr = reinterpret_cast<cl_f4 *>(y + row * (long)cols);
+    float *yr = y + row * (long)cols;
 #pragma unroll
     for (int i = 0; i < VPT; ++i) s += hsum4(v[i]);
+    if (ODD) s += e;
     const float n = (float)cols;
     const float mean = wave_sum(s) / n;
     float q = 0.0f;
@@ -134,69 +238,24 @@ __global__ void __launch_bounds__(256) layer_norm_wave_kernel(const float *__res
             q += hsum4(d * d);
         }
     }
+    if (has_tail) q += (e - mean) * (e - mean);
     const float var = wave_sum(q) / n;
-    const float rsd = 1.0f / sqrtf(var + eps);
+    const float sd = sqrtf(var + eps), rsd = 1.0f / sd;
+    const float sdc = rsd > 0.0f ? sd : 0.0f;  // (row_norm's divisor)
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
         const int c = lane + 64 * i;
-        if (c < nvec) {
-            const cl_f4 o = ((v[i] - mean) * rsd) * s_gb[c] + s_gb[nvec + c];
-            __builtin_nontemporal_store(o, yr + c);
-        }
+        if (c < nvec)
+            row_store<ODD>(yr, c, row_norm4<ODD>(v[i] - mean, sdc, rsd) * s_gb[c] + s_gb[nvec + c]);
     }
-}
-
-// Any width: one wave per row, the row re-read from memory on each pass.
-__global__ void __launch_bounds__(256) softmax_loop_kernel(const float *__restrict__ x,
-                                                           float *__restrict__ y, int rows,
-                                                           int cols) {
-    const int lane = threadIdx.x & 63;
-    const long row = (long)blockIdx.x * kRowsPerBlock + (threadIdx.x >> 6);
-    if (row >= rows) return;
-    const float *xr = x + row * (long)cols;
-    float *yr = y + row * (long)cols;
-    // pass 1: running (max, sum of exp) per lane, then merged across lanes
-    float m = -INFINITY, s = 0.0f;
-    for (int c = lane; c < cols; c += 64) {
-        const float xv = xr[c];
-        const float nm = fmaxf(m, xv);
-        s = (m == -INFINITY ? 0.0f : s * expf(m - nm)) + expf(xv - nm);
-        m = nm;
-    }
-    const float gm = wave_max(m);
-    s = (m == -INFINITY) ? 0.0f : s * expf(m - gm);
-    s = wave_sum(s);
-    for (int c = lane; c < cols; c += 64) yr[c] = expf(xr[c] - gm) / s;
-}
-
-__global__ void __launch_bounds__(256) layer_norm_loop_kernel(const float *__restrict__ x,
-                                                              const float *__restrict__ gamma,
-                                                              const float *__restrict__ beta,
-                                                              float *__restrict__ y, int rows,
-                                                              int cols, float eps) {
-    const int lane = threadIdx.x & 63;
-    const long row = (long)blockIdx.x * kRowsPerBlock + (threadIdx.x >> 6);
-    if (row >= rows) return;
-    const float *xr = x + row * (long)cols;
-    float *yr = y + row * (long)cols;
-    const float n = (float)cols;
-    float s = 0.0f;
-    for (int c = lane; c < cols; c += 64) s += xr[c];
-    const float mean = wave_sum(s) / n;
-    float q = 0.0f;
-    for (int c = lane; c < cols; c += 64) {
-        const float d = xr[c] - mean;
-        q += d * d;
-    }
-    const float sd = sqrtf(wave_sum(q) / n + eps);
-    for (int c = lane; c < cols; c += 64) yr[c] = ((xr[c] - mean) / sd) * gamma[c] + beta[c];
+    if (has_tail) yr[4 * nvec + lane] = row_norm<ODD>(e - mean, sdc, rsd) * eg + eb;
 }
 
 // ---- backward and loss rows ----------------------------------------------
 
 // Softmax backward (backend.rs:2163-2183): dx = y * (dy - sum(dy * y)) per
 // row, the row of y and of dy held in registers.
-template <int VPT>
+template <int VPT, bool ODD>
 __global__ void __launch_bounds__(256) softmax_bw_wave_kernel(const float *__restrict__ y,
                                                               const float *__restrict__ dy,
                                                               float *__restrict__ dx, int rows,
@@ -205,41 +264,30 @@ __global__ void __launch_bounds__(256) softmax_bw_wave_kernel(const float *__res
     const long row = (long)blockIdx.x * kRowsPerBlock + (threadIdx.x >> 6);
     if (row >= rows) return;
     const int nvec = cols >> 2;
-    const cl_f4 *yr = reinterpret_cast<const cl_f4 *>(y + row * (long)cols);
-    const cl_f4 *gr = reinterpret_cast<const cl_f4 *>(dy + row * (long)cols);
-    cl_f4 *o = reinterpret_cast<cl_f4 *>(dx + row * (long)cols);
+    const float *yr = y + row * (long)cols, *gr = dy + row * (long)cols;
+    float *o = dx + row * (long)cols;
+    const bool has_tail = ODD && lane < (cols & 3);
     cl_f4 vy[VPT], vg[VPT];
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
         const int c = lane + 64 * i;
         const bool in = c < nvec;
-        vy[i] = in ? __builtin_nontemporal_load(yr + c) : (cl_f4){0.f, 0.f, 0.f, 0.f};
-        vg[i] = in ? __builtin_nontemporal_load(gr + c) : (cl_f4){0.f, 0.f, 0.f, 0.f};
+        vy[i] = in ? row_load<ODD>(yr, c) : (cl_f4){0.f, 0.f, 0.f, 0.f};
+        vg[i] = in ? row_load<ODD>(gr, c) : (cl_f4){0.f, 0.f, 0.f, 0.f};
     }
+    const float ey = has_tail ? yr[4 * nvec + lane] : 0.0f;
+    const float eg = has_tail ? gr[4 * nvec + lane] : 0.0f;
     float s = 0.0f;
 #pragma unroll
     for (int i = 0; i < VPT; ++i) s += hsum4(vg[i] * vy[i]);
+    if (ODD) s += eg * ey;
     s = wave_sum(s);
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
         const int c = lane + 64 * i;
-        if (c < nvec) __builtin_nontemporal_store(vy[i] * (vg[i] - s), o + c);
+        if (c < nvec) row_store<ODD>(o, c, vy[i] * (vg[i] - s));
     }
-}
-
-__global__ void __launch_bounds__(256) softmax_bw_loop_kernel(const float *__restrict__ y,
-                                                              const float *__restrict__ dy,
-                                                              float *__restrict__ dx, int rows,
-                                                              int cols) {
-    const int lane = threadIdx.x & 63;
-    const long row = (long)blockIdx.x * kRowsPerBlock + (threadIdx.x >> 6);
-    if (row >= rows) return;
-    const float *yr = y + row * (long)cols, *gr = dy + row * (long)cols;
-    float *o = dx + row * (long)cols;
-    float s = 0.0f;
-    for (int c = lane; c < cols; c += 64) s += gr[c] * yr[c];
-    s = wave_sum(s);
-    for (int c = lane; c < cols; c += 64) o[c] = yr[c] * (gr[c] - s);
+    if (has_tail) o[4 * nvec + lane] = ey * (eg - s);
 }
 
 // Rust's `f32 as usize` saturates: NaN and negative targets read class 0.
@@ -254,7 +302,7 @@ __device__ __forceinline__ long target_class(float v) {
 // give 0; a class >= cols raises the error flag and gives 0.
 // MODE 0 writes v to rowv[row].  MODE 1 is the backward (backend.rs:
 // 2686-2712): grad = (exp(l - max) / sum - [j == t]) * g / rows.
-template <int VPT, int MODE>
+template <int VPT, int MODE, bool ODD>
 __global__ void __launch_bounds__(256) cross_entropy_wave_kernel(
     const float *__restrict__ logits, const float *__restrict__ targets, long used, int rows,
     int cols, const float *__restrict__ grad_loss, float *__restrict__ out, int *err_flag) {
@@ -262,17 +310,19 @@ __global__ void __launch_bounds__(256) cross_entropy_wave_kernel(
     const long row = (long)blockIdx.x * kRowsPerBlock + (threadIdx.x >> 6);
     if (row >= rows) return;
     const int nvec = cols >> 2;
-    cl_f4 *go = MODE == 1 ? reinterpret_cast<cl_f4 *>(out + row * (long)cols) : nullptr;
+    float *go = MODE == 1 ? out + row * (long)cols : nullptr;
+    const bool has_tail = ODD && lane < (cols & 3);
     // The row's loads go out first: read after the target (and a branch on
     // it), they would wait one memory latency per row.
-    const cl_f4 *lr = reinterpret_cast<const cl_f4 *>(logits + row * (long)cols);
+    const float *lr = logits + row * (long)cols;
     cl_f4 v[VPT];
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
         const int c = lane + 64 * i;
-        v[i] = c < nvec ? __builtin_nontemporal_load(lr + c)
+        v[i] = c < nvec ? row_load<ODD>(lr, c)
                         : (cl_f4){-INFINITY, -INFINITY, -INFINITY, -INFINITY};
     }
+    float e = has_tail ? lr[4 * nvec + lane] : -INFINITY;
     long t = -1;
     if (row < used) {
         t = target_class(targets[row]);
@@ -285,7 +335,8 @@ __global__ void __launch_bounds__(256) cross_entropy_wave_kernel(
         if (MODE == 0) {
             if (lane == 0) out[row] = 0.0f;
         } else {
-            for (int c = lane; c < nvec; c += 64) go[c] = (cl_f4){0.f, 0.f, 0.f, 0.f};
+            for (int c = lane; c < nvec; c += 64) row_store<ODD>(go, c, (cl_f4){0.f, 0.f, 0.f, 0.f});
+            if (has_tail) go[4 * nvec + lane] = 0.0f;
         }
         return;
     }
@@ -298,8 +349,9 @@ __global__ void __launch_bounds__(256) cross_entropy_wave_kernel(
         for (int i = 0; i < VPT; ++i)
             if (lane + 64 * i == tv) lt = v[i][ts];
         lt = __shfl(lt, tv & 63, 64);
+        if (ODD && t >= 4l * nvec) lt = __shfl(e, (int)(t - 4l * nvec), 64);
     }
-    float m = -INFINITY;
+    float m = ODD ? e : -INFINITY;
 #pragma unroll
     for (int i = 0; i < VPT; ++i) m = fmaxf(m, hmax4(v[i]));
     m = wave_max(m);
@@ -307,10 +359,13 @@ __global__ void __launch_bounds__(256) cross_entropy_wave_kernel(
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
         if (lane + 64 * i < nvec) {
-            v[i] = (cl_f4){fast_exp(v[i].x - m), fast_exp(v[i].y - m), fast_exp(v[i].z - m),
-                           fast_exp(v[i].w - m)};
+            v[i] = fast_exp4(v[i], m);
             s += hsum4(v[i]);
         }
+    }
+    if (has_tail) {
+        e = fast_exp(e - m);
+        s += e;
     }
     s = wave_sum(s);
     if (MODE == 0) {
@@ -329,53 +384,13 @@ __global__ void __launch_bounds__(256) cross_entropy_wave_kernel(
             const long j0 = 4l * c;
             if (t >= j0 && t < j0 + 4) p[t - j0] -= 1.0f;
             const cl_f4 x = p * g;
-            __builtin_nontemporal_store((cl_f4){div_exact(x.x, fr, rr), div_exact(x.y, fr, rr),
-                                                div_exact(x.z, fr, rr), div_exact(x.w, fr, rr)},
-                                        go + c);
+            row_store<ODD>(go, c, (cl_f4){div_exact(x.x, fr, rr), div_exact(x.y, fr, rr),
+                                          div_exact(x.z, fr, rr), div_exact(x.w, fr, rr)});
         }
     }
-}
-
-// Any width: the same, re-reading the row.
-template <int MODE>
-__global__ void __launch_bounds__(256) cross_entropy_loop_kernel(
-    const float *__restrict__ logits, const float *__restrict__ targets, long used, int rows,
-    int cols, const float *__restrict__ grad_loss, float *__restrict__ out, int *err_flag) {
-    const int lane = threadIdx.x & 63;
-    const long row = (long)blockIdx.x * kRowsPerBlock + (threadIdx.x >> 6);
-    if (row >= rows) return;
-    float *go = MODE == 1 ? out + row * (long)cols : nullptr;
-    long t = -1;
-    if (row < used) {
-        t = target_class(targets[row]);
-        if (t >= cols) {
-            if (lane == 0) atomicOr(err_flag, kErrClassRange);
-            t = -1;
-        }
-    }
-    if (t < 0) {
-        if (MODE == 0) {
-            if (lane == 0) out[row] = 0.0f;
-        } else {
-            for (int c = lane; c < cols; c += 64) go[c] = 0.0f;
-        }
-        return;
-    }
-    const float *lr = logits + row * (long)cols;
-    float m = -INFINITY;
-    for (int c = lane; c < cols; c += 64) m = fmaxf(m, lr[c]);
-    m = wave_max(m);
-    float s = 0.0f;
-    for (int c = lane; c < cols; c += 64) s += fast_exp(lr[c] - m);
-    s = wave_sum(s);
-    if (MODE == 0) {
-        if (lane == 0) out[row] = (lr[t] - m) - logf(s);
-        return;
-    }
-    const float inv = 1.0f / s, g = grad_loss[0], fr = (float)rows;
-    for (int c = lane; c < cols; c += 64) {
-        const float p = fast_exp(lr[c] - m) * inv - (c == t ? 1.0f : 0.0f);
-        go[c] = (p * g) / fr;
+    if (has_tail) {
+        const float p = e * inv - (t == 4l * nvec + lane ? 1.0f : 0.0f);
+        go[4 * nvec + lane] = div_exact(p * g, fr, rr);
     }
 }
 
@@ -399,6 +414,21 @@ __global__ void __launch_bounds__(256) cross_entropy_loop_kernel(
 // per four rows.
 constexpr int kBlockThreads = 512;
 constexpr int kBlockWaves = kBlockThreads / 64;
+constexpr int kSlot = 4 * kBlockThreads;  // floats from one of a thread's vectors to its next
+
+// A row of kMaxP vectors per thread is 104 registers: held to 128 in all, two
+// workgroups still share a CU, one loading or storing while the other reduces
+// ([1024, 50257] cross entropy 35 us, 56 us while the row's addresses took
+// registers too and one workgroup filled a CU: hence row_load's uniform base
+// plus a thread offset).
+constexpr int kMaxP = 26;
+// (row_step keeps the compiler from running several vectors' arithmetic at
+// once there, whose temporaries would spill.)
+template <int P>
+__device__ __forceinline__ void row_step() {
+    if constexpr (P == kMaxP) __builtin_amdgcn_sched_barrier(0);
+}
+#define CLOVE_ROW_WAVES(P) __attribute__((amdgpu_waves_per_eu((P) == kMaxP ? 4 : 2)))
 
 // Workgroup-wide max / sum; every thread gets the result.  Each call needs
 // its own `slot` (kBlockWaves floats of LDS): a slot reused by a later
@@ -423,23 +453,26 @@ __device__ __forceinline__ float block_sum(float v, float *slot) {
     return r;
 }
 
-template <int P>
-__global__ void __launch_bounds__(kBlockThreads) softmax_block_kernel(const float *__restrict__ x,
+template <int P, bool ODD>
+__global__ void __launch_bounds__(kBlockThreads)
+    CLOVE_ROW_WAVES(P) softmax_block_kernel(const float *__restrict__ x,
                                                                       float *__restrict__ y,
                                                                       int cols) {
     __shared__ float red[2][kBlockWaves];
     const long row = blockIdx.x;
     const int nvec = cols >> 2;
-    const cl_f4 *xr = reinterpret_cast<const cl_f4 *>(x + row * (long)cols);
-    cl_f4 *yr = reinterpret_cast<cl_f4 *>(y + row * (long)cols);
+    const float *xr = x + row * (long)cols;
+    float *yr = y + row * (long)cols;
+    const bool has_tail = ODD && (int)threadIdx.x < (cols & 3);
     cl_f4 v[P];
 #pragma unroll
     for (int i = 0; i < P; ++i) {
         const int c = threadIdx.x + kBlockThreads * i;
-        v[i] = c < nvec ? __builtin_nontemporal_load(xr + c)
+        v[i] = c < nvec ? row_load<ODD>(xr + kSlot * i, threadIdx.x)
                         : (cl_f4){-INFINITY, -INFINITY, -INFINITY, -INFINITY};
     }
-    float m = -INFINITY;
+    float e = has_tail ? xr[4 * nvec + threadIdx.x] : -INFINITY;
+    float m = ODD ? e : -INFINITY;
 #pragma unroll
     for (int i = 0; i < P; ++i) m = fmaxf(m, hmax4(v[i]));
     m = block_max(m, red[0]);
@@ -447,68 +480,136 @@ __global__ void __launch_bounds__(kBlockThreads) softmax_block_kernel(const floa
 #pragma unroll
     for (int i = 0; i < P; ++i) {
         if (threadIdx.x + kBlockThreads * i < nvec) {
-            v[i] = (cl_f4){fast_exp(v[i].x - m), fast_exp(v[i].y - m), fast_exp(v[i].z - m),
-                           fast_exp(v[i].w - m)};
+            v[i] = row_exp4<ODD>(v[i], m);
             s += hsum4(v[i]);
         }
+        row_step<P>();
     }
-    const float inv = 1.0f / block_sum(s, red[1]);
+    if (has_tail) {
+        e = row_exp<ODD>(e - m);
+        s += e;
+    }
+    s = block_sum(s, red[1]);
+    const float inv = 1.0f / s;
 #pragma unroll
     for (int i = 0; i < P; ++i) {
         const int c = threadIdx.x + kBlockThreads * i;
-        if (c < nvec) __builtin_nontemporal_store(v[i] * inv, yr + c);
+        if (c < nvec) row_store<ODD>(yr + kSlot * i, threadIdx.x, row_div4<ODD>(v[i], s, inv));
+        row_step<P>();
+    }
+    if (has_tail) yr[4 * nvec + threadIdx.x] = row_div<ODD>(e, s, inv);
+}
+
+// Layer norm of rows past the wave kernel's 8192 columns: the same arithmetic
+// with a workgroup per row, gamma and beta from L2.
+template <int P, bool ODD>
+__global__ void __launch_bounds__(kBlockThreads)
+    CLOVE_ROW_WAVES(P) layer_norm_block_kernel(
+    const float *__restrict__ x, const float *__restrict__ gamma, const float *__restrict__ beta,
+    float *__restrict__ y, int cols, float eps) {
+    __shared__ float red[2][kBlockWaves];
+    const long row = blockIdx.x;
+    const int nvec = cols >> 2;
+    const float *xr = x + row * (long)cols;
+    float *yr = y + row * (long)cols;
+    const bool has_tail = ODD && (int)threadIdx.x < (cols & 3);
+    cl_f4 v[P];
+#pragma unroll
+    for (int i = 0; i < P; ++i) {
+        const int c = threadIdx.x + kBlockThreads * i;
+        v[i] = c < nvec ? row_load<ODD>(xr + kSlot * i, threadIdx.x) : (cl_f4){0.f, 0.f, 0.f, 0.f};
+    }
+    const float e = has_tail ? xr[4 * nvec + threadIdx.x] : 0.0f;
+    float s = ODD ? e : 0.0f;
+#pragma unroll
+    for (int i = 0; i < P; ++i) s += hsum4(v[i]);
+    const float n = (float)cols;
+    const float mean = block_sum(s, red[0]) / n;
+    float q = has_tail ? (e - mean) * (e - mean) : 0.0f;
+#pragma unroll
+    for (int i = 0; i < P; ++i) {
+        if (threadIdx.x + kBlockThreads * i < nvec) {
+            const cl_f4 d = v[i] - mean;
+            q += hsum4(d * d);
+        }
+        row_step<P>();
+    }
+    const float var = block_sum(q, red[1]) / n;
+    const float sd = sqrtf(var + eps), rsd = 1.0f / sd;
+    const float sdc = rsd > 0.0f ? sd : 0.0f;
+    using gvec = typename std::conditional<ODD, cl_f4u, cl_f4>::type;
+    const gvec *g4 = reinterpret_cast<const gvec *>(gamma);
+    const gvec *b4 = reinterpret_cast<const gvec *>(beta);
+#pragma unroll
+    for (int i = 0; i < P; ++i) {
+        const int c = threadIdx.x + kBlockThreads * i;
+        if (c < nvec)
+            row_store<ODD>(yr + kSlot * i, threadIdx.x, row_norm4<true>(v[i] - mean, sdc, rsd) * (cl_f4)(g4 + kBlockThreads * i)[threadIdx.x] +
+                                      (cl_f4)(b4 + kBlockThreads * i)[threadIdx.x]);
+        row_step<P>();
+    }
+    if (has_tail) {
+        const int j = 4 * nvec + threadIdx.x;
+        yr[j] = row_norm<true>(e - mean, sdc, rsd) * gamma[j] + beta[j];
     }
 }
 
-template <int P>
+template <int P, bool ODD>
 __global__ void __launch_bounds__(kBlockThreads) softmax_bw_block_kernel(
     const float *__restrict__ y, const float *__restrict__ dy, float *__restrict__ dx, int cols) {
     __shared__ float red[kBlockWaves];
     const long row = blockIdx.x;
     const int nvec = cols >> 2;
-    const cl_f4 *yr = reinterpret_cast<const cl_f4 *>(y + row * (long)cols);
-    const cl_f4 *gr = reinterpret_cast<const cl_f4 *>(dy + row * (long)cols);
-    cl_f4 *o = reinterpret_cast<cl_f4 *>(dx + row * (long)cols);
+    const float *yr = y + row * (long)cols, *gr = dy + row * (long)cols;
+    float *o = dx + row * (long)cols;
+    const bool has_tail = ODD && (int)threadIdx.x < (cols & 3);
     cl_f4 vy[P], vg[P];
 #pragma unroll
     for (int i = 0; i < P; ++i) {
         const int c = threadIdx.x + kBlockThreads * i;
         const bool in = c < nvec;
-        vy[i] = in ? __builtin_nontemporal_load(yr + c) : (cl_f4){0.f, 0.f, 0.f, 0.f};
-        vg[i] = in ? __builtin_nontemporal_load(gr + c) : (cl_f4){0.f, 0.f, 0.f, 0.f};
+        vy[i] = in ? row_load<ODD>(yr + kSlot * i, threadIdx.x) : (cl_f4){0.f, 0.f, 0.f, 0.f};
+        vg[i] = in ? row_load<ODD>(gr + kSlot * i, threadIdx.x) : (cl_f4){0.f, 0.f, 0.f, 0.f};
     }
+    const float ey = has_tail ? yr[4 * nvec + threadIdx.x] : 0.0f;
+    const float eg = has_tail ? gr[4 * nvec + threadIdx.x] : 0.0f;
     float s = 0.0f;
 #pragma unroll
     for (int i = 0; i < P; ++i) s += hsum4(vg[i] * vy[i]);
+    if (ODD) s += eg * ey;
     s = block_sum(s, red);
 #pragma unroll
     for (int i = 0; i < P; ++i) {
         const int c = threadIdx.x + kBlockThreads * i;
-        if (c < nvec) __builtin_nontemporal_store(vy[i] * (vg[i] - s), o + c);
+        if (c < nvec) row_store<ODD>(o + kSlot * i, threadIdx.x, vy[i] * (vg[i] - s));
     }
+    if (has_tail) o[4 * nvec + threadIdx.x] = ey * (eg - s);
 }
 
 // Cross entropy and its backward with a workgroup per row (the wave
 // kernel's contract and arithmetic).  l[target] comes from the registers of
 // the thread holding it, through LDS, published before the max reduction's
 // barrier.
-template <int P, int MODE>
-__global__ void __launch_bounds__(kBlockThreads) cross_entropy_block_kernel(
+template <int P, int MODE, bool ODD>
+__global__ void __launch_bounds__(kBlockThreads)
+    CLOVE_ROW_WAVES(P) cross_entropy_block_kernel(
     const float *__restrict__ logits, const float *__restrict__ targets, long used, int rows,
     int cols, const float *__restrict__ grad_loss, float *__restrict__ out, int *err_flag) {
     __shared__ float red[2][kBlockWaves];
     __shared__ float s_lt;
     const long row = blockIdx.x;
     const int nvec = cols >> 2;
-    const cl_f4 *lr = reinterpret_cast<const cl_f4 *>(logits + row * (long)cols);
-    cl_f4 *go = MODE == 1 ? reinterpret_cast<cl_f4 *>(out + row * (long)cols) : nullptr;
+    const float *lr = logits + row * (long)cols;
+    float *go = MODE == 1 ? out + row * (long)cols : nullptr;
+    const bool has_tail = ODD && (int)threadIdx.x < (cols & 3);
     cl_f4 v[P];
 #pragma unroll
     for (int i = 0; i < P; ++i) {
         const int c = threadIdx.x + kBlockThreads * i;
-        v[i] = c < nvec ? __builtin_nontemporal_load(lr + c)
+        v[i] = c < nvec ? row_load<ODD>(lr + kSlot * i, threadIdx.x)
                         : (cl_f4){-INFINITY, -INFINITY, -INFINITY, -INFINITY};
     }
+    float e = has_tail ? lr[4 * nvec + threadIdx.x] : -INFINITY;
     long t = -1;  // the same for every thread of the row
     if (row < used) {
         t = target_class(targets[row]);
@@ -522,7 +623,8 @@ __global__ void __launch_bounds__(kBlockThreads) cross_entropy_block_kernel(
             if (threadIdx.x == 0) out[row] = 0.0f;
         } else {
             for (int c = threadIdx.x; c < nvec; c += kBlockThreads)
-                go[c] = (cl_f4){0.f, 0.f, 0.f, 0.f};
+                row_store<ODD>(go, c, (cl_f4){0.f, 0.f, 0.f, 0.f});
+            if (has_tail) go[4 * nvec + threadIdx.x] = 0.0f;
         }
         return;
     }
@@ -531,10 +633,11 @@ __global__ void __launch_bounds__(kBlockThreads) cross_entropy_block_kernel(
         if (tv % kBlockThreads == (int)threadIdx.x) {
 #pragma unroll
             for (int i = 0; i < P; ++i)
-                if (i == tv / kBlockThreads) s_lt = v[i][ts];
+                if (tv < nvec && i == tv / kBlockThreads) s_lt = v[i][ts];
         }
+        if (has_tail && t == 4l * nvec + threadIdx.x) s_lt = e;
     }
-    float m = -INFINITY;
+    float m = ODD ? e : -INFINITY;
 #pragma unroll
     for (int i = 0; i < P; ++i) m = fmaxf(m, hmax4(v[i]));
     m = block_max(m, red[0]);
@@ -542,10 +645,13 @@ __global__ void __launch_bounds__(kBlockThreads) cross_entropy_block_kernel(
 #pragma unroll
     for (int i = 0; i < P; ++i) {
         if (threadIdx.x + kBlockThreads * i < nvec) {
-            v[i] = (cl_f4){fast_exp(v[i].x - m), fast_exp(v[i].y - m), fast_exp(v[i].z - m),
-                           fast_exp(v[i].w - m)};
+            v[i] = fast_exp4(v[i], m);
             s += hsum4(v[i]);
         }
+    }
+    if (has_tail) {
+        e = fast_exp(e - m);
+        s += e;
     }
     s = block_sum(s, red[1]);
     if (MODE == 0) {
@@ -564,10 +670,13 @@ __global__ void __launch_bounds__(kBlockThreads) cross_entropy_block_kernel(
             const long j0 = 4l * c;
             if (t >= j0 && t < j0 + 4) p[t - j0] -= 1.0f;
             const cl_f4 xg = p * g;
-            __builtin_nontemporal_store((cl_f4){div_exact(xg.x, fr, rr), div_exact(xg.y, fr, rr),
-                                                div_exact(xg.z, fr, rr), div_exact(xg.w, fr, rr)},
-                                        go + c);
+            row_store<ODD>(go + kSlot * i, threadIdx.x, (cl_f4){div_exact(xg.x, fr, rr), div_exact(xg.y, fr, rr),
+                                          div_exact(xg.z, fr, rr), div_exact(xg.w, fr, rr)});
         }
+    }
+    if (has_tail) {
+        const float p = e * inv - (t == 4l * nvec + threadIdx.x ? 1.0f : 0.0f);
+        go[4 * nvec + threadIdx.x] = div_exact(p * g, fr, rr);
     }
 }
 
@@ -665,20 +774,149 @@ __global__ void __launch_bounds__(kBlockThreads) cross_entropy_rows2_kernel(
     }
 }
 
+// ---- rows past the registers ---------------------------------------------
+//
+// Rows of more than 4 * 512 * kMaxP columns: a workgroup per row still, its
+// vectors walked kLoopVec at a time at any alignment, and the row read again
+// (from the last-level cache) where its values are needed a second time.
+constexpr int kLoopVec = 4;
+
+// f(j, x) for every element j of a row of `cols`, this thread's share.
+template <class F>
+__device__ __forceinline__ void row_walk(const float *row, int cols, F f) {
+    const int nvec = cols >> 2;
+    for (int c0 = threadIdx.x; c0 < nvec; c0 += kLoopVec * kBlockThreads) {
+        cl_f4 v[kLoopVec];
+#pragma unroll
+        for (int u = 0; u < kLoopVec; ++u) {
+            const int c = c0 + u * kBlockThreads;
+            if (c < nvec) v[u] = *(reinterpret_cast<const cl_f4u *>(row) + c);
+        }
+#pragma unroll
+        for (int u = 0; u < kLoopVec; ++u) {
+            const int c = c0 + u * kBlockThreads;
+            if (c < nvec)
+#pragma unroll
+                for (int k = 0; k < 4; ++k) f(4 * c + k, v[u][k]);
+        }
+    }
+    const int j = 4 * nvec + threadIdx.x;
+    if ((int)threadIdx.x < (cols & 3)) f(j, row[j]);
+}
+
+// The row's max and sum of exp(x - max) in one walk: a running max and a sum
+// relative to it per thread, the threads' sums then brought to the row's max.
+// A max of -inf counts as 0 in the subtractions (-inf entries give 0, not
+// NaN); NaN entries reach the sum.  A row of -inf alone sums to 0.
+__device__ __forceinline__ void row_max_sum(const float *row, int cols, float red[2][kBlockWaves],
+                                            float *m_out, float *s_out) {
+    float m = -INFINITY, s = 0.0f;
+    row_walk(row, cols, [&](int, float x) {
+        if (x > m) {
+            s *= m == -INFINITY ? 1.0f : close_exp(m - x);
+            m = x;
+        }
+        s += close_exp(x - (m == -INFINITY ? 0.0f : m));
+    });
+    const float gm = block_max(m, red[0]);
+    if (m != -INFINITY) s *= close_exp(m - gm);
+    *m_out = gm;
+    *s_out = block_sum(s, red[1]);
+}
+
+__global__ void __launch_bounds__(kBlockThreads) softmax_loop_kernel(const float *__restrict__ x,
+                                                                     float *__restrict__ y,
+                                                                     int cols) {
+    __shared__ float red[2][kBlockWaves];
+    const float *xr = x + (long)blockIdx.x * cols;
+    float *yr = y + (long)blockIdx.x * cols;
+    float m, s;
+    row_max_sum(xr, cols, red, &m, &s);
+    const float inv = 1.0f / s;
+    row_walk(xr, cols, [&](int j, float v) { yr[j] = row_div<true>(close_exp(v - m), s, inv); });
+}
+
+__global__ void __launch_bounds__(kBlockThreads) layer_norm_loop_kernel(
+    const float *__restrict__ x, const float *__restrict__ gamma, const float *__restrict__ beta,
+    float *__restrict__ y, int cols, float eps) {
+    __shared__ float red[2][kBlockWaves];
+    const float *xr = x + (long)blockIdx.x * cols;
+    float *yr = y + (long)blockIdx.x * cols;
+    const float n = (float)cols;
+    float s = 0.0f;
+    row_walk(xr, cols, [&](int, float v) { s += v; });
+    const float mean = block_sum(s, red[0]) / n;
+    float q = 0.0f;
+    row_walk(xr, cols, [&](int, float v) { q += (v - mean) * (v - mean); });
+    const float sd = sqrtf(block_sum(q, red[1]) / n + eps), rsd = 1.0f / sd;
+    const float sdc = rsd > 0.0f ? sd : 0.0f;
+    row_walk(xr, cols, [&](int j, float v) {
+        yr[j] = row_norm<true>(v - mean, sdc, rsd) * gamma[j] + beta[j];
+    });
+}
+
+__global__ void __launch_bounds__(kBlockThreads) softmax_bw_loop_kernel(
+    const float *__restrict__ y, const float *__restrict__ dy, float *__restrict__ dx, int cols) {
+    __shared__ float red[kBlockWaves];
+    const float *yr = y + (long)blockIdx.x * cols, *gr = dy + (long)blockIdx.x * cols;
+    float *o = dx + (long)blockIdx.x * cols;
+    float s = 0.0f;
+    row_walk(yr, cols, [&](int j, float v) { s += gr[j] * v; });
+    s = block_sum(s, red);
+    row_walk(yr, cols, [&](int j, float v) { o[j] = v * (gr[j] - s); });
+}
+
+template <int MODE>
+__global__ void __launch_bounds__(kBlockThreads) cross_entropy_loop_kernel(
+    const float *__restrict__ logits, const float *__restrict__ targets, long used, int cols,
+    float rows, const float *__restrict__ grad_loss, float *__restrict__ out, int *err_flag) {
+    __shared__ float red[2][kBlockWaves];
+    const long row = blockIdx.x;
+    const float *lr = logits + row * (long)cols;
+    float *go = MODE == 1 ? out + row * (long)cols : nullptr;
+    long t = -1;  // the same for every thread of the row
+    if (row < used) {
+        t = target_class(targets[row]);
+        if (t >= cols) {
+            if (threadIdx.x == 0) atomicOr(err_flag, kErrClassRange);
+            t = -1;
+        }
+    }
+    if (t < 0) {
+        if (MODE == 0) {
+            if (threadIdx.x == 0) out[row] = 0.0f;
+        } else {
+            for (int j = threadIdx.x; j < cols; j += kBlockThreads) go[j] = 0.0f;
+        }
+        return;
+    }
+    float m, s;
+    row_max_sum(lr, cols, red, &m, &s);
+    if (MODE == 0) {
+        if (threadIdx.x == 0) out[row] = (lr[t] - m) - logf(s);
+        return;
+    }
+    const float inv = 1.0f / s, g = grad_loss[0], rr = 1.0f / rows;
+    row_walk(lr, cols, [&](int j, float v) {
+        const float p = fast_exp(v - m) * inv - (j == t ? 1.0f : 0.0f);
+        go[j] = div_exact(p * g, rows, rr);
+    });
+}
+
 // Vectors per thread of the row-per-workgroup kernels for this width, or 0
-// for the one-wave-per-row kernels (width not a multiple of 4, at most 1024
-// columns, or beyond 16 vectors per thread).
+// for the one-wave-per-row kernels (at most 1024 columns), or -1 for a row
+// that the registers do not hold.
 int pick_block_p(int cols) {
-    if (cols % 4 != 0) return 0;
     const int nvec = cols / 4;
     if (nvec <= 256) return 0;
     int p = 1;
-    while (p * kBlockThreads < nvec) p <<= 1;
-    return p <= 16 ? p : 0;
+    while (p < 16 && p * kBlockThreads < nvec) p <<= 1;
+    if (p * kBlockThreads < nvec) p = kMaxP;
+    return p * kBlockThreads >= nvec ? p : -1;
 }
 
+// Vectors per lane of the wave-per-row kernels, or 0 past 8192 columns.
 int pick_vpt(int cols) {
-    if (cols % 4 != 0) return 0;
     const int need = (cols / 4 + 63) / 64;
     int v = 1;
     while (v < need) v <<= 1;
@@ -687,32 +925,63 @@ int pick_vpt(int cols) {
 
 bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
+// launch(P, ODD) with the constants the row-per-workgroup kernels are built
+// for.
+template <class F>
+void with_block_p(int p, bool odd, F launch) {
+    auto go = [&](auto P) {
+        if (odd) launch(P, std::true_type{});
+        else launch(P, std::false_type{});
+    };
+    switch (p) {
+    case 1: go(std::integral_constant<int, 1>{}); break;
+    case 2: go(std::integral_constant<int, 2>{}); break;
+    case 4: go(std::integral_constant<int, 4>{}); break;
+    case 8: go(std::integral_constant<int, 8>{}); break;
+    case 16: go(std::integral_constant<int, 16>{}); break;
+    default: go(std::integral_constant<int, kMaxP>{}); break;
+    }
+}
+
+// The same for the wave-per-row kernels, up to MAXV vectors per lane.
+template <int MAXV, class F>
+void with_vpt(int v, bool odd, F launch) {
+    auto go = [&](auto V) {
+        if (odd) launch(V, std::true_type{});
+        else launch(V, std::false_type{});
+    };
+    switch (v) {
+    case 1: go(std::integral_constant<int, 1>{}); return;
+    case 2: go(std::integral_constant<int, 2>{}); return;
+    case 4: go(std::integral_constant<int, 4>{}); return;
+    default: break;
+    }
+    if constexpr (MAXV >= 32) {
+        if (v == 8) go(std::integral_constant<int, 8>{});
+        else if (v == 16) go(std::integral_constant<int, 16>{});
+        else go(std::integral_constant<int, 32>{});
+    }
+}
+
 }  // namespace
 
 void softmax_rows(const float *x, float *y, size_t rows, size_t cols, hipStream_t s) {
     if (!rows || !cols) return;
     const unsigned grid = (unsigned)((rows + kRowsPerBlock - 1) / kRowsPerBlock);
     const int r = (int)rows, c = (int)cols;
-    const bool al = aligned16(x) && aligned16(y);
+    const bool odd = c % 4 != 0 || !aligned16(x) || !aligned16(y);
     const unsigned nrows = (unsigned)rows;
-    switch (al ? pick_block_p(c) : 0) {
-    case 1: softmax_block_kernel<1><<<nrows, kBlockThreads, 0, s>>>(x, y, c); return;
-    case 2: softmax_block_kernel<2><<<nrows, kBlockThreads, 0, s>>>(x, y, c); return;
-    case 4: softmax_block_kernel<4><<<nrows, kBlockThreads, 0, s>>>(x, y, c); return;
-    case 8: softmax_block_kernel<8><<<nrows, kBlockThreads, 0, s>>>(x, y, c); return;
-    case 16: softmax_block_kernel<16><<<nrows, kBlockThreads, 0, s>>>(x, y, c); return;
-    default: break;
-    }
-    const int vpt = al ? pick_vpt(c) : 0;
-    switch (vpt) {
-    case 1: softmax_wave_kernel<1><<<grid, 256, 0, s>>>(x, y, r, c); break;
-    case 2: softmax_wave_kernel<2><<<grid, 256, 0, s>>>(x, y, r, c); break;
-    case 4: softmax_wave_kernel<4><<<grid, 256, 0, s>>>(x, y, r, c); break;
-    case 8: softmax_wave_kernel<8><<<grid, 256, 0, s>>>(x, y, r, c); break;
-    case 16: softmax_wave_kernel<16><<<grid, 256, 0, s>>>(x, y, r, c); break;
-    case 32: softmax_wave_kernel<32><<<grid, 256, 0, s>>>(x, y, r, c); break;
-    default: softmax_loop_kernel<<<grid, 256, 0, s>>>(x, y, r, c); break;
-    }
+    const int p = pick_block_p(c);
+    if (p < 0)
+        softmax_loop_kernel<<<nrows, kBlockThreads, 0, s>>>(x, y, c);
+    else if (p > 0)
+        with_block_p(p, odd, [&](auto P, auto O) {
+            softmax_block_kernel<P(), O()><<<nrows, kBlockThreads, 0, s>>>(x, y, c);
+        });
+    else
+        with_vpt<4>(pick_vpt(c), odd, [&](auto V, auto O) {
+            softmax_wave_kernel<V(), O()><<<grid, 256, 0, s>>>(x, y, r, c);
+        });
 }
 
 void layer_norm_rows(const float *x, const float *gamma, const float *beta, float *y,
@@ -720,18 +989,22 @@ void layer_norm_rows(const float *x, const float *gamma, const float *beta, floa
     if (!rows || !cols) return;
     const unsigned grid = (unsigned)((rows + kRowsPerBlock - 1) / kRowsPerBlock);
     const int r = (int)rows, c = (int)cols;
-    const bool al = aligned16(x) && aligned16(y) && aligned16(gamma) && aligned16(beta);
-    const int vpt = al ? pick_vpt(c) : 0;
-    const size_t lds = 2 * (size_t)c * sizeof(float);
-    switch (vpt) {
-    case 1: layer_norm_wave_kernel<1><<<grid, 256, lds, s>>>(x, gamma, beta, y, r, c, eps); break;
-    case 2: layer_norm_wave_kernel<2><<<grid, 256, lds, s>>>(x, gamma, beta, y, r, c, eps); break;
-    case 4: layer_norm_wave_kernel<4><<<grid, 256, lds, s>>>(x, gamma, beta, y, r, c, eps); break;
-    case 8: layer_norm_wave_kernel<8><<<grid, 256, lds, s>>>(x, gamma, beta, y, r, c, eps); break;
-    case 16: layer_norm_wave_kernel<16><<<grid, 256, lds, s>>>(x, gamma, beta, y, r, c, eps); break;
-    case 32: layer_norm_wave_kernel<32><<<grid, 256, lds, s>>>(x, gamma, beta, y, r, c, eps); break;
-    default: layer_norm_loop_kernel<<<grid, 256, 0, s>>>(x, gamma, beta, y, r, c, eps); break;
-    }
+    const bool odd = c % 4 != 0 || !aligned16(x) || !aligned16(y) || !aligned16(gamma) ||
+                     !aligned16(beta);
+    const unsigned nrows = (unsigned)rows;
+    const int vpt = pick_vpt(c), p = pick_block_p(c);
+    const size_t lds = 2 * (size_t)(c / 4) * sizeof(cl_f4);
+    if (vpt > 0)
+        with_vpt<32>(vpt, odd, [&](auto V, auto O) {
+            layer_norm_wave_kernel<V(), O()><<<grid, 256, lds, s>>>(x, gamma, beta, y, r, c, eps);
+        });
+    else if (p > 0)
+        with_block_p(p, odd, [&](auto P, auto O) {
+            layer_norm_block_kernel<P(), O()><<<nrows, kBlockThreads, 0, s>>>(x, gamma, beta, y, c,
+                                                                             eps);
+        });
+    else
+        layer_norm_loop_kernel<<<nrows, kBlockThreads, 0, s>>>(x, gamma, beta, y, c, eps);
 }
 
 void softmax_backward_rows(const float *y, const float *dy, float *dx, size_t rows, size_t cols,
@@ -739,25 +1012,19 @@ void softmax_backward_rows(const float *y, const float *dy, float *dx, size_t ro
     if (!rows || !cols) return;
     const unsigned grid = (unsigned)((rows + kRowsPerBlock - 1) / kRowsPerBlock);
     const int r = (int)rows, c = (int)cols;
-    const bool al = aligned16(y) && aligned16(dy) && aligned16(dx);
+    const bool odd = c % 4 != 0 || !aligned16(y) || !aligned16(dy) || !aligned16(dx);
     const unsigned nrows = (unsigned)rows;
-    switch (al ? pick_block_p(c) : 0) {
-    case 1: softmax_bw_block_kernel<1><<<nrows, kBlockThreads, 0, s>>>(y, dy, dx, c); return;
-    case 2: softmax_bw_block_kernel<2><<<nrows, kBlockThreads, 0, s>>>(y, dy, dx, c); return;
-    case 4: softmax_bw_block_kernel<4><<<nrows, kBlockThreads, 0, s>>>(y, dy, dx, c); return;
-    case 8: softmax_bw_block_kernel<8><<<nrows, kBlockThreads, 0, s>>>(y, dy, dx, c); return;
-    case 16: softmax_bw_block_kernel<16><<<nrows, kBlockThreads, 0, s>>>(y, dy, dx, c); return;
-    default: break;
-    }
-    const int vpt = al ? pick_vpt(c) : 0;
-    switch (vpt) {
-    case 1: softmax_bw_wave_kernel<1><<<grid, 256, 0, s>>>(y, dy, dx, r, c); break;
-    case 2: softmax_bw_wave_kernel<2><<<grid, 256, 0, s>>>(y, dy, dx, r, c); break;
-    case 4: softmax_bw_wave_kernel<4><<<grid, 256, 0, s>>>(y, dy, dx, r, c); break;
-    case 8: softmax_bw_wave_kernel<8><<<grid, 256, 0, s>>>(y, dy, dx, r, c); break;
-    case 16: softmax_bw_wave_kernel<16><<<grid, 256, 0, s>>>(y, dy, dx, r, c); break;
-    default: softmax_bw_loop_kernel<<<grid, 256, 0, s>>>(y, dy, dx, r, c); break;
-    }
+    const int p = pick_block_p(c);
+    if (p < 0)
+        softmax_bw_loop_kernel<<<nrows, kBlockThreads, 0, s>>>(y, dy, dx, c);
+    else if (p > 0)
+        with_block_p(p, odd, [&](auto P, auto O) {
+            softmax_bw_block_kernel<P(), O()><<<nrows, kBlockThreads, 0, s>>>(y, dy, dx, c);
+        });
+    else
+        with_vpt<4>(pick_vpt(c), odd, [&](auto V, auto O) {
+            softmax_bw_wave_kernel<V(), O()><<<grid, 256, 0, s>>>(y, dy, dx, r, c);
+        });
 }
 
 template <int MODE>
@@ -767,33 +1034,30 @@ static void cross_entropy_launch(const float *logits, const float *targets, size
     const unsigned grid = (unsigned)((rows + kRowsPerBlock - 1) / kRowsPerBlock);
     const int r = (int)rows, c = (int)cols;
     const long u = (long)used;
-    const bool al = aligned16(logits) && (MODE == 0 || aligned16(out));
+    const bool odd = c % 4 != 0 || !aligned16(logits) || (MODE == 1 && !aligned16(out));
     const unsigned nrows = (unsigned)rows;
-    if (MODE == 0 && al && (pick_block_p(c) == 1 || pick_block_p(c) == 2)) {
+    const int p = pick_block_p(c);
+    if (MODE == 0 && !odd && (p == 1 || p == 2)) {
         const unsigned pairs = (unsigned)((rows + 1) / 2);
-        if (pick_block_p(c) == 1)
+        if (p == 1)
             cross_entropy_rows2_kernel<1><<<pairs, kBlockThreads, 0, s>>>(logits, targets, u, r, c, out, err_flag);
         else
             cross_entropy_rows2_kernel<2><<<pairs, kBlockThreads, 0, s>>>(logits, targets, u, r, c, out, err_flag);
         return;
     }
-    switch (al ? pick_block_p(c) : 0) {
-    case 1: cross_entropy_block_kernel<1, MODE><<<nrows, kBlockThreads, 0, s>>>(logits, targets, u, r, c, grad_loss, out, err_flag); return;
-    case 2: cross_entropy_block_kernel<2, MODE><<<nrows, kBlockThreads, 0, s>>>(logits, targets, u, r, c, grad_loss, out, err_flag); return;
-    case 4: cross_entropy_block_kernel<4, MODE><<<nrows, kBlockThreads, 0, s>>>(logits, targets, u, r, c, grad_loss, out, err_flag); return;
-    case 8: cross_entropy_block_kernel<8, MODE><<<nrows, kBlockThreads, 0, s>>>(logits, targets, u, r, c, grad_loss, out, err_flag); return;
-    case 16: cross_entropy_block_kernel<16, MODE><<<nrows, kBlockThreads, 0, s>>>(logits, targets, u, r, c, grad_loss, out, err_flag); return;
-    default: break;
-    }
-    const int vpt = al ? pick_vpt(c) : 0;
-    switch (vpt) {
-    case 1: cross_entropy_wave_kernel<1, MODE><<<grid, 256, 0, s>>>(logits, targets, u, r, c, grad_loss, out, err_flag); break;
-    case 2: cross_entropy_wave_kernel<2, MODE><<<grid, 256, 0, s>>>(logits, targets, u, r, c, grad_loss, out, err_flag); break;
-    case 4: cross_entropy_wave_kernel<4, MODE><<<grid, 256, 0, s>>>(logits, targets, u, r, c, grad_loss, out, err_flag); break;
-    case 8: cross_entropy_wave_kernel<8, MODE><<<grid, 256, 0, s>>>(logits, targets, u, r, c, grad_loss, out, err_flag); break;
-    case 16: cross_entropy_wave_kernel<16, MODE><<<grid, 256, 0, s>>>(logits, targets, u, r, c, grad_loss, out, err_flag); break;
-    default: cross_entropy_loop_kernel<MODE><<<grid, 256, 0, s>>>(logits, targets, u, r, c, grad_loss, out, err_flag); break;
-    }
+    if (p < 0)
+        cross_entropy_loop_kernel<MODE><<<nrows, kBlockThreads, 0, s>>>(
+            logits, targets, u, c, (float)r, grad_loss, out, err_flag);
+    else if (p > 0)
+        with_block_p(p, odd, [&](auto P, auto O) {
+            cross_entropy_block_kernel<P(), MODE, O()><<<nrows, kBlockThreads, 0, s>>>(
+                logits, targets, u, r, c, grad_loss, out, err_flag);
+        });
+    else
+        with_vpt<4>(pick_vpt(c), odd, [&](auto V, auto O) {
+            cross_entropy_wave_kernel<V(), MODE, O()><<<grid, 256, 0, s>>>(
+                logits, targets, u, r, c, grad_loss, out, err_flag);
+        });
 }
 
 void cross_entropy_rows(const float *logits, const float *targets, size_t used, size_t rows,
