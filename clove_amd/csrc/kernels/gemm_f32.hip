@@ -31,78 +31,13 @@
 #include <cstdint>
 #include <cstdlib>
 
+#include "gemm_common.h"
 #include "launch.hpp"
 
 namespace clove {
 namespace k {
 
 namespace {
-
-typedef float f4 __attribute__((ext_vector_type(4)));
-typedef float f16v __attribute__((ext_vector_type(16)));
-typedef __attribute__((address_space(3))) void lds_void;
-
-// Raw buffer resource over [base, base + bytes): stride 0, word 3 = 32-bit
-// data format (DATA_FORMAT = 4 in bits 15..18), the gfx9-family setting.
-// Reads at offsets >= bytes return 0 (and a DMA lane past the end writes 0
-// to LDS).
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void *base, uint32_t bytes) {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), (short)0, (int)bytes,
-                                             0x00020000);
-}
-
-struct GemmArgs {
-    const float *A, *B;
-    float *C;
-    float *ws;        // split-K partial tiles [splits][tiles][BM*BN]
-    int M, N, K, tiles_n, k_per_split, splits;
-    GemmEpilogue epi;
-    int tiles;        // tiles of C (the grid's x dimension is padded to 8 * per_xcd)
-    int per_xcd;      // ceil(tiles / 8)
-};
-
-// Tile order.  Workgroups are dealt to the 8 XCDs round-robin (workgroup L
-// runs on XCD L % 8), each with its own L2.  Workgroup L takes position
-// V = (L % 8) * per_xcd + L / 8 of a grouped order, so each XCD walks one
-// contiguous range of it; the grouped order visits kGroupM tile rows column
-// by column.  At 4096^3 (32 x 16 tiles of 128 x 256) an XCD then owns an
-// 8 x 8 block of tiles whose concurrently running workgroups share A and B
-// slabs in its L2 (the plain row-major order gave each XCD 2 tile columns
-// and all 32 tile rows, so every A slab was fetched for just two tiles).
-constexpr int kGroupM = 8;
-__device__ __forceinline__ bool gemm_tile(const GemmArgs &g, int *tile) {
-    const int L = blockIdx.x;
-    const int V = (L % 8) * g.per_xcd + L / 8;
-    if (V >= g.tiles) return false;
-    const int tiles_m = g.tiles / g.tiles_n;
-    const int group_size = kGroupM * g.tiles_n;
-    const int first = (V / group_size) * kGroupM;
-    const int rows = min(kGroupM, tiles_m - first);
-    const int r = V % group_size;
-    *tile = (first + r % rows) * g.tiles_n + r / rows;
-    return true;
-}
-
-// Epilogue: C = act(acc + bias[(row*N + col) % bias_n]), each step rounded
-// in f32 exactly as Clove's separate Add (backend.rs:1489) and ReLU
-// (:1823) / GELU (:1924) passes round it.
-// bcol: bias[col] when the caller has loaded it already (GEMM_BIAS_COL), so
-// that the load is not repeated after every store to C, which may alias it.
-__device__ __forceinline__ float epilogue(const GemmEpilogue &e, float v, int row, int col, int N,
-                                          const float *bcol = nullptr) {
-#pragma clang fp contract(off)
-    if (e.bias_mode == GEMM_BIAS_COL) v = v + (bcol ? *bcol : e.bias[col]);
-    else if (e.bias_mode == GEMM_BIAS_SCALAR) v = v + e.bias[0];
-    else if (e.bias_mode == GEMM_BIAS_MOD) v = v + e.bias[((uint64_t)row * N + col) % e.bias_n];
-    if (e.act == GEMM_ACT_RELU) {
-        v = v > 0.0f ? v : 0.0f;
-    } else if (e.act == GEMM_ACT_GELU) {
-        const float k = 0x1.988452p-1f;  // (2/pi).sqrt() in f32, backend.rs:1924
-        const float x3 = (v * v) * v;
-        v = 0.5f * v * (1.0f + tanhf(k * (v + 0.044715f * x3)));
-    }
-    return v;
-}
 
 // One accumulator element read out of its AGPR for the fused epilogue.
 // Without it the compiler copies every accumulator of the wave into VGPRs
@@ -1515,6 +1450,17 @@ void launch_small(const GemmPlan &p, const GemmArgs &g, hipStream_t s) {
     else launch_small_m<4>(p, g, s);
 }
 
+// The second launch of a split product: C from its parked BM x BN tiles.
+void reduce_splits(const GemmPlan &p, int BM, int BN, const float *ws, float *C,
+                   const GemmEpilogue &epi, hipStream_t s) {
+    if (p.splits <= 1) return;
+    const int64_t work = (int64_t)p.tiles * BM * (BN / 4);
+    int64_t blocks = (work + 63) / 64;
+    if (blocks > 32768) blocks = 32768;
+    gemm_splitk_reduce<<<(unsigned)blocks, 64, 0, s>>>(ws, C, p.M, p.N, BM, BN, p.tiles_n, p.tiles,
+                                                       p.splits, epi);
+}
+
 }  // namespace
 
 // Tile shape and K split above 64 rows, for operands under 2 GiB (the DMA
@@ -1570,6 +1516,55 @@ static TileChoice choose_tiles(int M, int N, int K, int num_cus, bool only64 = f
             if (best_t == 0.0 || t < best_t) {
                 best_t = t;
                 best = {cfg, made};
+            }
+        }
+    }
+    return best;
+}
+
+// Tile shape and K split on the bf16 matrix cores (gemm_bf16x3.hip) for a
+// product over 64 rows.  A CU takes its workgroups at the larger of their
+// issue time (thr, us per 16 k of a workgroup, several sharing the CU) and
+// the latency of one's own steps (lat, times the rounds of co-resident
+// workgroups); a split adds the reduce launch and its traffic, an unsplit tile
+// its epilogue, a lane's outputs one after another (bias + GELU, about 0.3 us
+// each: 1554 x 768 x 3072 fused takes 114 us in 256 x 128 tiles, 78 in 128 x
+// 128, where the product alone takes 65 and 60).  The figures are fitted to 45
+// shapes; the picks were within 14% of the best of 15 (shape, split) pairs
+// measured for each, and most within 5%.
+// max_chain: the longest k range one accumulator may sum.
+struct X3Choice {
+    int shape, splits;
+};
+static void plan_x3(GemmPlan &p, int shape, int splits) {
+    const int BM = kX3BM[shape], BN = kX3BN[shape], BK = kX3BK[shape];
+    const int slabs = (p.K + BK - 1) / BK;
+    p.x3 = shape;
+    p.tiles_n = (p.N + BN - 1) / BN;
+    p.tiles = ((p.M + BM - 1) / BM) * p.tiles_n;
+    p.k_per_split = (slabs + splits - 1) / splits * BK;
+    p.splits = (p.K + p.k_per_split - 1) / p.k_per_split;
+    p.ws_floats = p.splits > 1 ? (size_t)p.splits * p.tiles * BM * BN : 0;
+}
+static X3Choice choose_x3(int M, int N, int K, int num_cus, int max_chain) {
+    static const double thr[] = {0, 1.20, 0.65, 0.70}, lat[] = {0, 1.07, 0.75, 0.56};
+    static const int slots[] = {0, 2, 3, 1}, lane_outputs[] = {0, 128, 64, 32};
+    X3Choice best{GEMM_X3_NONE, 1};
+    double best_t = 0.0;
+    for (int sh = GEMM_X3_256x128; sh <= GEMM_X3_128x128_W8; ++sh) {
+        const int BM = kX3BM[sh], BN = kX3BN[sh], BK = kX3BK[sh], slabs = (K + BK - 1) / BK;
+        const int tiles = ((M + BM - 1) / BM) * ((N + BN - 1) / BN);
+        for (int sp = 1; sp <= 32 && (sp == 1 || sp <= slabs / 2); ++sp) {
+            const int per = (slabs + sp - 1) / sp, made = (slabs + per - 1) / per;
+            if (per * BK > max_chain && sp < 32 && sp < slabs / 2) continue;
+            // workgroups of the fullest XCD over its CUs
+            const double u = std::ceil((double)((tiles + 7) / 8) * made / (num_cus / 8.0));
+            double t = 5.0 + per * (BK / 16) * std::max(u * thr[sh], std::ceil(u / slots[sh]) * lat[sh]);
+            if (made == 1) t += 0.3 * lane_outputs[sh];
+            else t += 4.0 + (2.0 * made + 1.0) * 4.0 * M * N / 5e6;
+            if (best_t == 0.0 || t < best_t) {
+                best_t = t;
+                best = {sh, made};
             }
         }
     }
@@ -1716,6 +1711,15 @@ GemmPlan gemm_plan(int M, int N, int K, int num_cus, int force_cfg, bool a_align
     // (CLOVE_GEMM_CFG=5).  Where the DMA kernels take the shape, choose_tiles
     // weighs 64x128 tiles and the K split against them (either tiling runs
     // on DMA whatever the alignment of the rows).
+    if (force_cfg > CFG_COUNT - 1 && force_cfg < CFG_COUNT + GEMM_X3_128x128_W8 &&
+        (uint64_t)M * K * 4 < (1ull << 31) && b_bytes < (1ull << 31)) {
+        // a bf16x3 tile shape by index (tests): split until the chip is filled
+        const int shape = force_cfg - CFG_COUNT + 1;
+        const int tiles = ((M + kX3BM[shape] - 1) / kX3BM[shape]) * ((N + kX3BN[shape] - 1) / kX3BN[shape]);
+        const int want = std::min(num_cus / tiles, (K + 31) / 32 / 2);
+        plan_x3(p, shape, std::max(1, std::min(want, 32)));
+        return p;
+    }
     int cfg = M <= 32 ? CFG_32x128 : (M <= 64 ? (long_k64 ? CFG_64x128 : CFG_64x64) : CFG_128x128);
     if (force_cfg >= 0 && force_cfg < CFG_COUNT) cfg = force_cfg;
     const bool modeled = force_cfg < 0 && M > 64 && (uint64_t)M * K * 4 < (1ull << 31) &&
@@ -1734,6 +1738,19 @@ GemmPlan gemm_plan(int M, int N, int K, int num_cus, int force_cfg, bool a_align
     // 40001 157 -> 104 us, 33 x 4096 x 50257 316 -> 241, 64 x 4096 x 50256
     // 280 -> 247, 64 x 1024 x 32000 45 -> 41 (40 x 4096 x 32000 149 -> 151,
     // 64 x 8192 x 8192 78 -> 82 the other way; the rest within 1%).
+    // Over 64 rows and 0.7 GFLOP the bf16 matrix cores take the product; the
+    // FP32 MFMA tiles stay below that, where launches, the reduce pass and a
+    // workgroup's first slab are most of the time (917 x 301 x 624, 0.34
+    // GFLOP: 14.6 against 16.5 us; 1912 x 136 x 719 10.9 against 13.7; 1747 x
+    // 1171 x 177, 0.72 GFLOP: 23.1 against 20.2; 4096^3 944 against 640).  A
+    // K range of one accumulator is kept to 1.25 times what the FP32 plan
+    // would sum in one, which keeps the error below that plan's.
+    if (modeled && 2.0 * M * N * K >= 7e8) {
+        const int chain = ((K + 15) / 16 + choice.splits - 1) / choice.splits * 16;
+        const X3Choice c = choose_x3(M, N, K, num_cus, chain + chain / 4);
+        plan_x3(p, c.shape, c.splits);
+        return p;
+    }
     const bool modeled64 = long_k64 && force_cfg < 0;
     if (modeled64) choice = choose_tiles(M, N, K, num_cus, true);
     cfg = choice.cfg;
@@ -1798,6 +1815,13 @@ bool gemm_f32_transposed(const GemmPlan &p, const float *A, const float *B, floa
                          bool ta, bool tb, hipStream_t s) {
     if (ta == tb) return false;  // exactly one operand read transposed (the matmul backward)
     if (p.small || p.skinny || p.strip || p.K <= 0 || (p.splits > 1 && !ws)) return false;
+    if (p.x3) {
+        const GemmArgs g{A, B, C, ws, p.M, p.N, p.K, p.tiles_n, p.k_per_split, p.splits,
+                         GemmEpilogue{}, p.tiles, (p.tiles + 7) / 8};
+        gemm_bf16x3(p, g, ta, tb, s);
+        reduce_splits(p, kX3BM[p.x3], kX3BN[p.x3], ws, C, GemmEpilogue{}, s);
+        return true;
+    }
     if (((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(B)) & 15) != 0) return false;
     if (p.cfg != CFG_128x256 && p.cfg != CFG_128x128 && p.cfg != CFG_64x128) return false;
     const GemmArgs g{A, B, C, ws, p.M, p.N, p.K, p.tiles_n, p.k_per_split, p.splits,
@@ -1806,13 +1830,7 @@ bool gemm_f32_transposed(const GemmPlan &p, const float *A, const float *B, floa
     // split K: each split parks its tile in ws, then the splits are summed in
     // order (gemm_f32's reduce)
     auto reduce = [&] {
-        if (p.splits <= 1) return;
-        const int BM = kCfgBM[p.cfg], BN = kCfgBN[p.cfg];
-        const int64_t work = (int64_t)p.tiles * BM * (BN / 4);
-        int64_t blocks = (work + 63) / 64;
-        if (blocks > 32768) blocks = 32768;
-        gemm_splitk_reduce<<<(unsigned)blocks, 64, 0, s>>>(ws, C, p.M, p.N, BM, BN, p.tiles_n,
-                                                           p.tiles, p.splits, GemmEpilogue{});
+        reduce_splits(p, kCfgBM[p.cfg], kCfgBN[p.cfg], ws, C, GemmEpilogue{}, s);
     };
     if (!p.interior) {
         // ragged tiles or a K tail: the DMA kernel's edge form, whose 16-byte
@@ -1917,14 +1935,12 @@ void gemm_f32(const GemmPlan &p, const float *A, const float *B, float *C, float
     if (p.skinny) {
         const dim3 grid((unsigned)p.tiles, (unsigned)p.splits);
         launch_skinny(p, g, grid, s);
-        if (p.splits > 1) {
-            const int BM = 32 * p.mb, BN = 32 * p.nb;
-            const int64_t work = (int64_t)p.tiles * BM * (BN / 4);
-            int64_t blocks = (work + 63) / 64;
-            if (blocks > 32768) blocks = 32768;
-            gemm_splitk_reduce<<<(unsigned)blocks, 64, 0, s>>>(ws, C, p.M, p.N, BM, BN, p.tiles_n,
-                                                               p.tiles, p.splits, epi);
-        }
+        reduce_splits(p, 32 * p.mb, 32 * p.nb, ws, C, epi, s);
+        return;
+    }
+    if (p.x3) {
+        gemm_bf16x3(p, g, false, false, s);
+        reduce_splits(p, kX3BM[p.x3], kX3BN[p.x3], ws, C, epi, s);
         return;
     }
     switch (q.cfg) {
@@ -1936,14 +1952,7 @@ void gemm_f32(const GemmPlan &p, const float *A, const float *B, float *C, float
     case CFG_64x128: launch_cfg<64, 128, 16, 32, 64>(q, g, s); break;
     default: launch_cfg<128, 256, 16, 64, 128>(q, g, s); break;
     }
-    if (p.splits > 1) {
-        const int BM = kCfgBM[q.cfg], BN = kCfgBN[q.cfg];
-        const int64_t work = (int64_t)p.tiles * BM * (BN / 4);
-        int64_t blocks = (work + 63) / 64;
-        if (blocks > 32768) blocks = 32768;
-        gemm_splitk_reduce<<<(unsigned)blocks, 64, 0, s>>>(ws, C, p.M, p.N, BM, BN, p.tiles_n,
-                                                           p.tiles, p.splits, epi);
-    }
+    reduce_splits(p, kCfgBM[q.cfg], kCfgBN[q.cfg], ws, C, epi, s);
 }
 
 }  // namespace k

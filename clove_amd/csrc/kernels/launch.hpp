@@ -108,7 +108,12 @@ struct GemmPlan {
     // strip over the whole K (k_per_wave k per wave, `waves` waves); one
     // launch, no workspace.  tiles_n = strips, tiles = halves * strips.
     bool strip;
+    // Tiled on the bf16 matrix cores, three bf16 pieces per f32 value
+    // (gemm_bf16x3.hip): one of the tile shapes below, 0 for none.
+    int x3;
 };
+enum { GEMM_X3_NONE = 0, GEMM_X3_256x128 = 1, GEMM_X3_128x128 = 2, GEMM_X3_128x128_W8 = 3 };
+constexpr int kX3BM[] = {0, 256, 128, 128}, kX3BN[] = {0, 128, 128, 128}, kX3BK[] = {0, 16, 16, 32};
 // Optional epilogue fused into the GEMM store: bias add with Clove's
 // broadcast rule (bias read at flat index % bias_n) and an activation.
 enum { GEMM_BIAS_NONE = 0, GEMM_BIAS_COL = 1, GEMM_BIAS_SCALAR = 2, GEMM_BIAS_MOD = 3 };

@@ -1,0 +1,158 @@
+"""GPU parity of the matmul on the bf16 matrix cores (three bf16 pieces per
+f32 value), against float64.
+
+Every rounding of the kernel is one of f32 on a partial sum: at most four per
+MFMA step of 16 k and product, six products, so 1.5 per k; and the products it
+leaves out are at most 2^-26 |a b|.  The bound per element is therefore (1.5 K
++ 1) 2^-24 sum |a b|, or half a subnormal step (2^-150) per rounding where sums
+are subnormal; over a whole random matrix the roundings add as a random
+walk, and the 2-norm error stays below 2.5e-8 sqrt(K) (the FP32 MFMA kernel
+measures 1.8e-8 sqrt(K), this one 1.6e-8).
+"""
+import numpy as np
+import pytest
+
+from conftest import rng
+
+pytestmark = pytest.mark.gpu
+
+TILES = ["7", "8", "9"]  # 256x128, 128x128, 128x128 with eight waves
+
+
+def check64(got, a, b, what):
+    a64, b64 = a.astype(np.float64), b.astype(np.float64)
+    k = a.shape[1]
+    want = a64 @ b64
+    bound = (1.5 * k + 1) * 2.0**-24 * (np.abs(a64) @ np.abs(b64)) + 1.5 * k * 2.0**-150
+    assert np.all(np.abs(got - want) <= bound), what
+    return want
+
+
+@pytest.mark.parametrize("cfg", TILES)
+@pytest.mark.parametrize("m,k,n", [(1, 1, 1), (65, 16, 128), (128, 32, 128), (129, 33, 127),
+                                   (256, 15, 129), (257, 47, 255), (300, 1030, 514),
+                                   (255, 4099, 131), (512, 512, 384), (1000, 777, 1001)])
+def test_tile_edges(hip, monkeypatch, cfg, m, k, n):
+    """Tiles, slabs and splits that the shape ends inside, rows at any 4-byte
+    alignment; a repeated call gives the same bits, and the fused bias + GELU
+    the bits of the separate calls."""
+    monkeypatch.setenv("CLOVE_GEMM_CFG", cfg)
+    g = rng(m + 3 * k + 7 * n)
+    a = g.standard_normal((m, k), dtype=np.float32)
+    b = g.standard_normal((k, n), dtype=np.float32)
+    ta, tb = hip.tensor(a), hip.tensor(b)
+    got = hip.matmul(ta, tb)
+    want = check64(got.numpy(), a, b, f"{cfg}: {m}x{k}x{n}")
+    if m * n > 10000:
+        err = np.linalg.norm(got.numpy() - want) / np.linalg.norm(want)
+        assert err <= 2.5e-8 * np.sqrt(k) + 1e-7, err
+    assert np.array_equal(hip.matmul(ta, tb).numpy(), got.numpy())
+    bias = hip.tensor(g.standard_normal(n, dtype=np.float32))
+    gr = hip.Graph()
+    x, w, bi = gr.input((m, k)), gr.input((k, n)), gr.input((n,))
+    model = gr.compile([gr.op("gelu", gr.op("add", gr.op("matmul", x, w), bi))])
+    (fused,) = model.execute([ta, tb, bias])
+    assert np.array_equal(fused.numpy(), hip.gelu(hip.add(got, bias)).numpy())
+
+
+@pytest.mark.parametrize("m,k,n", [(1000, 700, 700), (2050, 1028, 3000), (777, 1001, 1003),
+                                   (4096, 128, 1000)])
+def test_planned_forward_and_gradients(hip, monkeypatch, m, k, n):
+    """Shapes the plan sends to the bf16 matrix cores in all three products
+    (plain, B transposed, A transposed), aligned or not; the gradients match
+    explicit transposes bit for bit."""
+    g = rng(m + k + n)
+    a = g.standard_normal((m, k), dtype=np.float32)
+    b = g.standard_normal((k, n), dtype=np.float32)
+    dc = g.standard_normal((m, n), dtype=np.float32)
+    ta, tb, tc = hip.tensor(a), hip.tensor(b), hip.tensor(dc)
+    check64(hip.matmul(ta, tb).numpy(), a, b, "forward")
+    da, db = (t.numpy() for t in hip.matmul_backward(ta, tb, tc))
+    check64(da, dc, b.T, "grad a")
+    check64(db, a.T, dc, "grad b")
+    monkeypatch.setenv("CLOVE_GEMM_TRANSPOSED", "0")
+    da0, db0 = (t.numpy() for t in hip.matmul_backward(ta, tb, tc))
+    assert np.array_equal(da, da0) and np.array_equal(db, db0)
+
+
+@pytest.mark.parametrize("off", [1, 2, 3])
+def test_offset_operands(hip, off):
+    """A and B that start `off` floats past a 16-byte boundary."""
+    g = rng(off)
+    a = g.standard_normal((900, 800), dtype=np.float32)
+    b = g.standard_normal((800, 700), dtype=np.float32)
+    bufs = [hip.tensor(np.concatenate([np.full(off, np.nan, np.float32), x.ravel()]))
+            for x in (a, b)]
+    ta, tb = (hip.wrap(t.device_ptr + 4 * off, x.shape) for t, x in zip(bufs, (a, b)))
+    check64(hip.matmul(ta, tb).numpy(), a, b, f"offset {off}")
+
+
+@pytest.mark.parametrize("cfg", TILES)
+def test_pieces_hold_every_bit(hip, monkeypatch, cfg):
+    """Products with the identity, a permutation and powers of two are exact:
+    no bit of an operand is dropped."""
+    monkeypatch.setenv("CLOVE_GEMM_CFG", cfg)
+    g = rng(5)
+    a = g.standard_normal((300, 256), dtype=np.float32)
+    a[:, ::3] *= np.exp2(g.integers(-60, 60, (300, 1))).astype(np.float32)
+    eye = np.eye(256, dtype=np.float32)
+    assert np.array_equal(hip.matmul(hip.tensor(a), hip.tensor(eye)).numpy(), a)
+    p = eye[g.permutation(256)] * np.exp2(g.integers(-20, 20, 256)).astype(np.float32)
+    assert np.array_equal(hip.matmul(hip.tensor(a), hip.tensor(p)).numpy(), a @ p)
+
+
+@pytest.mark.parametrize("cfg", TILES)
+@pytest.mark.parametrize("sa,sb", [(1e-36, 1e30), (1e-33, 1e25), (1e-40, 1e36), (1e-25, 1e-20),
+                                   (1e30, 1e-35), (1e18, 1e18)])
+def test_far_scales(hip, monkeypatch, cfg, sa, sb):
+    """Operands near the ends of f32's range, where the bf16 pieces would
+    lose bits: the tile is computed on the FP32 MFMA instead."""
+    monkeypatch.setenv("CLOVE_GEMM_CFG", cfg)
+    g = rng(9)
+    a = (g.standard_normal((200, 96)) * sa).astype(np.float32)
+    b = (g.standard_normal((96, 140)) * sb).astype(np.float32)
+    check64(hip.matmul(hip.tensor(a), hip.tensor(b)).numpy(), a, b, f"{sa} x {sb}")
+
+
+@pytest.mark.parametrize("cfg", TILES)
+def test_special_values(hip, monkeypatch, cfg):
+    """Infinities, NaN, the lowest f32 and single tiny entries: the results
+    of f32 arithmetic, elsewhere as if they were not there."""
+    monkeypatch.setenv("CLOVE_GEMM_CFG", cfg)
+    g = rng(10)
+    a = g.standard_normal((300, 64), dtype=np.float32)
+    b = np.abs(g.standard_normal((64, 200), dtype=np.float32)) + 0.5
+    a[3, 5] = np.inf
+    a[7, 63] = -np.inf
+    a[131, 0] = np.nan
+    a[140, 2] = np.finfo(np.float32).min
+    b[2, 150] = 0.0
+    a[260, 9] = 1e-38
+    with np.errstate(all="ignore"):
+        want = a.astype(np.float64) @ b.astype(np.float64)
+        want32 = want.astype(np.float32)
+    got = hip.matmul(hip.tensor(a), hip.tensor(b)).numpy()
+    assert np.array_equal(np.isnan(got), np.isnan(want32))
+    inf = np.isinf(want32)
+    assert np.array_equal(got[inf], want32[inf])
+    rest = np.isfinite(want32)
+    scale = np.abs(np.nan_to_num(a.astype(np.float64), posinf=0, neginf=0)) @ np.abs(b)
+    assert np.all(np.abs(got[rest] - want[rest]) <= (97 * 2.0**-24 * scale)[rest])
+
+
+def test_plan_takes_special_values(hip):
+    """The same through the default plan and the split-K reduce."""
+    g = rng(11)
+    a = g.standard_normal((700, 1500), dtype=np.float32)
+    b = g.standard_normal((1500, 700), dtype=np.float32)
+    a[650, 1400] = np.inf
+    b[0, 0] = np.nan
+    a[0, 700] = 1e-39
+    with np.errstate(all="ignore"):
+        want = a.astype(np.float64) @ b.astype(np.float64)
+    got = hip.matmul(hip.tensor(a), hip.tensor(b)).numpy()
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    inf = np.isinf(want)
+    assert np.array_equal(got[inf], want[inf].astype(np.float32))
+    ok = np.isfinite(want)
+    assert np.max(np.abs(got[ok] - want[ok])) < 1e-3
