@@ -193,7 +193,8 @@ hipError_t paged_scratch_address(float **ptr);
 // Workspace floats needed for a given shape (0 when one partition suffices).
 size_t paged_workspace_floats(int num_seqs, int num_heads, int head_dim, int max_ctx,
                               int part_tokens);
-int paged_part_tokens(int num_seqs, int num_heads, int capacity, int block_size, int num_cus);
+int paged_part_tokens(int num_seqs, int num_heads, int head_dim, int capacity, int block_size,
+                      int num_cus);
 // Head dims 64/128/256 with block sizes 8/16/32 run a fixed-shape kernel;
 // every other head_dim in [1, kPagedMaxHeadDim] and block size >= 1 runs
 // the general one.

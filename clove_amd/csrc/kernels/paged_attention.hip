@@ -41,7 +41,7 @@
 // flight, 80.8% with non-temporal loads, 82.0% with the pipeline.
 //
 // Softmax.  Each wave keeps a running (max, sum, acc) (online softmax); a
-// partition's (max, sum, acc) goes to a workspace that a one-wave-per-(b, h)
+// partition's (max, sum, acc) goes to a workspace that a one-workgroup-per-(b, h)
 // kernel merges with the log-sum-exp rule (a device-wide fence plus ticket
 // inside the partition kernel would write back the per-XCD L2s and costs
 // far more than the second launch).
@@ -738,36 +738,108 @@ __global__ void __launch_bounds__(256) paged_general_kernel(PagedArgs a) {
 }
 
 // Merges the partitions of each (b, h) with the log-sum-exp rule:
-// out = sum_p O_p e^(M_p - M) / sum_p L_p e^(M_p - M).  One wave per (b, h);
+// out = sum_p O_p e^(M_p - M) / sum_p L_p e^(M_p - M).  One workgroup per (b, h);
 // sequences that fit one partition were written by the partition kernel.
-__global__ void __launch_bounds__(256) paged_merge_kernel(PagedArgs a) {
-    const int lane = threadIdx.x & 63;
-    const int pair = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (pair >= a.num_seqs * a.num_heads) return;
+// The work is a few memory round trips, so their number is what counts: lane
+// p reads partition p's maximum and sum (one trip for up to 64 partitions),
+// the weights e^(M_p - M) meet in LDS, and then groups of threads, one per V
+// floats of the row, each add their share of the partitions' rows, eight
+// loads in flight; the groups are added in group order (deterministic).  At 2
+// sequences of 32 partitions, 32 heads of 128: 4.6 us against 19.9 for one wave
+// per (b, h) walking the partitions three times.
+constexpr int kMergeThreads = 256;
+constexpr int kMergeParts = 256;  // partitions weighed at a time
+template <int V>
+__global__ void __launch_bounds__(kMergeThreads) paged_merge_kernel(PagedArgs a, int lpg) {
+    typedef float vec __attribute__((ext_vector_type(V)));
+    __shared__ float wgt[kMergeParts];
+    __shared__ float stat[2][kMergeThreads / 64];
+    __shared__ float grp[kMergeThreads * V];
+    const int pair = blockIdx.x;
     const int b = pair / a.num_heads;
     const int D = a.head_dim;
     const int ctx = clamp_ctx(a, b, false);
     const int n_parts = (ctx + a.part_tokens - 1) / a.part_tokens;
     if (n_parts <= 1) return;
+    const int tid = threadIdx.x, wave = tid >> 6;
     const float *ws = a.partials + (size_t)pair * a.max_parts * (D + 2);
-    float M = -INFINITY;
-#pragma unroll 8
-    for (int p = 0; p < n_parts; ++p) M = fmaxf(M, ws[p * (D + 2) + D]);
-    float L = 0.0f;
-#pragma unroll 8
-    for (int p = 0; p < n_parts; ++p) {
-        const float mp = ws[p * (D + 2) + D];
-        L += mp == -INFINITY ? 0.0f : ws[p * (D + 2) + D + 1] * fast_exp(mp - M);
-    }
-    const float invL = 1.0f / L;
-    for (int d = lane; d < D; d += 64) {
-        float O = 0.0f;
-#pragma unroll 8
-        for (int p = 0; p < n_parts; ++p) {
-            const float mp = ws[p * (D + 2) + D];
-            O += mp == -INFINITY ? 0.0f : ws[p * (D + 2) + d] * fast_exp(mp - M);
+    float m = -INFINITY;
+    for (int p = tid; p < n_parts; p += kMergeThreads) m = fmaxf(m, ws[(size_t)p * (D + 2) + D]);
+    m = wave_max(m);
+    if ((tid & 63) == 0) stat[0][wave] = m;
+    __syncthreads();
+    float M = stat[0][0];
+#pragma unroll
+    for (int w = 1; w < kMergeThreads / 64; ++w) M = fmaxf(M, stat[0][w]);
+
+    const int nv = D / V;                     // vectors of a row
+    const int groups = kMergeThreads / lpg;   // lpg: threads of a group, a power of two
+    const int g = tid / lpg, gl = tid % lpg;
+    float l = 0.0f;
+    constexpr int kMaxSteps = kPagedMaxHeadDim / kMergeThreads;  // vectors of a row per thread
+    vec o[kMaxSteps];
+#pragma unroll
+    for (int i = 0; i < kMaxSteps; ++i)
+#pragma unroll
+        for (int e = 0; e < V; ++e) o[i][e] = 0.0f;
+    for (int p0 = 0; p0 < n_parts; p0 += kMergeParts) {
+        const int np = min(kMergeParts, n_parts - p0);
+        float w = -1.0f;  // a partition with no visible key: left out of both sums
+        if (tid < np) {
+            const float *row = ws + (size_t)(p0 + tid) * (D + 2);
+            const float mp = row[D];
+            if (mp != -INFINITY) {
+                w = fast_exp(mp - M);
+                l += row[D + 1] * w;
+            }
         }
-        a.out[(size_t)pair * D + d] = O * invL;
+        if (p0) __syncthreads();  // the weights before are read
+        wgt[tid] = w;
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < kMaxSteps; ++i) {
+            const int c = gl + i * lpg;
+            if (c >= nv) break;
+            constexpr int kBatch = 8;
+            for (int q0 = g; q0 < np; q0 += kBatch * groups) {
+                vec v[kBatch];
+#pragma unroll
+                for (int u = 0; u < kBatch; ++u) {
+                    const int q = q0 + u * groups;
+                    if (q < np)
+                        v[u] = *reinterpret_cast<const vec *>(ws + (size_t)(p0 + q) * (D + 2) + V * c);
+                }
+#pragma unroll
+                for (int u = 0; u < kBatch; ++u) {
+                    const int q = q0 + u * groups;
+                    if (q < np && !(wgt[q] < 0.0f)) o[i] += v[u] * wgt[q];
+                }
+            }
+        }
+    }
+    l = wave_sum(l);
+    if ((tid & 63) == 0) stat[1][wave] = l;
+    __syncthreads();
+    float L = stat[1][0];
+#pragma unroll
+    for (int w = 1; w < kMergeThreads / 64; ++w) L += stat[1][w];
+    const float invL = 1.0f / L;
+#pragma unroll
+    for (int i = 0; i < kMaxSteps; ++i) {
+        if (i * lpg >= nv) break;  // the same for every thread
+        const int c = gl + i * lpg;
+        if (i) __syncthreads();
+#pragma unroll
+        for (int e = 0; e < V; ++e) grp[V * tid + e] = o[i][e];
+        __syncthreads();
+        if (g == 0 && c < nv) {
+            vec s = o[i];
+            for (int k = 1; k < groups; ++k)
+#pragma unroll
+                for (int e = 0; e < V; ++e) s[e] += grp[V * (k * lpg + gl) + e];
+#pragma unroll
+            for (int e = 0; e < V; ++e) a.out[(size_t)pair * D + V * c + e] = s[e] * invL;
+        }
     }
 }
 
@@ -886,24 +958,28 @@ bool paged_supported(int head_dim, int block_size) {
 
 // Partition length: long partitions stream best, but the grid should still
 // hold about two workgroups per CU when every context is full; the result
-// is a power of two between 256 and 2048 tokens, rounded to whole KV
-// blocks.  CLOVE_PAGED_PART overrides it (tuning only; the output does not
-// depend on it beyond summation order).
-int paged_part_tokens(int num_seqs, int num_heads, int capacity, int block_size, int num_cus) {
-    int tokens;
+// is a power of two between 64 and 2048 tokens, rounded to whole KV blocks: few
+// heads are a chain of loads per workgroup, so short partitions win until the
+// chip is full (merge included, 64- or 128- against 256-token ones: 1 sequence
+// of 8 heads of 128 over 4096 tokens 12.7 against 25.0 us, of 12 heads of 80
+// over 300 11.6 against 28.3, 4 of 16 heads of 64 over 500 8.8 against 14.4;
+// 32-token ones gain nothing more).  Below 256 only while the partials fit the allocation-free entry's scratch, so that it takes every
+// shape it took with 256-token partitions.  CLOVE_PAGED_PART overrides it
+// (tuning only; the output does not depend on it beyond summation order).
+int paged_part_tokens(int num_seqs, int num_heads, int head_dim, int capacity, int block_size,
+                      int num_cus) {
+    const auto whole = [&](int tokens) { return std::max(1, tokens / block_size) * block_size; };
     const char *v = std::getenv("CLOVE_PAGED_PART");
-    if (v && *v) {
-        tokens = std::atoi(v);
-    } else {
-        const int64_t groups = (int64_t)num_seqs * ((num_heads + 3) / 4);
-        const int64_t want = 2LL * num_cus;
-        tokens = 256;
-        while (tokens < 2048 && groups * ((capacity + 2 * tokens - 1) / (2 * tokens)) >= want)
-            tokens *= 2;
-    }
-    int blocks = tokens / block_size;
-    if (blocks < 1) blocks = 1;
-    return blocks * block_size;
+    if (v && *v) return whole(std::atoi(v));
+    const int64_t groups = (int64_t)num_seqs * ((num_heads + 3) / 4);
+    const int64_t want = 2LL * num_cus;
+    int tokens = 64;
+    while (tokens < 2048 && groups * ((capacity + 2 * tokens - 1) / (2 * tokens)) >= want)
+        tokens *= 2;
+    while (tokens < 256 && paged_workspace_floats(num_seqs, num_heads, head_dim, capacity,
+                                                  whole(tokens)) > kPagedScratchFloats)
+        tokens *= 2;
+    return whole(tokens);
 }
 
 size_t paged_workspace_floats(int num_seqs, int num_heads, int head_dim, int max_ctx,
@@ -1016,9 +1092,15 @@ void paged_attention(const PagedArgs &a, hipStream_t s) {
         { return; }
 #undef CLOVE_PAGED_CASE
     }
-    const int pairs = a.num_seqs * a.num_heads;
-    if (a.max_parts > 1)
-        paged_merge_kernel<<<(unsigned)((pairs + 3) / 4), 256, 0, s>>>(a);
+    if (a.max_parts > 1) {
+        // rows of D + 2 floats start 8-byte aligned when D is even
+        const unsigned pairs = (unsigned)(a.num_seqs * a.num_heads);
+        const int nv = a.head_dim % 2 == 0 ? a.head_dim / 2 : a.head_dim;
+        int lpg = 16;
+        while (lpg < kMergeThreads && lpg < nv) lpg *= 2;
+        if (a.head_dim % 2 == 0) paged_merge_kernel<2><<<pairs, kMergeThreads, 0, s>>>(a, lpg);
+        else paged_merge_kernel<1><<<pairs, kMergeThreads, 0, s>>>(a, lpg);
+    }
 }
 
 void paged_append(float *k_cache, float *v_cache, const float *k_new, const float *v_new,

@@ -396,7 +396,7 @@ static k::PagedArgs paged_args(const HipBackend::PagedRaw &r, size_t *ws) {
     a.block_size = (int)bs;
     a.max_blocks = r.max_blocks;
     const int cap = (int)(r.max_blocks * bs);
-    a.part_tokens = k::paged_part_tokens((int)B, (int)H, cap, (int)bs, ctx().num_cus);
+    a.part_tokens = k::paged_part_tokens((int)B, (int)H, (int)D, cap, (int)bs, ctx().num_cus);
     a.max_parts = std::max(1, (cap + a.part_tokens - 1) / a.part_tokens);
     CLOVE_REQUIRE(a.max_parts < 65536, CLOVE_HIP_ERR_SHAPE, "too many context partitions");
     a.scale = r.scale;

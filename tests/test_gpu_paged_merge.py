@@ -1,0 +1,41 @@
+"""GPU parity of the paged decode's partition merge and of short partitions,
+against the CPU oracle at the decode's bound (2e-3 relative, 1e-5 absolute).
+"""
+import numpy as np
+import pytest
+
+import oracle
+from conftest import assert_close
+from test_gpu_paged import ATOL, RTOL, make, run
+
+pytestmark = pytest.mark.gpu
+
+
+# Partition counts at the edges of the merge: two, one lane per partition
+# (64, 65), one round of weights (256) and several (up to 630); row lengths
+# odd, below and past the thread groups; heads whose context fits one
+# partition or is empty beside long ones.
+@pytest.mark.parametrize("D,H", [(1, 2), (7, 3), (50, 1), (64, 4), (128, 5), (300, 1), (513, 1),
+                                 (1024, 1)])
+@pytest.mark.parametrize("ctx", [(9, 16, 0), (512, 520, 8), (2048, 2049, 1), (5040, 3, 2600)])
+def test_merge_edges(hip, monkeypatch, D, H, ctx):
+    monkeypatch.setenv("CLOVE_PAGED_PART", "8")
+    bs, B = 8, len(ctx)
+    mb = max(ctx) // bs + 1
+    q, kn, vn, kv, bt, cl = make(D + max(ctx), B, H, D, bs, B * mb + 1, mb, ctx)
+    want = oracle.paged_attention(q, None, None, kv, bt, cl).reshape(B, H * D)
+    got = run(hip, q, None, None, kv, bt, cl)
+    assert_close(got, want, RTOL, ATOL, f"D={D} ctx={ctx}")
+    assert np.array_equal(got, run(hip, q, None, None, kv, bt, cl))  # fixed order
+
+
+# Few heads: the plan cuts the context into 64- and 128-token partitions.
+@pytest.mark.parametrize("B,H,D,bs,ctx", [(1, 1, 64, 16, 4096), (1, 8, 128, 16, 1000),
+                                          (1, 12, 80, 16, 300), (2, 4, 128, 32, 129),
+                                          (3, 2, 1024, 8, 700), (1, 3, 96, 100, 1500)])
+def test_short_partitions_as_planned(hip, B, H, D, bs, ctx):
+    mb = ctx // bs + 1
+    q, kn, vn, kv, bt, cl = make(B + D + ctx, B, H, D, bs, B * mb + 1, mb,
+                                 [ctx - 17 * b for b in range(B)])
+    want = oracle.paged_attention(q, kn, vn, kv, bt, cl).reshape(B, H * D)
+    assert_close(run(hip, q, kn, vn, kv, bt, cl), want, RTOL, ATOL, f"{B} x {H} x {D} over {ctx}")
