@@ -160,9 +160,16 @@ void HipBackend::flash_attention_into(const Tensor &q, const Tensor &k, const Te
     // tab_pos0); passing the mask offset as its q_pos and shifting the table
     // origin by the difference keeps that row at s + q_pos.
     const bool q_tab = tab != nullptr && vec4;
+    const int cus = ctx().num_cus;
+    const bool causal = (flags & CLOVE_ATTN_CAUSAL) != 0;
+    const size_t wsf = k::attention_workspace_floats((int)B, (int)S, (int)Sk, num_heads, D, mask_q,
+                                                     mask_k, causal, cus);
+    TensorNode ws;
+    if (wsf) ws = new_tensor({wsf}, CLOVE_HIP_F32);
     k::attention_prefill(qp, kp, v.f32(), out.f32(), (int)B, (int)S, (int)Sk, num_heads, D,
-                         mask_q, mask_k, (flags & CLOVE_ATTN_CAUSAL) != 0, sc,
-                         q_tab ? tab->f32() : nullptr, t0 - (q_pos - mask_q), s);
+                         mask_q, mask_k, causal, sc,
+                         q_tab ? tab->f32() : nullptr, t0 - (q_pos - mask_q),
+                         ws ? ws->f32() : nullptr, cus, s);
 }
 
 TensorNode HipBackend::flash_attention(const TensorNode &q_, const TensorNode &k_,

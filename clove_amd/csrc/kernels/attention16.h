@@ -1,6 +1,6 @@
 // attention16.h -- the 16-query-per-wave attention prefill kernel on
-// v_mfma_f32_16x16x4_f32, shared by flash_attention.hip (head dim 64, the
-// fixed-shape build) and attention_general.hip (every other head dim).
+// v_mfma_f32_16x16x4_f32 for the head dims that the bf16x3 kernel does not take
+// (flash_attention.hip): past 128, or not a multiple of 8.
 //
 // 8 waves = 128 queries per workgroup, the K and V tiles (32 or 64 keys,
 // double buffered through LDS, one barrier per block) shared by all of them.
@@ -12,10 +12,10 @@
 //   the lane's own P element i: no shuffles; element e of O^T block jd is
 //   dim 16jd + 4q + e of query r.
 //
-// DP is the head dim the tiles are laid out for (a multiple of 16).  With
-// GEN the real head dim D = a.D <= DP arrives at run time: dims at or past D
-// load as zero in Q, K and V (zero terms in q . k; output dims that are never
-// stored), so one instantiation serves every D in (DP - 16, DP].  VEC4 moves
+// DP is the head dim the tiles are laid out for (a multiple of 16), D = a.D <=
+// DP the real one, known at run time: dims at or past D load as zero in Q, K and
+// V (zero terms in q . k; output dims that are never stored), so one
+// instantiation serves every D in (DP - 16, DP].  VEC4 moves
 // 16-byte pieces (D % 4 == 0, 16-byte aligned rows); without it every float
 // moves on its own (any D, 4-byte alignment) and RoPE on q is applied by the
 // caller beforehand.
@@ -49,12 +49,13 @@ struct AttnArgs {
     const float2 *rope_tab;  // (cos, sin) per (position, pair) to rotate q, or null
     int tab_pos0;            // position of rope_tab's first row
     int D;                   // head dim (the GEN kernels read it; others use their DP)
+    int splits;              // workgroups that share a query block's keys (bf16x3 kernel)
+    float *part;             // their partial results: [splits][B*S*H][D], then (m, sum) pairs
 };
 
-template <int DP, bool CAUSAL, bool GEN, bool VEC4>
+template <int DP, bool CAUSAL, bool VEC4>
 __global__ void __launch_bounds__(512, (DP <= 128 ? 4 : 2)) attention16_kernel(AttnArgs a) {
     static_assert(DP % 16 == 0, "tiles are laid out in 16-dim groups");
-    static_assert(VEC4 || GEN, "the fixed-shape build moves 16-byte pieces");
     // pitches measured conflict-free at DP = 64 and 128 (SQ_LDS_BANK_CONFLICT 0):
     // a K read takes 16 rows x two 16-byte slots, a PV step 4 rows x 16 floats
     constexpr int kPK = DP + 8;
@@ -75,7 +76,7 @@ __global__ void __launch_bounds__(512, (DP <= 128 ? 4 : 2)) attention16_kernel(A
     __shared__ __attribute__((aligned(16))) float sK[2][BK * kPK];
     __shared__ __attribute__((aligned(16))) float sV[2][BK * kPV];
 
-    const int D = GEN ? a.D : DP;
+    const int D = a.D;
     const int L = blockIdx.x;
     const int BH = a.B * a.H;
     const int qb = a.nqb - 1 - L / BH;
@@ -102,11 +103,11 @@ __global__ void __launch_bounds__(512, (DP <= 128 ? 4 : 2)) attention16_kernel(A
         const int d0 = 16 * g + 4 * q4;
         cl_f4 v = {0.f, 0.f, 0.f, 0.f};
         if (VEC4) {
-            if (q_ok && (!GEN || d0 < D)) v = *reinterpret_cast<const cl_f4 *>(qrow + d0);
+            if (q_ok && d0 < D) v = *reinterpret_cast<const cl_f4 *>(qrow + d0);
             // RoPE: q's pairs (dims d0 + {0,1} and {2,3}, whole pairs in this
             // lane) rotated with the arithmetic of the RoPE pass, before the
             // scale: the values that pass would have stored.
-            if (trow && (!GEN || d0 < D)) {
+            if (trow && d0 < D) {
                 const float2 t0 = trow[d0 / 2], t1 = trow[d0 / 2 + 1];
                 cl_f4 r;
                 r.x = v.x * t0.x - v.y * t0.y;
@@ -158,7 +159,7 @@ __global__ void __launch_bounds__(512, (DP <= 128 ? 4 : 2)) attention16_kernel(A
     for (int i = 0; i < kPer; ++i) {
         const int idx = threadIdx.x + 512 * i;
         const int key = idx / kRowElems, dim = (idx % kRowElems) * (VEC4 ? 4 : 1);
-        const bool ok = (kElems % 512 == 0 || idx < kElems) && (!GEN || dim < D);
+        const bool ok = (kElems % 512 == 0 || idx < kElems) && dim < D;
         tkey[i] = key;
         toff[i] = ok ? ((uint32_t)key * (uint32_t)HD + (uint32_t)(h * D + dim)) * 4u : kOutside;
     }
@@ -304,7 +305,7 @@ __global__ void __launch_bounds__(512, (DP <= 128 ? 4 : 2)) attention16_kernel(A
     for (int jd = 0; jd < kG; ++jd) {
         const int d0 = 16 * jd + 4 * q4;
         if (VEC4) {
-            if (!GEN || d0 < D) *reinterpret_cast<cl_f4 *>(orow + d0) = o[jd] * inv;
+            if (d0 < D) *reinterpret_cast<cl_f4 *>(orow + d0) = o[jd] * inv;
         } else {
 #pragma unroll
             for (int e = 0; e < 4; ++e)
@@ -313,7 +314,7 @@ __global__ void __launch_bounds__(512, (DP <= 128 ? 4 : 2)) attention16_kernel(A
     }
 }
 
-// Every head dim other than the fixed-shape builds' (attention_general.hip):
+// Every head dim the bf16x3 kernel does not take (attention_general.hip):
 // a.D in [1, kAttnMaxHeadDim]; 16-byte rows when a.D % 4 == 0, else a
 // null rope_tab (q already rotated).  grid = B * H * nqb workgroups.
 void attention_prefill_general(const AttnArgs &a, bool causal, unsigned grid, hipStream_t s);

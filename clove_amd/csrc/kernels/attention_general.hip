@@ -1,5 +1,5 @@
-// attention_general.hip -- the attention prefill at every head dim the
-// fixed-shape builds (64 and 128, flash_attention.hip) do not cover.
+// attention_general.hip -- the attention prefill at every head dim the bf16x3
+// kernel (flash_attention.hip) does not take: past 128, or not a multiple of 8.
 //
 // Clove gives head_dim = dim / num_heads with no restriction (nn.rs:519,
 // nn/attention.rs:47), and the lazy FlashAttention step takes it from the
@@ -20,11 +20,11 @@ namespace {
 template <int DP>
 void launch(const AttnArgs &a, bool causal, unsigned grid, hipStream_t s) {
     if (a.D % 4 == 0) {
-        if (causal) attention16_kernel<DP, true, true, true><<<grid, 512, 0, s>>>(a);
-        else attention16_kernel<DP, false, true, true><<<grid, 512, 0, s>>>(a);
+        if (causal) attention16_kernel<DP, true, true><<<grid, 512, 0, s>>>(a);
+        else attention16_kernel<DP, false, true><<<grid, 512, 0, s>>>(a);
     } else {
-        if (causal) attention16_kernel<DP, true, true, false><<<grid, 512, 0, s>>>(a);
-        else attention16_kernel<DP, false, true, false><<<grid, 512, 0, s>>>(a);
+        if (causal) attention16_kernel<DP, true, false><<<grid, 512, 0, s>>>(a);
+        else attention16_kernel<DP, false, false><<<grid, 512, 0, s>>>(a);
     }
 }
 

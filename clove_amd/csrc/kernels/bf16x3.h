@@ -1,0 +1,56 @@
+// bf16x3.h -- f32 values as three bf16 pieces, for products on the bf16 matrix
+// cores (gemm_bf16x3.hip, flash_attention.hip).
+//
+// x = x1 + x2 + x3 with x1 = bf16(x), x2 = bf16(x - x1), x3 = bf16(x - x1 - x2),
+// each rounded to nearest: 3 x 8 bits hold f32's 24 exactly, as long as the
+// last piece is no subnormal (|x| >= 2^-102) and the first does not round to
+// infinity.  A product x y keeps x1y1 + (x1y2 + x2y1) + (x2y2 + x1y3 + x3y1);
+// the three left out are at most 2^-26 |x y| together, a quarter of one f32
+// rounding, of random sign.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+namespace clove {
+namespace k {
+
+typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
+typedef float f2 __attribute__((ext_vector_type(2)));
+typedef unsigned u4 __attribute__((ext_vector_type(4)));
+typedef unsigned short us2 __attribute__((ext_vector_type(2)));
+
+// split_pair's tiny key of 2^-102: a least key below it means that some value
+// was too small for its pieces.
+constexpr unsigned short kTinyKey = 2 * (25 << 7);
+
+// The six products, smallest first: piece of the first operand, of the second.
+constexpr int kPieceA[6] = {2, 0, 1, 1, 0, 0}, kPieceB[6] = {0, 2, 1, 0, 1, 0};
+
+__device__ __forceinline__ unsigned bf16_pair(float a, float b) {
+    return __builtin_bit_cast(unsigned, __builtin_convertvector((f2){a, b}, bf2));
+}
+
+// Two floats as one dword of each of the three pieces.  *tiny keeps the least
+// 2 |x1| - 1 seen, as 16-bit integers of the bf16 bits (a zero wraps to the
+// largest): the smallest nonzero magnitude, at one operation per value.
+__device__ __forceinline__ void split_pair(float a, float b, unsigned *p1, unsigned *p2,
+                                           unsigned *p3, us2 *tiny) {
+    const unsigned h = bf16_pair(a, b);
+    const float ra = a - __uint_as_float(h << 16), rb = b - __uint_as_float(h & 0xffff0000u);
+    const unsigned m = bf16_pair(ra, rb);
+    *p1 = h;
+    *p2 = m;
+    *p3 = bf16_pair(ra - __uint_as_float(m << 16), rb - __uint_as_float(m & 0xffff0000u));
+    const us2 key = __builtin_bit_cast(us2, h) * (us2){2, 2} + (us2){0xffff, 0xffff};
+    *tiny = __builtin_elementwise_min(*tiny, key);
+}
+
+// LDS contents are published by a wait for this wave's LDS operations and a
+// bare barrier: __syncthreads() would also wait for the slab in flight.
+__device__ __forceinline__ void lds_barrier() {
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
+}  // namespace k
+}  // namespace clove

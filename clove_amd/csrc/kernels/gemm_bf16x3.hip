@@ -4,13 +4,9 @@
 // v_mfma_f32_32x32x16_bf16 does the multiply-adds of eight
 // v_mfma_f32_32x32x2_f32 in half the cycles of one: an f32 product as six bf16
 // products still runs at 2.6 times the FP32 MFMA's rate.
-//  * x = x1 + x2 + x3 with x1 = bf16(x), x2 = bf16(x - x1), x3 = bf16(x - x1
-//    - x2), each rounded to nearest: 3 x 8 bits hold f32's 24 exactly (no
-//    bit of an operand is dropped; a product with a one-hot or power-of-two
-//    operand is exact, as in f32).
-//  * x y = x1y1 + (x1y2 + x2y1) + (x2y2 + x1y3 + x3y1), accumulated in f32 by
-//    the MFMAs; the three products left out are at most 2^-26 |x y| together,
-//    a quarter of one f32 rounding, of random sign.
+// The pieces (bf16x3.h) hold every bit of an operand, so a product with a
+// one-hot or power-of-two operand is exact, as in f32; the MFMAs accumulate in
+// f32.
 // Error against float64 (normal data, 4096 x K x 4096, relative 2-norm): K =
 // 64 1.13e-7, 512 3.5e-7, 1024 4.8e-7, 4096 1.02e-6 -- the FP32 MFMA kernel
 // 1.44e-7, 4.1e-7, 5.7e-7, 1.15e-6.
@@ -24,6 +20,7 @@
 #include <cstdint>
 #include <type_traits>
 
+#include "bf16x3.h"
 #include "gemm_common.h"
 #include "launch.hpp"
 
@@ -32,34 +29,7 @@ namespace k {
 
 namespace {
 
-typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
-typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
-typedef float f2 __attribute__((ext_vector_type(2)));
-typedef unsigned u4 __attribute__((ext_vector_type(4)));
-typedef unsigned short us2 __attribute__((ext_vector_type(2)));
-
 constexpr uint32_t kOutside = 0x80000000u;     // past the end of both operands (each under 2 GiB)
-constexpr unsigned short kTinyKey = 2 * (25 << 7);  // tiny_key of 2^-102
-
-__device__ __forceinline__ unsigned bf16_pair(float a, float b) {
-    return __builtin_bit_cast(unsigned, __builtin_convertvector((f2){a, b}, bf2));
-}
-
-// Two floats as one dword of each of the three pieces.  *tiny keeps the least
-// 2 |x1| - 1 seen, as 16-bit integers of the bf16 bits (a zero wraps to the
-// largest): the smallest nonzero magnitude, at one operation per value.
-__device__ __forceinline__ void split_pair(float a, float b, unsigned *p1, unsigned *p2,
-                                           unsigned *p3, us2 *tiny) {
-    const unsigned h = bf16_pair(a, b);
-    const float ra = a - __uint_as_float(h << 16), rb = b - __uint_as_float(h & 0xffff0000u);
-    const unsigned m = bf16_pair(ra, rb);
-    *p1 = h;
-    *p2 = m;
-    *p3 = bf16_pair(ra - __uint_as_float(m << 16), rb - __uint_as_float(m & 0xffff0000u));
-    const us2 key = __builtin_bit_cast(us2, h) * (us2){2, 2} + (us2){0xffff, 0xffff};
-    *tiny = __builtin_elementwise_min(*tiny, key);
-}
-
 // One operand's share of a thread: OCT octets (eight consecutive k of one row
 // of A, or of one column of B) of a slab of R rows.  KC: the operand's k are
 // consecutive in memory (A, or B given transposed): an octet is two 16-byte
@@ -174,12 +144,6 @@ struct Operand {
     }
 };
 
-// LDS contents are published by a wait for this wave's LDS operations and a
-// bare barrier: __syncthreads() would also wait for the slab in flight.
-__device__ __forceinline__ void lds_barrier() {
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-}
-
 // A workgroup of T / 64 waves, each WM x WN of a BM x BN tile, walking slabs of
 // BK k.  While slab s multiplies out of one LDS stage, slab s + 1 (in
 // registers) is split into the other and the f32 values of slab s + 2 set out;
@@ -279,13 +243,12 @@ gemm_bf16x3_kernel(GemmArgs g) {
                 read_a(r);
             }
             if ((r + 1) % IB != 0) read_a(r + 1);
-            constexpr int pa[6] = {2, 0, 1, 1, 0, 0}, pb[6] = {0, 2, 1, 0, 1, 0};
 #pragma unroll
             for (int p = 0; p < 6; ++p)
 #pragma unroll
                 for (int j = 0; j < JB; ++j)
                     acc[r % IB][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                        fa[r & 1][pa[p]], fb[j][pb[p]], acc[r % IB][j], 0, 0, 0);
+                        fa[r & 1][kPieceA[p]], fb[j][kPieceB[p]], acc[r % IB][j], 0, 0, 0);
 #pragma unroll
             for (int u = r * UNITS / REG; u < (r + 1) * UNITS / REG; ++u) {
                 if constexpr (decltype(next)::value) {

@@ -49,9 +49,9 @@ void ordered_sum(const float *x, size_t n, float sign, float div, float *out, hi
 void transpose(const float *in, float *out, size_t R, size_t C, hipStream_t s);
 
 // flash_attention.hip -- attention prefill and RoPE.  q [B, S, H*D], k, v
-// [B, Sk, H*D], out [B, S, H*D]; D in [1, kAttnMaxHeadDim].  D 64 and 128
-// run fixed-shape kernels, every other D the general one; all four tensors
-// 16-byte aligned when D % 4 == 0, else 4-byte aligned with a null
+// [B, Sk, H*D], out [B, S, H*D]; D in [1, kAttnMaxHeadDim].  Multiples of 8 up
+// to 128 run on the bf16 matrix cores, every other D on the FP32 MFMA; all four
+// tensors 16-byte aligned when D % 4 == 0, else 4-byte aligned with a null
 // q_rope_tab (the caller rotates q first).
 constexpr int kAttnMaxHeadDim = 256;
 bool attention_supported(int head_dim);
@@ -61,7 +61,12 @@ bool attention_supported(int head_dim);
 // applies).
 void attention_prefill(const float *q, const float *k, const float *v, float *out, int B, int S,
                        int Sk, int H, int D, int q_pos, int k_pos, bool causal, float scale,
-                       const float *q_rope_tab, int tab_pos0, hipStream_t s);
+                       const float *q_rope_tab, int tab_pos0, float *ws, int num_cus,
+                       hipStream_t s);
+// Floats of the workspace `ws` (0: none needed) for a shape whose keys are
+// split over workgroups.
+size_t attention_workspace_floats(int B, int S, int Sk, int H, int D, int q_pos, int k_pos,
+                                  bool causal, int num_cus);
 // freq.div[j] = 10000^(2j / D) (powf on the host, as backend.rs:2818 forms it).
 struct AttnFreq {
     float div[128];

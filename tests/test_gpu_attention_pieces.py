@@ -1,0 +1,109 @@
+"""GPU parity of the attention prefill on the bf16 matrix cores, against
+float64: head dims on and off its tile sizes, ragged blocks, keys split over
+workgroups, and values its bf16 pieces cannot hold.
+
+The bound: scores and output are f32 sums, so the relative 2-norm error over
+random inputs stays within a few 1e-7 (measured 1e-7 to 6e-7; the FP32 MFMA
+kernels measure 2.5e-7 to 6e-7); 2e-6 is asked.
+"""
+import numpy as np
+import pytest
+
+from conftest import rng
+
+pytestmark = pytest.mark.gpu
+
+
+def attention64(q, k, v, heads, past, causal):
+    q, k, v = (x.astype(np.float64) for x in (q, k, v))
+    B, S, X = q.shape
+    D, Sk = X // heads, k.shape[1]
+    out = np.empty_like(q)
+    hidden = np.arange(Sk)[None, :] > np.arange(S)[:, None] + past
+    for b in range(B):
+        for h in range(heads):
+            c = slice(h * D, (h + 1) * D)
+            s = q[b, :, c] @ k[b, :, c].T / np.sqrt(D)
+            if causal:
+                s[hidden] = -np.inf
+            p = np.exp(s - s.max(1, keepdims=True))
+            out[b, :, c] = p @ v[b, :, c] / p.sum(1, keepdims=True)
+    return out
+
+
+def inputs(seed, B, S, past, H, D):
+    g = rng(seed)
+    return [g.standard_normal((B, n, H * D), dtype=np.float32) for n in (S, S + past, S + past)]
+
+
+def run(hip, q, k, v, H, past, causal):
+    flags = hip.ATTN_CAUSAL if causal else 0
+    return hip.flash_attention(hip.tensor(q), hip.tensor(k), hip.tensor(v), H, q_pos=past,
+                               flags=flags).numpy()
+
+
+def check(got, want, what):
+    err = np.linalg.norm(got - want) / np.linalg.norm(want)
+    assert err <= 2e-6, (what, err)
+    assert np.max(np.abs(got - want)) <= 2e-5 * np.abs(want).max(), what
+
+
+# One query and key; blocks of 128 and 256 queries and of 32 keys that the
+# lengths end inside, at and past; few queries over many keys (split), many
+# queries (unsplit); every tile size with a head dim below it.
+@pytest.mark.parametrize("D", [8, 32, 40, 64, 72, 96, 104, 128])
+@pytest.mark.parametrize("B,S,past,H", [(1, 1, 0, 1), (1, 31, 33, 2), (2, 128, 0, 2),
+                                        (1, 257, 63, 2), (3, 5, 1500, 1), (1, 600, 0, 3)])
+@pytest.mark.parametrize("causal", [True, False])
+def test_shapes(hip, D, B, S, past, H, causal):
+    q, k, v = inputs(D + S + past, B, S, past, H, D)
+    got = run(hip, q, k, v, H, past, causal)
+    check(got, attention64(q, k, v, H, past, causal), f"D={D} {B}x{S}+{past}")
+    assert np.array_equal(got, run(hip, q, k, v, H, past, causal))  # fixed order
+
+
+@pytest.mark.parametrize("D", [64, 80, 96, 128])
+@pytest.mark.parametrize("scale_q,scale_k,scale_v", [(1e-33, 1e33, 1), (1e33, 1e-33, 1),
+                                                     (1, 1, 1e-36), (1, 1, 1e32)])
+def test_far_scales(hip, D, scale_q, scale_k, scale_v):
+    """Values near the ends of f32's range go through the FP32 MFMA."""
+    q, k, v = inputs(D, 1, 150, 40, 2, D)
+    q, k, v = (x * np.float32(s) for x, s in zip((q, k, v), (scale_q, scale_k, scale_v)))
+    check(run(hip, q, k, v, 2, 40, True), attention64(q, k, v, 2, 40, True), f"D={D}")
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("S,past", [(300, 0), (40, 900)])
+def test_special_values(hip, D, S, past):
+    """NaN and infinite values reach the queries that see them, in one split or
+    another, and no other query or dim; single tiny values change nothing else.
+    (A masked key weighs 0, and 0 times an infinite v is NaN in an f32 sum: the
+    infinity's own dim is only looked at where its key is visible.)"""
+    q, k, v = inputs(D + S, 1, S, past, 1, D)
+    q[0, 3, 1] = 1e-39
+    k[0, 2, 5] = 1e-38
+    k[0, past + 20, 0] = np.nan          # queries 20.. see it
+    v[0, past + 30, 7] = np.inf          # queries 30.. see it, in dim 7
+    keep = np.ones(D, bool)
+    keep[7] = False
+    got = run(hip, q, k, v, 1, past, True)[0]
+    assert np.all(np.isnan(got[20:]))
+    want = attention64(q, np.nan_to_num(k), np.nan_to_num(v, posinf=0.0), 1, past, True)[0]
+    check(got[:20, keep], want[:20, keep], "rows before the NaN")
+    k[0, past + 20, 0] = 0.0
+    got = run(hip, q, k, v, 1, past, True)[0]
+    assert np.all(np.isinf(got[30:, 7]))
+    want = attention64(q, k, np.nan_to_num(v, posinf=0.0), 1, past, True)[0]
+    check(got[:, keep], want[:, keep], "dims beside the infinity")
+
+
+def test_no_visible_key(hip):
+    """Queries before every key get zeros, in split and unsplit launches."""
+    for S, Sk in ((64, 64), (10, 3000)):
+        g = rng(S)
+        q = g.standard_normal((1, S, 256), dtype=np.float32)
+        k, v = (g.standard_normal((1, Sk, 256), dtype=np.float32) for _ in range(2))
+        got = hip.flash_attention(hip.tensor(q), hip.tensor(k), hip.tensor(v), 2, q_pos=0,
+                                  k_pos=S - 4, flags=hip.ATTN_CAUSAL).numpy()
+        assert np.all(got[0, :S - 4] == 0.0)
+        assert np.array_equal(got[0, S - 4], v[0, 0])
