@@ -1112,21 +1112,52 @@ __global__ void __launch_bounds__(64 * kStripWaves) gemm_strip_kernel(GemmArgs g
 // adjacent column strips whose 64-byte row pieces share 128-byte lines in
 // its L2.
 // Needs K % 4 == 0, a 16-byte aligned A and A, B under 2 GiB (the plan
-// checks them).
+// checks them).  The other forms take any K and alignment (SMALL_ANY) and one
+// operand transposed (SMALL_TA: A stored [K][M]; SMALL_TB: B stored [N][K]):
+// small_load puts the same values into the same registers, so the sums and
+// the bits are those of the vector form on a transposed copy.  The backward of
+// a 64 x 784 x 128 layer then runs without its transposes (4-5 us each, a
+// product 3-4 us): 12.5 -> 7.9 us a call at 50 x 784 x 128, and the training
+// step around it 94 -> 85 us.  Loading a k-contiguous operand value by value
+// instead of in 16-byte pieces cost 21.7 against 9.3 us at the backward of 64 x
+// 201 x 1000: 16 cache lines per load, four times the loads.
 template <int MB>
 struct SmallBatch {
     f4 a[4][MB];
     float b[4][4];
 };
+enum SmallForm { SMALL_VEC = 0, SMALL_ANY, SMALL_TA, SMALL_TB };
+
+// Four consecutive k of one operand, from byte offset `off` of the lane's first
+// k, `past` k further on, k_step bytes apart; zero from k `left` on (counted
+// from the lane's first) and where off says outside.  KVEC (k_step 4): one
+// 16-byte load (buffer loads need 4-byte alignment) where `whole` says that
+// every lane's four are inside, so no load reaches past the operand's end.
+template <bool KVEC>
+__device__ __forceinline__ f4 small_load(__amdgpu_buffer_rsrc_t rsrc, uint32_t off, int past,
+                                         int left, bool whole, uint32_t k_step) {
+    constexpr uint32_t kOutside = 0x80000000u;
+    if (KVEC && whole)
+        return __builtin_bit_cast(
+            f4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)off, 4 * past, 0));
+    f4 v;
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+        v[t] = __builtin_bit_cast(
+            float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, (int)(past + t < left ? off : kOutside),
+                                                        (int)((uint32_t)(past + t) * k_step), 0));
+    return v;
+}
 
 // One tile V of product g (the body of the small-path kernels).
-template <int W, int MB, int NBATCH, bool EPI>
+template <int W, int MB, int NBATCH, bool EPI, int FORM>
 __device__ __forceinline__ void small_tile(const GemmArgs &g, int V) {
     constexpr int kRows = 16 * MB;
     constexpr int kPitch = 17;
     __shared__ float red[W * kRows * kPitch];
     const int M = g.M, N = g.N, K = g.K;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int l16 = lane & 15, q = lane >> 4;
     const int m0 = (V / g.tiles_n) * kRows, n0 = (V % g.tiles_n) * 16;
     const int kpw = g.k_per_split;  // 64 * NBATCH
@@ -1141,11 +1172,15 @@ __device__ __forceinline__ void small_tile(const GemmArgs &g, int V) {
 #pragma unroll
     for (int i = 0; i < MB; ++i) {
         const int row = m0 + 16 * i + l16;
-        aoff[i] = row < M && k_lane < K ? ((uint32_t)row * (uint32_t)K + (uint32_t)k_lane) * 4u
-                                        : kOutside;
+        aoff[i] = row < M && k_lane < K
+                      ? (FORM == SMALL_TA ? (uint32_t)k_lane * (uint32_t)M + (uint32_t)row
+                                          : (uint32_t)row * (uint32_t)K + (uint32_t)k_lane) * 4u
+                      : kOutside;
     }
-    const uint32_t boff = col < N && k_lane < K ? ((uint32_t)k_lane * (uint32_t)N + (uint32_t)col) * 4u
-                                                : kOutside;
+    const uint32_t boff = col < N && k_lane < K
+                              ? (FORM == SMALL_TB ? (uint32_t)col * (uint32_t)K + (uint32_t)k_lane
+                                                  : (uint32_t)k_lane * (uint32_t)N + (uint32_t)col) * 4u
+                              : kOutside;
     const uint32_t row_bytes = (uint32_t)N * 4u;
     const int groups = ke > kb ? (ke - kb + 15) / 16 : 0;
 
@@ -1155,6 +1190,22 @@ __device__ __forceinline__ void small_tile(const GemmArgs &g, int V) {
 #pragma unroll
         for (int d = 0; d < 4; ++d) {
             const int gi = g0 + d;
+            if constexpr (FORM != SMALL_VEC) {
+                // a group past the wave's k range is left out (its products
+                // too), one that ends inside it goes value by value
+                if (gi >= groups) continue;
+                const bool whole = kb + 16 * gi + 16 <= ke;
+#pragma unroll
+                for (int i = 0; i < MB; ++i)
+                    x.a[d][i] = small_load<FORM != SMALL_TA>(rsrc_a, aoff[i], 16 * gi, ke - k_lane,
+                                                             whole,
+                                                             FORM == SMALL_TA ? 4u * (uint32_t)M : 4u);
+                const f4 b = small_load<FORM == SMALL_TB>(rsrc_b, boff, 16 * gi, ke - k_lane, whole,
+                                                          FORM == SMALL_TB ? 4u : row_bytes);
+#pragma unroll
+                for (int t = 0; t < 4; ++t) x.b[d][t] = b[t];
+                continue;
+            }
             const bool ok = gi < groups && kb + 16 * gi + 4 * q < ke;
 #pragma unroll
             for (int i = 0; i < MB; ++i)
@@ -1180,7 +1231,8 @@ __device__ __forceinline__ void small_tile(const GemmArgs &g, int V) {
         // keep each batch whole and ahead of the previous batch's MFMAs
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int d = 0; d < 4; ++d)
+        for (int d = 0; d < 4; ++d) {
+            if (FORM != SMALL_VEC && 4 * bi + d >= groups) continue;
 #pragma unroll
             for (int t = 0; t < 4; ++t)
 #pragma unroll
@@ -1188,6 +1240,7 @@ __device__ __forceinline__ void small_tile(const GemmArgs &g, int V) {
                     acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(buf[bi & 1].a[d][i][t],
                                                                   buf[bi & 1].b[d][t], acc[i], 0,
                                                                   0, 0);
+        }
         __builtin_amdgcn_sched_barrier(0);
     }
 
@@ -1238,12 +1291,12 @@ __device__ __forceinline__ void small_tile(const GemmArgs &g, int V) {
     }
 }
 
-template <int W, int MB, int NBATCH, bool EPI>
+template <int W, int MB, int NBATCH, bool EPI, int FORM>
 __global__ void __launch_bounds__(64 * W) gemm_small_kernel(GemmArgs g) {
     const int L = blockIdx.x;
     const int V = (L % 8) * g.per_xcd + L / 8;
     if (V >= g.tiles) return;
-    small_tile<W, MB, NBATCH, EPI>(g, V);
+    small_tile<W, MB, NBATCH, EPI, FORM>(g, V);
 }
 
 // Grouped form (the planner's horizontal MatMul groups): one launch covers
@@ -1262,7 +1315,7 @@ __global__ void __launch_bounds__(64 * W) gemm_small_grouped_kernel(GroupedArgs 
     const int L = blockIdx.x;
     int p = 0;
     while (p + 1 < ga.count && L >= ga.starts[p + 1]) ++p;
-    small_tile<W, 1, 1, true>(ga.prob[p], L - ga.starts[p]);
+    small_tile<W, 1, 1, true, SMALL_VEC>(ga.prob[p], L - ga.starts[p]);
 }
 
 // K = 0: C = epilogue(0) (bias and activation still apply).  A kernel rather
@@ -1427,27 +1480,32 @@ void launch_strip(const GemmPlan &p, const GemmArgs &g, hipStream_t s) {
 }
 
 template <int W, int MB, int NBATCH>
-void launch_small_b(const GemmPlan &p, const GemmArgs &g, hipStream_t s) {
+void launch_small_b(const GemmArgs &g, SmallForm form, hipStream_t s) {
     const bool epi = g.epi.bias_mode != GEMM_BIAS_NONE || g.epi.act != GEMM_ACT_NONE;
     const unsigned grid = (unsigned)(8 * g.per_xcd);
-    if (epi) gemm_small_kernel<W, MB, NBATCH, true><<<grid, 64 * W, 0, s>>>(g);
-    else gemm_small_kernel<W, MB, NBATCH, false><<<grid, 64 * W, 0, s>>>(g);
+    auto go = [&](auto kernel) { kernel<<<grid, 64 * W, 0, s>>>(g); };
+    if (form == SMALL_TA) go(gemm_small_kernel<W, MB, NBATCH, false, SMALL_TA>);
+    else if (form == SMALL_TB) go(gemm_small_kernel<W, MB, NBATCH, false, SMALL_TB>);
+    else if (form == SMALL_ANY && epi) go(gemm_small_kernel<W, MB, NBATCH, true, SMALL_ANY>);
+    else if (form == SMALL_ANY) go(gemm_small_kernel<W, MB, NBATCH, false, SMALL_ANY>);
+    else if (epi) go(gemm_small_kernel<W, MB, NBATCH, true, SMALL_VEC>);
+    else go(gemm_small_kernel<W, MB, NBATCH, false, SMALL_VEC>);
 }
 
 template <int MB>
-void launch_small_m(const GemmPlan &p, const GemmArgs &g, hipStream_t s) {
+void launch_small_m(const GemmPlan &p, const GemmArgs &g, SmallForm form, hipStream_t s) {
     switch (p.waves) {
-    case 2: launch_small_b<2, MB, 1>(p, g, s); return;
-    case 4: launch_small_b<4, MB, 1>(p, g, s); return;
-    case 8: launch_small_b<8, MB, 1>(p, g, s); return;
-    default: launch_small_b<16, MB, 1>(p, g, s); return;
+    case 2: launch_small_b<2, MB, 1>(g, form, s); return;
+    case 4: launch_small_b<4, MB, 1>(g, form, s); return;
+    case 8: launch_small_b<8, MB, 1>(g, form, s); return;
+    default: launch_small_b<16, MB, 1>(g, form, s); return;
     }
 }
 
-void launch_small(const GemmPlan &p, const GemmArgs &g, hipStream_t s) {
-    if (p.mb == 1) launch_small_m<1>(p, g, s);
-    else if (p.mb == 2) launch_small_m<2>(p, g, s);
-    else launch_small_m<4>(p, g, s);
+void launch_small(const GemmPlan &p, const GemmArgs &g, SmallForm form, hipStream_t s) {
+    if (p.mb == 1) launch_small_m<1>(p, g, form, s);
+    else if (p.mb == 2) launch_small_m<2>(p, g, form, s);
+    else launch_small_m<4>(p, g, form, s);
 }
 
 // The second launch of a split product: C from its parked BM x BN tiles.
@@ -1599,15 +1657,19 @@ GemmPlan gemm_plan(int M, int N, int K, int num_cus, int force_cfg, bool a_align
     // most 64 k each.  Longer K keeps the tiled or skinny split-K forms, which
     // spread it over every CU (at M = 32, N = K = 4096 this path with 16
     // waves and 4 batches per wave measured 22.1 us against the skinny
-    // kernel's 19.2 us).
+    // kernel's 19.2 us).  K % 4 != 0 or an A off a 16-byte boundary takes the
+    // SMALL_ANY form: at M x K x N = 64 x 783 x 128 4.0 us against the split
+    // tiles' 9.7, 250 x 1001 x 250 5.6 against 12.2, 1000 x 3 x 200 the same 4.1
+    // (all with the gap between calls).
     {
         int mb = 1;
         auto tiles_for = [&](int b) { return ((M + 16 * b - 1) / (16 * b)) * ((N + 15) / 16); };
         while (mb < 4 && tiles_for(mb) > num_cus) mb *= 2;
         const int tiles = tiles_for(mb);
-        if (force_cfg < 0 && !force_skinny && K >= 4 && K % 4 == 0 && K <= 1024 && a_aligned &&
-            tiles <= num_cus && b_bytes < (1ull << 31) && (uint64_t)M * K * 4 < (1ull << 31)) {
+        if (force_cfg < 0 && !force_skinny && K <= 1024 && tiles <= num_cus &&
+            b_bytes < (1ull << 31) && (uint64_t)M * K * 4 < (1ull << 31)) {
             p.small = true;
+            p.any_k = K % 4 != 0 || !a_aligned;
             p.mb = mb;
             int w = 2;
             while (w < 16 && w * 64 < K) w *= 2;
@@ -1814,7 +1876,13 @@ void gemm_f32_grouped(const GemmPlan *plans, const float *const *A, const float 
 bool gemm_f32_transposed(const GemmPlan &p, const float *A, const float *B, float *C, float *ws,
                          bool ta, bool tb, hipStream_t s) {
     if (ta == tb) return false;  // exactly one operand read transposed (the matmul backward)
-    if (p.small || p.skinny || p.strip || p.K <= 0 || (p.splits > 1 && !ws)) return false;
+    if (p.skinny || p.strip || p.K <= 0 || (p.splits > 1 && !ws)) return false;
+    if (p.small) {
+        const GemmArgs g{A, B, C, ws, p.M, p.N, p.K, p.tiles_n, p.k_per_split, 1,
+                         GemmEpilogue{}, p.tiles, (p.tiles + 7) / 8};
+        launch_small(p, g, ta ? SMALL_TA : SMALL_TB, s);
+        return true;
+    }
     if (p.x3) {
         const GemmArgs g{A, B, C, ws, p.M, p.N, p.K, p.tiles_n, p.k_per_split, p.splits,
                          GemmEpilogue{}, p.tiles, (p.tiles + 7) / 8};
@@ -1925,7 +1993,7 @@ void gemm_f32(const GemmPlan &p, const float *A, const float *B, float *C, float
     GemmArgs g{A, B, C, ws, p.M, p.N, p.K, p.tiles_n, p.k_per_split, p.splits, epi,
                p.tiles, (p.tiles + 7) / 8};
     if (p.small) {
-        launch_small(p, g, s);
+        launch_small(p, g, p.any_k ? SMALL_ANY : SMALL_VEC, s);
         return;
     }
     if (p.strip) {

@@ -108,7 +108,9 @@ struct GemmPlan {
     int k_per_wave;    // a whole number of pipeline chunks
     // Small path: one workgroup of `waves` waves per 16 x 16 tile of C, K
     // split inside the workgroup (k_per_split k per wave); no workspace.
+    // any_k: K % 4 != 0 or A off a 16-byte boundary.
     bool small;
+    bool any_k;
     // Strip path (M <= 32): one workgroup per 16-row half of a 32-column
     // strip over the whole K (k_per_wave k per wave, `waves` waves); one
     // launch, no workspace.  tiles_n = strips, tiles = halves * strips.

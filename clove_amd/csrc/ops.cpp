@@ -293,7 +293,7 @@ static k::GemmPlan prepare_matmul(const Tensor &a, const Tensor &b, const Tensor
 // A product the grouped small kernel can take: the small path, and for a
 // softmax epilogue whole rows in one 16-column tile.
 static bool groupable(const k::GemmPlan &p, int act) {
-    return p.small && (act != k::GEMM_ACT_SOFTMAX || p.N <= 16);
+    return p.small && !p.any_k && (act != k::GEMM_ACT_SOFTMAX || p.N <= 16);
 }
 
 void HipBackend::matmul_into(const Tensor &a, const Tensor &b, Tensor &out, const Tensor *bias,
@@ -303,9 +303,11 @@ void HipBackend::matmul_into(const Tensor &a, const Tensor &b, Tensor &out, cons
     hipStream_t s = ctx().stream;
     TensorNode ws;
     if (p.ws_floats) ws = new_tensor({p.ws_floats}, CLOVE_HIP_F32);
-    if (act == k::GEMM_ACT_SOFTMAX && !(p.small && p.tiles_n == 1)) {
-        // only the small path with one tile column holds whole rows: product
-        // and bias into a temporary, then the row softmax into `out`
+    if (act == k::GEMM_ACT_SOFTMAX && !(p.small && !p.any_k && p.tiles_n == 1)) {
+        // only the small path with one tile column holds whole rows (at K % 4 !=
+        // 0 it leaves them to the row kernel, whose exponential such products
+        // had): product and bias into a temporary, then the row softmax into
+        // `out`
         epi.act = k::GEMM_ACT_NONE;
         TensorNode tmp = new_tensor(out.shape, CLOVE_HIP_F32);
         k::gemm_f32(p, a.f32(), b.f32(), tmp->f32(), ws ? ws->f32() : nullptr, epi, s);
