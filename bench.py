@@ -60,6 +60,9 @@ sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBS = 8000.0        # MI355X HBM3E, AMD published
 FP32_MFMA_PEAK_TFS = 157.3   # MI355X dense FP32 matrix, AMD published
+# large products and the prefill multiply f32 values as three bf16 pieces, six
+# bf16 products each: a sixth of the dense bf16 matrix rate (2.5 PFLOP/s)
+BF16X3_PEAK_TFS = 2500.0 / 6
 METRIC = "fused-op HBM GB/s (% of peak); f32 GEMM TFLOP/s; paged-decode tokens/s"
 
 
@@ -299,7 +302,7 @@ def bench_matmul(ca, oracle, args, out, skinny_only=False):
     flops = 2.0 * 4096 ** 3
     tf = flops / (per.mean() * 1e-3) / 1e12
     part = {"value": round(tf, 2), "unit": "TFLOP/s", "ms": round(per.mean(), 4),
-            "roofline": roofline("mfma", tf, FP32_MFMA_PEAK_TFS, "TFLOP/s")}
+            "roofline": roofline("mfma", tf, round(BF16X3_PEAK_TFS, 1), "TFLOP/s")}
     if not args.no_cpu:
         def leg():
             ah, bh = a.numpy(), b.numpy()
@@ -320,7 +323,7 @@ def bench_matmul(ca, oracle, args, out, skinny_only=False):
                          gemm_atol(want[0]))
         defer(leg)
     out["matmul_4096"] = part
-    log(f"matmul 4096^3: {tf:.1f} TFLOP/s ({tf / FP32_MFMA_PEAK_TFS:.1%} of FP32 MFMA peak), "
+    log(f"matmul 4096^3: {tf:.1f} TFLOP/s ({tf / BF16X3_PEAK_TFS:.1%} of a sixth of the bf16 peak), "
         f"{per.mean():.3f} ms")
     # the planner's GEMM with a fused bias + GELU epilogue (one step)
     bias = ca.empty((4096,)).fill_normal(7)
@@ -331,7 +334,7 @@ def bench_matmul(ca, oracle, args, out, skinny_only=False):
     wall, per = timed(ca, lambda: model.execute([a, b, bias])[0], steps, args.warmup)
     tf = flops / (per.mean() * 1e-3) / 1e12
     epart = {"value": round(tf, 2), "unit": "TFLOP/s", "ms": round(per.mean(), 4),
-             "roofline": roofline("mfma", tf, FP32_MFMA_PEAK_TFS, "TFLOP/s")}
+             "roofline": roofline("mfma", tf, round(BF16X3_PEAK_TFS, 1), "TFLOP/s")}
     if not args.no_cpu:
         def eleg():
             ah, bh, biash = a.numpy(), b.numpy(), bias.numpy()
@@ -448,7 +451,7 @@ def bench_mlp(ca, oracle, args, out):
 
 def bench_backward(ca, oracle, args, out):
     """The backward row: each op at a config-sized shape, HBM roofline (the
-    matmul backward: FP32 MFMA), CPU baseline on a bounded sample."""
+    matmul backward: a sixth of the bf16 matrix peak), CPU baseline on a bounded sample."""
     g = np.random.Generator(np.random.PCG64(7))
     R, Cc, N = 8192, 4096, 4096 * 4096
     targets = ca.tensor(g.integers(0, Cc, R).astype(np.float32))
@@ -546,14 +549,14 @@ def bench_backward(ca, oracle, args, out):
                                "unit": "us/step (wall, 4 tensors, 1 launch)",
                                "gpu_us": round(per.mean() * 1e3, 2)}
     log(f"adamw MLP parameters: {wall * 1e3:.1f} us/step wall")
-    # matmul backward at 4096^3: grad_a and grad_b, two GEMMs and two transposes
+    # matmul backward at 4096^3: grad_a and grad_b, two GEMMs
     dc = ca.empty((4096, 4096)).fill_normal(8)
     steps = max(5, args.steps // 10)
     wall, per = timed(ca, lambda: ca.matmul_backward(a, b, dc), steps, max(15, args.warmup // 2))
     flops = 4.0 * 4096 ** 3
     tf = flops / (per.mean() * 1e-3) / 1e12
     part = {"value": round(tf, 2), "unit": "TFLOP/s", "ms": round(per.mean(), 4),
-            "roofline": roofline("mfma", tf, FP32_MFMA_PEAK_TFS, "TFLOP/s")}
+            "roofline": roofline("mfma", tf, round(BF16X3_PEAK_TFS, 1), "TFLOP/s")}
     if oracle is not None:
         def leg(part=part):
             ah, bh, dch = a.numpy(), b.numpy(), dc.numpy()
@@ -566,8 +569,8 @@ def bench_backward(ca, oracle, args, out):
                                               "full grad_a and grad_b at 4096^3, one run")
         defer(leg)
     out["matmul_backward_4096"] = part
-    log(f"matmul backward 4096^3: {tf:.1f} TFLOP/s ({tf / FP32_MFMA_PEAK_TFS:.1%} of FP32 MFMA "
-        f"peak), {per.mean():.3f} ms")
+    log(f"matmul backward 4096^3: {tf:.1f} TFLOP/s ({tf / BF16X3_PEAK_TFS:.1%} of a sixth "
+        f"of the bf16 peak), {per.mean():.3f} ms")
 
 
 def backward_parity(ca, name, want, y, dy, x, targets, one, a, b):
@@ -634,7 +637,7 @@ def cpu_backward(oracle, name, y, dy, x, targets, a, b, nbytes):
 def bench_attention(ca, oracle, args, out):
     """Attention prefill (the fused FlashAttention step): B=1, S=4096, H=32,
     D=128, causal + RoPE; algorithmic FLOPs 4*D*H*S(S+1)/2 (QK^T and PV over
-    the visible keys); FP32 MFMA roofline.  Also RoPE alone (HBM)."""
+    the visible keys); roofline a sixth of the bf16 matrix peak.  Also RoPE alone (HBM)."""
     B, S, H, D = 1, 4096, 32, 128
     q = ca.empty((B, S, H * D)).fill_normal(31)
     k = ca.empty((B, S, H * D)).fill_normal(32)
@@ -644,7 +647,7 @@ def bench_attention(ca, oracle, args, out):
     flops = 4.0 * D * H * S * (S + 1) / 2
     tf = flops / (per.mean() * 1e-3) / 1e12
     part = {"value": round(tf, 2), "unit": "TFLOP/s", "ms": round(per.mean(), 4),
-            "roofline": roofline("mfma", tf, FP32_MFMA_PEAK_TFS, "TFLOP/s")}
+            "roofline": roofline("mfma", tf, round(BF16X3_PEAK_TFS, 1), "TFLOP/s")}
     if oracle is not None:
         def leg():
             qh, kh, vh = q.numpy(), k.numpy(), v.numpy()
@@ -667,7 +670,7 @@ def bench_attention(ca, oracle, args, out):
         defer(leg)
     out["flash_attention_4096"] = part
     log(f"attention prefill S=4096 H=32 D=128 causal+rope: {tf:.1f} TFLOP/s "
-        f"({tf / FP32_MFMA_PEAK_TFS:.1%} of FP32 MFMA peak), {per.mean():.3f} ms")
+        f"({tf / BF16X3_PEAK_TFS:.1%} of a sixth of the bf16 peak), {per.mean():.3f} ms")
     xs_sets = [ca.empty((1, S, H * D)).fill_normal(34)
                for _ in range(input_sets(args, 4 * S * H * D))]
     x = xs_sets[0]
@@ -696,16 +699,16 @@ def bench_attention(ca, oracle, args, out):
 PART_KERNELS = {
     "copy_reference": ["clove_chain_flatten_b0"],
     "chain_broadcast": ["clove_chain_mul_add_gelu_mul_b0020"],
-    "softmax": ["softmax_block_kernel<2>"],
-    "layer_norm": ["layer_norm_wave_kernel<16>"],
+    "softmax": ["softmax_block_kernel<2, false>"],
+    "layer_norm": ["layer_norm_wave_kernel<16, false>"],
     "matmul_skinny_32": ["gemm_skinny_kernel<1, 4, 4, 8>", "gemm_splitk_reduce"],
-    "paged_decode": ["paged_heads_kernel<128, 16, 4>", "paged_merge_kernel"],
-    "paged_decode_d96": ["paged_general_kernel<8, 3, true, 1>", "paged_merge_kernel"],
-    "softmax_backward": ["softmax_bw_block_kernel<2>"],
+    "paged_decode": ["paged_heads_kernel<128, 16, 4>", "paged_merge_kernel<2>"],
+    "paged_decode_d96": ["paged_general_kernel<8, 3, true, 1>", "paged_merge_kernel<2>"],
+    "softmax_backward": ["softmax_bw_block_kernel<2, false>"],
     "gelu_backward": ["clove_chain_gelugrad_b00"],
     "broadcast_grad": ["bcast_grad_cols4_kernel", "bcast_grad_final_kernel"],
     "cross_entropy": ["cross_entropy_rows2_kernel<2>", "ordered_sum_kernel"],
-    "cross_entropy_backward": ["cross_entropy_block_kernel<2, 1>"],
+    "cross_entropy_backward": ["cross_entropy_block_kernel<2, 1, false>"],
     "mse": ["sq_diff_partial_kernel<true>", "ordered_sum_kernel"],
     "mse_backward": ["mse_backward_kernel<true>"],
     "rope": ["rope_rows_kernel<true>"],
