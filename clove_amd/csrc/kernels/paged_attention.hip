@@ -963,7 +963,13 @@ bool paged_supported(int head_dim, int block_size) {
 // chip is full (merge included, 64- or 128- against 256-token ones: 1 sequence
 // of 8 heads of 128 over 4096 tokens 12.7 against 25.0 us, of 12 heads of 80
 // over 300 11.6 against 28.3, 4 of 16 heads of 64 over 500 8.8 against 14.4;
-// 32-token ones gain nothing more).  Below 256 only while the partials fit the allocation-free entry's scratch, so that it takes every
+// 32-token ones gain nothing more).  A context that one partition walks in
+// about the time of the merge launch keeps one: up to 256 tokens of heads up to
+// 64, 160 of wider ones (4 sequences of 12 heads of 64 over 100 tokens 6.6 us
+// against 10.0 split, over 200 8.8 against 10.0, over 256 10.1 against 10.2,
+// over 300 13.4 against 9.6; 16 of 8 heads of 128 over 100 7.3 against 10.2,
+// over 160 9.3 against 10.1, over 200 12.0 against 11.6; 4 of 16 of 96 over
+// 128 9.8 against 11.1, over 200 12.7 against 11.8).  Below 256 only while the partials fit the allocation-free entry's scratch, so that it takes every
 // shape it took with 256-token partitions.  CLOVE_PAGED_PART overrides it
 // (tuning only; the output does not depend on it beyond summation order).
 int paged_part_tokens(int num_seqs, int num_heads, int head_dim, int capacity, int block_size,
@@ -973,7 +979,7 @@ int paged_part_tokens(int num_seqs, int num_heads, int head_dim, int capacity, i
     if (v && *v) return whole(std::atoi(v));
     const int64_t groups = (int64_t)num_seqs * ((num_heads + 3) / 4);
     const int64_t want = 2LL * num_cus;
-    int tokens = 64;
+    int tokens = capacity <= (head_dim <= 64 ? 256 : 160) ? 256 : 64;
     while (tokens < 2048 && groups * ((capacity + 2 * tokens - 1) / (2 * tokens)) >= want)
         tokens *= 2;
     while (tokens < 256 && paged_workspace_floats(num_seqs, num_heads, head_dim, capacity,

@@ -39,3 +39,13 @@ def test_short_partitions_as_planned(hip, B, H, D, bs, ctx):
                                  [ctx - 17 * b for b in range(B)])
     want = oracle.paged_attention(q, kn, vn, kv, bt, cl).reshape(B, H * D)
     assert_close(run(hip, q, kn, vn, kv, bt, cl), want, RTOL, ATOL, f"{B} x {H} x {D} over {ctx}")
+
+
+# The longest contexts that keep one partition, and one block more.
+@pytest.mark.parametrize("D,blocks", [(64, 16), (64, 17), (128, 10), (128, 11), (80, 10), (80, 11)])
+def test_one_partition_edge(hip, D, blocks):
+    B, H, bs = 2, 6, 16
+    ctx = [blocks * bs, blocks * bs - 3]
+    q, kn, vn, kv, bt, cl = make(D + blocks, B, H, D, bs, B * blocks + 1, blocks, ctx)
+    want = oracle.paged_attention(q, kn, vn, kv, bt, cl).reshape(B, H * D)
+    assert_close(run(hip, q, kn, vn, kv, bt, cl), want, RTOL, ATOL, f"D={D} {blocks} blocks")
