@@ -828,10 +828,17 @@ bool attention_supported(int head_dim) { return head_dim >= 1 && head_dim <= kAt
 struct AttnX3Plan {
     int dp, qb, splits;
 };
+// Up to 64 queries over up to 64 keys, a workgroup to a CU, the split of the
+// operands costs more than the faster products give, and the FP32 MFMA kernel takes the call (with RoPE, FP32 first:
+// 64 queries of 12 heads of 80 13.2 against 15.6 us, of 8 of 64 11.0 against
+// 12.7, of 16 of 96 14.5 against 15.8; 100 queries 18.2 against 16.1, 15.0
+// against 13.7, 20.4 against 17.1).
+constexpr int kShort = 64;
 static AttnX3Plan attention_x3_plan(int B, int S, int Sk, int H, int D, int q_pos, int k_pos,
                                     bool causal, int num_cus) {
     AttnX3Plan p{0, 0, 1};
     if (D % 8 != 0 || D > 128) return p;
+    if (S <= kShort && Sk <= kShort && (int64_t)B * H <= num_cus) return p;
     static const float lone[] = {1.25f, 1.8f, 2.6f, 3.9f}, full[] = {1.8f, 2.9f, 4.3f, 4.8f};
     static const int per_cu[] = {4, 2, 2, 1};
     const int c = (D + 31) / 32 - 1;

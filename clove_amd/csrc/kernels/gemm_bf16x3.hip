@@ -39,8 +39,7 @@ constexpr uint32_t kOutside = 0x80000000u;     // past the end of both operands 
 // In LDS a piece of a slab is [R][BK] bf16, octet o of row r in slot o ^ ((r >>
 // 4) & 1) at BK = 16, o ^ ((r >> 2) & 3) at BK = 32: a wave's fragment read
 // (lane l: row l % 32, octet 2 step + l / 32) then touches every bank group
-// once per phase (0 SQ_LDS_BANK_CONFLICT cycles), and so do the KC = false
-// stores.
+// once per phase, and so do the KC = false stores.
 template <int R, int BK, int T, bool KC>
 struct Operand {
     static constexpr int OPR = BK / 8;  // octets per row

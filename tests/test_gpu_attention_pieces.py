@@ -99,7 +99,7 @@ def test_special_values(hip, D, S, past):
 
 def test_no_visible_key(hip):
     """Queries before every key get zeros, in split and unsplit launches."""
-    for S, Sk in ((64, 64), (10, 3000)):
+    for S, Sk in ((64, 64), (80, 80), (10, 3000)):
         g = rng(S)
         q = g.standard_normal((1, S, 256), dtype=np.float32)
         k, v = (g.standard_normal((1, Sk, 256), dtype=np.float32) for _ in range(2))
@@ -107,3 +107,12 @@ def test_no_visible_key(hip):
                                   k_pos=S - 4, flags=hip.ATTN_CAUSAL).numpy()
         assert np.all(got[0, :S - 4] == 0.0)
         assert np.array_equal(got[0, S - 4], v[0, 0])
+
+
+# Up to 64 queries and keys run on the FP32 MFMA, one more of either on the
+# bf16 pieces.
+@pytest.mark.parametrize("D", [8, 64, 80, 104, 128])
+@pytest.mark.parametrize("S,past", [(1, 63), (64, 0), (65, 0), (33, 31), (33, 32), (1, 64)])
+def test_short_calls(hip, D, S, past):
+    q, k, v = inputs(D + S, 2, S, past, 3, D)
+    check(run(hip, q, k, v, 3, past, True), attention64(q, k, v, 3, past, True), f"D={D} {S}+{past}")
