@@ -471,6 +471,8 @@ attention_x3_kernel(AttnArgs a) {
             }
         }
     };
+    // (a tile that Sk ends inside keeps the scalar offset at its first key, which is
+    // below Sk: a row past the end would carry it over 2^31 for k and v near 2 GiB)
     auto load_v = [&](int kb, auto whole) {
 #pragma unroll
         for (int u = 0; u < U; ++u)
@@ -478,9 +480,12 @@ attention_x3_kernel(AttnArgs a) {
             for (int e = 0; e < 8; ++e) {
                 const int ke = (e & 3) + 8 * (e >> 2);
                 uint32_t off = voff[u];
-                if constexpr (!decltype(whole)::value)
-                    off = kb + vkey[u] + ke < a.Sk ? off : kOutside;
-                xv[u][e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc_v, (int)off, (kb + ke) * HD * 4, 0));
+                int row = kb + ke;
+                if constexpr (!decltype(whole)::value) {
+                    off = kb + vkey[u] + ke < a.Sk ? off + (uint32_t)ke * (uint32_t)HD * 4u : kOutside;
+                    row = kb;
+                }
+                xv[u][e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc_v, (int)off, row * HD * 4, 0));
             }
     };
     auto split_octet = [&](const float *x, char *dst) {

@@ -116,3 +116,22 @@ def test_no_visible_key(hip):
 def test_short_calls(hip, D, S, past):
     q, k, v = inputs(D + S, 2, S, past, 3, D)
     check(run(hip, q, k, v, 3, past, True), attention64(q, k, v, 3, past, True), f"D={D} {S}+{past}")
+
+
+# Heads and keys whose k and v end just under 2 GiB, inside a block of 32 keys.
+@pytest.mark.parametrize("H,D,Sk", [(7, 64, 1198372), (7, 96, 798915)])
+def test_last_keys_near_2_gib(hip, H, D, Sk):
+    """The last block's byte offsets stay inside 32 bits up to the largest k and
+    v taken: a query that attends to the last Sk % 32 keys alone gets the mean
+    of their values (equal scores, the others' weights e^-200)."""
+    X, last = H * D, Sk % 32
+    assert 2**31 - 32 * X * 4 < Sk * X * 4 < 2**31 < (Sk - last + 11) * X * 4
+    k = hip.empty((1, Sk, X)).fill_uniform(0, 0.0, 0.0)
+    k.write((Sk - last) * X, np.full(last * X, 200 / np.sqrt(D), np.float32))
+    v = hip.empty((1, Sk, X)).fill_normal(7)
+    q = hip.tensor(np.ones((1, 1, X), np.float32))
+    got = hip.flash_attention(q, k, v, H, flags=0).numpy()[0, 0]
+    want = v.read((Sk - last) * X, last * X).reshape(last, X).astype(np.float64).mean(0)
+    assert np.max(np.abs(got - want)) <= 4 * 2.0**-24 * np.abs(want).max()
+    del k, v
+    hip.empty_cache()
