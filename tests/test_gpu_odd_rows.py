@@ -100,3 +100,21 @@ def test_odd_special_values(hip, cols):
     ok = ~np.isnan(want)
     assert_close(got[ok], want[ok], 1e-4, 1e-9, f"softmax special rows x{cols}")
     assert np.all(got[2, 1::2] == 0.0) and np.all(got[3, ::2] == 0.0)
+
+
+# The close softmax: odd widths of every kernel family, and every width past
+# 32768 columns (aligned ones in registers up to 53248, re-read past that).
+@pytest.mark.parametrize("cols", [67, 1001, 4099, 32769, 32772, 40000, 50257, 50304, 53248, 53252])
+def test_close_softmax_against_float64(hip, cols):
+    """Each entry against its row's largest, which the row sum's own rounding
+    leaves alone: y = y_max exp(x - x_max), x - x_max rounded to f32 as every
+    form does.  close_exp is within 1.5 ulp and the two quotients within half
+    of one each: 2.5 ulp of at most 2^-23."""
+    g = rng(cols)
+    x = g.normal(0, 4, (4, cols)).astype(np.float32)
+    y = hip.softmax(hip.tensor(x)).numpy().astype(np.float64)
+    top = np.arange(4), x.argmax(1)
+    d = (x - x[top][:, None]).astype(np.float64)
+    want = y[top][:, None] * np.exp(d)
+    assert np.max(np.abs(y - want) / want) <= 2.5 * 2.0**-23
+    assert np.all(np.abs(y.sum(1) - 1) <= 2.0**-24 * (cols / 512 + 16))
