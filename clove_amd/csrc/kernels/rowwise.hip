@@ -68,13 +68,29 @@ __device__ __forceinline__ float fast_exp(float x) {
 // exp(x) for x <= 0 to about 1.5 ulp: the rounding of x * log2(e) and the
 // part of log2(e) past f32 go back in as a first-order factor.  Below -200
 // (the result is 0 in f32 either way) x is held there, so -inf and the
-// lowest f32 give 0 and not inf - inf; a NaN stays one.
+// lowest f32 give 0 and not inf - inf; a NaN stays one.  The hardware 2^x gives
+// 0 where its result would be subnormal: SUB runs it 2^32 higher from there on
+// (the sum is exact), and is taken by a branch where x says so, since it is
+// a third more work on rows that hold no such entry (4 x 4000000: 1125 us
+// against 1337 with SUB throughout).
+constexpr float kExpNormal = -86.0f;  // e^x is normal from here on
+template <bool SUB>
 __device__ __forceinline__ float close_exp(float x) {
     x = x < -200.0f ? -200.0f : x;
     const float t = x * 0x1.715476p+0f;
     const float lo = __builtin_fmaf(x, 0x1.4ae0cp-26f, __builtin_fmaf(x, 0x1.715476p+0f, -t));
-    const float p = __builtin_amdgcn_exp2f(t);
-    return __builtin_fmaf(p, lo * 0.693147180559945f, p);
+    const float p = __builtin_amdgcn_exp2f(SUB ? t + 32.0f : t);
+    const float r = __builtin_fmaf(p, lo * 0.693147180559945f, p);
+    return SUB ? r * 0x1p-32f : r;
+}
+
+__device__ __forceinline__ float close_exp(float x) {
+    float r = close_exp<false>(x);
+    if (__builtin_expect(x < kExpNormal, 0)) {
+        asm volatile("");  // (keeps this a branch)
+        r = close_exp<true>(x);
+    }
+    return r;
 }
 
 // The softmax's exponential and final division.  Aligned rows of up to 32768
@@ -98,8 +114,20 @@ __device__ __forceinline__ float row_div(float e, float s, float inv) {
 
 template <bool CLOSE>
 __device__ __forceinline__ cl_f4 row_exp4(cl_f4 v, float m) {
-    return (cl_f4){row_exp<CLOSE>(v.x - m), row_exp<CLOSE>(v.y - m), row_exp<CLOSE>(v.z - m),
-                   row_exp<CLOSE>(v.w - m)};
+    const cl_f4 d = v - m;
+    if constexpr (!CLOSE) {
+        return (cl_f4){fast_exp(d.x), fast_exp(d.y), fast_exp(d.z), fast_exp(d.w)};
+    } else {
+        cl_f4 r;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) r[k] = close_exp<false>(d[k]);
+        if (__builtin_expect(fminf(fminf(d.x, d.y), fminf(d.z, d.w)) < kExpNormal, 0)) {
+            asm volatile("");
+#pragma unroll
+            for (int k = 0; k < 4; ++k) r[k] = close_exp(d[k]);
+        }
+        return r;
+    }
 }
 
 template <bool CLOSE>
@@ -785,9 +813,10 @@ __global__ void __launch_bounds__(kBlockThreads) cross_entropy_rows2_kernel(
 // (from the last-level cache) where its values are needed a second time.
 constexpr int kLoopVec = 4;
 
-// f(j, x) for every element j of a row of `cols`, this thread's share.
-template <class F>
-__device__ __forceinline__ void row_walk(const float *row, int cols, F f) {
+// This thread's share of a row of `cols`: fv(j, v) for its whole vectors, the
+// elements j .. j + 3, and f(j, x) for its one of the last cols % 4.
+template <class FV, class F>
+__device__ __forceinline__ void row_walk4(const float *row, int cols, FV fv, F f) {
     const int nvec = cols >> 2;
     for (int c0 = threadIdx.x; c0 < nvec; c0 += kLoopVec * kBlockThreads) {
         cl_f4 v[kLoopVec];
@@ -799,31 +828,42 @@ __device__ __forceinline__ void row_walk(const float *row, int cols, F f) {
 #pragma unroll
         for (int u = 0; u < kLoopVec; ++u) {
             const int c = c0 + u * kBlockThreads;
-            if (c < nvec)
-#pragma unroll
-                for (int k = 0; k < 4; ++k) f(4 * c + k, v[u][k]);
+            if (c < nvec) fv(4 * c, v[u]);
         }
     }
     const int j = 4 * nvec + threadIdx.x;
     if ((int)threadIdx.x < (cols & 3)) f(j, row[j]);
 }
 
+// f(j, x) for every element of it.
+template <class F>
+__device__ __forceinline__ void row_walk(const float *row, int cols, F f) {
+    row_walk4(
+        row, cols,
+        [&](int j, cl_f4 v) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) f(j + k, v[k]);
+        },
+        f);
+}
+
 // The row's max and sum of exp(x - max) in one walk: a running max and a sum
 // relative to it per thread, the threads' sums then brought to the row's max.
 // A max of -inf counts as 0 in the subtractions (-inf entries give 0, not
-// NaN); NaN entries reach the sum.  A row of -inf alone sums to 0.
+// NaN); NaN entries reach the sum.  A row of -inf alone sums to 0.  (The sum is
+// 1 or more: a subnormal term is no part of it.)
 __device__ __forceinline__ void row_max_sum(const float *row, int cols, float red[2][kBlockWaves],
                                             float *m_out, float *s_out) {
     float m = -INFINITY, s = 0.0f;
     row_walk(row, cols, [&](int, float x) {
         if (x > m) {
-            s *= m == -INFINITY ? 1.0f : close_exp(m - x);
+            s *= m == -INFINITY ? 1.0f : close_exp<false>(m - x);
             m = x;
         }
-        s += close_exp(x - (m == -INFINITY ? 0.0f : m));
+        s += close_exp<false>(x - (m == -INFINITY ? 0.0f : m));
     });
     const float gm = block_max(m, red[0]);
-    if (m != -INFINITY) s *= close_exp(m - gm);
+    if (m != -INFINITY) s *= close_exp<false>(m - gm);
     *m_out = gm;
     *s_out = block_sum(s, red[1]);
 }
@@ -837,7 +877,12 @@ __global__ void __launch_bounds__(kBlockThreads) softmax_loop_kernel(const float
     float m, s;
     row_max_sum(xr, cols, red, &m, &s);
     const float inv = 1.0f / s;
-    row_walk(xr, cols, [&](int j, float v) { yr[j] = row_div<true>(close_exp(v - m), s, inv); });
+    row_walk4(
+        xr, cols,
+        [&](int j, cl_f4 v) {
+            *reinterpret_cast<cl_f4u *>(yr + j) = row_div4<true>(row_exp4<true>(v, m), s, inv);
+        },
+        [&](int j, float v) { yr[j] = row_div<true>(close_exp(v - m), s, inv); });
 }
 
 __global__ void __launch_bounds__(kBlockThreads) layer_norm_loop_kernel(

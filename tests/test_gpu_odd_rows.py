@@ -118,3 +118,19 @@ def test_close_softmax_against_float64(hip, cols):
     want = y[top][:, None] * np.exp(d)
     assert np.max(np.abs(y - want) / want) <= 2.5 * 2.0**-23
     assert np.all(np.abs(y.sum(1) - 1) <= 2.0**-24 * (cols / 512 + 16))
+
+
+@pytest.mark.parametrize("cols", [7, 67, 1001, 4099, 32772, 50257, 60001])
+def test_close_softmax_subnormal_entries(hip, cols):
+    """Entries between 2^-149 and 2^-126 of the largest are subnormal, not 0;
+    the exponential, the quotient and the largest entry round once each, by at
+    most half of 2^-149 here."""
+    g = rng(cols)
+    x = g.uniform(-105, -80, (3, cols)).astype(np.float32)
+    x[:, cols // 3] = 0.0
+    x[1, cols - 1] = 1.0
+    y = hip.softmax(hip.tensor(x)).numpy().astype(np.float64)
+    top = np.arange(3), x.argmax(1)
+    want = y[top][:, None] * np.exp((x - x[top][:, None]).astype(np.float64))
+    assert np.any((want > 0) & (want < 2.0**-127))
+    assert np.all(np.abs(y - want) <= 2.5 * 2.0**-23 * want + 1.5 * 2.0**-149)
