@@ -471,8 +471,9 @@ attention_x3_kernel(AttnArgs a) {
             }
         }
     };
-    // (a tile that Sk ends inside keeps the scalar offset at its first key, which is
-    // below Sk: a row past the end would carry it over 2^31 for k and v near 2 GiB)
+    // (in a tile that Sk ends inside the scalar offset stops at the last row: past it
+    // every lane is outside, and for k and v near 2 GiB the row's offset would pass
+    // 2^31.  Adding the row to the lanes' offsets instead spilled registers.)
     auto load_v = [&](int kb, auto whole) {
 #pragma unroll
         for (int u = 0; u < U; ++u)
@@ -482,8 +483,8 @@ attention_x3_kernel(AttnArgs a) {
                 uint32_t off = voff[u];
                 int row = kb + ke;
                 if constexpr (!decltype(whole)::value) {
-                    off = kb + vkey[u] + ke < a.Sk ? off + (uint32_t)ke * (uint32_t)HD * 4u : kOutside;
-                    row = kb;
+                    off = row + vkey[u] < a.Sk ? off : kOutside;
+                    row = min(row, a.Sk - 1);
                 }
                 xv[u][e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc_v, (int)off, row * HD * 4, 0));
             }
