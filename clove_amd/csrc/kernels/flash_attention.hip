@@ -339,8 +339,8 @@ __device__ __forceinline__ void attention_f32(const AttnArgs &a, const int q0, c
 // keys, 5.9e-7 at 1031 keys unsplit, less split).
 //  * A workgroup that meets a value under 2^-102 in q, k or v, or ends with a
 //    sum that is not finite, computes its queries again with attention_f32.
-//    (A softmax weight may be that small: it is then under 2^-90 of the
-//    query's largest, and its pieces lose bits under 2^-126 at most.)
+//    Weights are taken relative to 2^-24 of the largest, so that all that f32
+//    holds relative to the largest (down to 2^-126) keep their pieces whole.
 template <int D, bool CAUSAL, int NW>
 __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)))
 attention_x3_kernel(AttnArgs a) {
@@ -590,10 +590,12 @@ attention_x3_kernel(AttnArgs a) {
 #pragma unroll
         for (int i = 0; i < 16; ++i) mloc = fmaxf(mloc, s[i]);
         mloc = fmaxf(mloc, __shfl_xor(mloc, 32, 64));
-        // lazy rescale, as in attention_f32
-        constexpr float kSlack = 8.0f;
-        if (__any(mloc > m + kSlack)) {
-            const float m_new = fmaxf(m, mloc);
+        // lazy rescale, as in attention_f32, but m stays 24 below the maximum: a
+        // weight goes up to 2^(24 + kSlack), and one of 2^-126 of the largest is
+        // 2^-102, whose third piece is still no bf16 subnormal
+        constexpr float kSlack = 8.0f, kLift = 24.0f;
+        if (__any(mloc - kLift > m + kSlack)) {
+            const float m_new = fmaxf(m, mloc - kLift);
             const float alpha = m_new == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m - m_new);
             lsum *= alpha;
 #pragma unroll
@@ -604,7 +606,7 @@ attention_x3_kernel(AttnArgs a) {
         }
         const float mz = m == -INFINITY ? 0.0f : m;
         float ps = 0.0f;
-        us2 any_size = {0xffff, 0xffff};  // weights may be tiny
+        us2 any_size = {0xffff, 0xffff};  // (a weight under 2^-126 of the largest may be tiny)
         // step t's weights, then its products; step 1's exponentials and splits
         // fall between step 0's MFMAs
 #pragma unroll

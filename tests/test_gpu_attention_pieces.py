@@ -135,3 +135,20 @@ def test_last_keys_near_2_gib(hip, H, D, Sk):
     assert np.max(np.abs(got - want)) <= 4 * 2.0**-24 * np.abs(want).max()
     del k, v
     hip.empty_cache()
+
+
+@pytest.mark.parametrize("D", [32, 64, 96, 128])
+@pytest.mark.parametrize("S,Sk", [(4, 200), (4, 3000), (300, 300)])
+def test_small_weights_keep_their_bits(hip, D, S, Sk):
+    """A weight of 2^-125.x of the largest on the one value that is not 0, and
+    large enough to make up for it.  Its score's rounding, 126 ln 2 2^-24 of the
+    weight, and that of the q . k sum bound the error: 2e-5."""
+    g = rng(D + Sk)
+    q = np.ones((1, S, D), np.float32)
+    k = np.zeros((1, Sk, D), np.float32)
+    v = np.zeros((1, Sk, D), np.float32)
+    k[0, Sk // 2, 0] = -125.3 * np.log(2) * np.sqrt(D)
+    v[0, Sk // 2] = g.uniform(0.5, 1, D) * 2.0**90
+    got = hip.flash_attention(hip.tensor(q), hip.tensor(k), hip.tensor(v), 1, flags=0).numpy()
+    want = attention64(q, k, v, 1, 0, False)
+    assert np.max(np.abs(got - want) / want) <= 2e-5
