@@ -20,9 +20,13 @@ typedef float f2 __attribute__((ext_vector_type(2)));
 typedef unsigned u4 __attribute__((ext_vector_type(4)));
 typedef unsigned short us2 __attribute__((ext_vector_type(2)));
 
-// split_pair's tiny key of 2^-102: a least key below it means that some value
-// was too small for its pieces.
-constexpr unsigned short kTinyKey = 2 * (25 << 7);
+// Operands are split as 2^24 x.  A value's lowest bit is 2^-149 or more, so no
+// piece is then a bf16 subnormal, and a product of operands, 2^48 times larger,
+// is normal wherever f32 holds it at all; the factor comes off the sums at the
+// end, exactly (or with the one rounding of a subnormal result).  |x| of 2^103
+// and sums of 2^79 overflow instead: those, infinities and NaN end as a sum that
+// is not finite, which is where a kernel takes the f32 values instead.
+constexpr float kPieceScale = 0x1p24f, kPieceUnscale = 0x1p-24f, kSumUnscale = 0x1p-48f;
 
 // The six products, smallest first: piece of the first operand, of the second.
 constexpr int kPieceA[6] = {2, 0, 1, 1, 0, 0}, kPieceB[6] = {0, 2, 1, 0, 1, 0};
@@ -30,6 +34,26 @@ constexpr int kPieceA[6] = {2, 0, 1, 1, 0, 0}, kPieceB[6] = {0, 2, 1, 0, 1, 0};
 __device__ __forceinline__ unsigned bf16_pair(float a, float b) {
     return __builtin_bit_cast(unsigned, __builtin_convertvector((f2){a, b}, bf2));
 }
+
+// Two floats, times 2^24 with SCALE, as one dword of each of the three pieces.
+template <bool SCALE>
+__device__ __forceinline__ void split_pair(float a, float b, unsigned *p1, unsigned *p2,
+                                           unsigned *p3) {
+    if constexpr (SCALE) {
+        a *= kPieceScale;
+        b *= kPieceScale;
+    }
+    const unsigned h = bf16_pair(a, b);
+    const float ra = a - __uint_as_float(h << 16), rb = b - __uint_as_float(h & 0xffff0000u);
+    const unsigned m = bf16_pair(ra, rb);
+    *p1 = h;
+    *p2 = m;
+    *p3 = bf16_pair(ra - __uint_as_float(m << 16), rb - __uint_as_float(m & 0xffff0000u));
+}
+
+// For operands that are not scaled: the tiny key of 2^-102: a least key below it means that some value
+// was too small for its pieces.
+constexpr unsigned short kTinyKey = 2 * (25 << 7);
 
 // Two floats as one dword of each of the three pieces.  *tiny keeps the least
 // 2 |x1| - 1 seen, as 16-bit integers of the bf16 bits (a zero wraps to the

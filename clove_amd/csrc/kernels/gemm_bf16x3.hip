@@ -11,8 +11,8 @@
 // 64 1.13e-7, 512 3.5e-7, 1024 4.8e-7, 4096 1.02e-6 -- the FP32 MFMA kernel
 // 1.44e-7, 4.1e-7, 5.7e-7, 1.15e-6.
 //
-// A value below 2^-102 (its pieces would reach bf16's subnormals), an
-// infinity, a NaN or a sum that leaves f32's range is not for this scheme: the
+// Operands go in as 2^24 x (bf16x3.h), which holds every value below 2^103.  One
+// past that, an infinity, a NaN or a sum past 2^79 is not for this scheme: the
 // workgroup that meets one computes its tile again from the f32 values on the
 // FP32 MFMA (redo below), so the result is then what f32 arithmetic gives.
 #include <hip/hip_runtime.h>
@@ -112,17 +112,17 @@ struct Operand {
             }
     }
     // the pieces of the loaded slab into `stage` (piece p at p * kPiece)
-    __device__ __forceinline__ void store(char *stage, us2 *tiny) const {
+    __device__ __forceinline__ void store(char *stage) const {
 #pragma unroll
-        for (int u = 0; u < OCT; ++u) store_octet(u, stage, tiny);
+        for (int u = 0; u < OCT; ++u) store_octet(u, stage);
     }
-    __device__ __forceinline__ void store_octet(int u, char *stage, us2 *tiny) const {
+    __device__ __forceinline__ void store_octet(int u, char *stage) const {
         {
             u4 p[3];
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 unsigned a, b, c;
-                split_pair(x[u][2 * e], x[u][2 * e + 1], &a, &b, &c, tiny);
+                split_pair<true>(x[u][2 * e], x[u][2 * e + 1], &a, &b, &c);
                 p[0][e] = a;
                 p[1][e] = b;
                 p[2][e] = c;
@@ -206,11 +206,10 @@ gemm_bf16x3_kernel(GemmArgs g) {
                 for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
     };
     clear();
-    us2 tiny = {0xffff, 0xffff};
     auto store = [&](int s) {
         char *st = smem + (s & 1) * STAGE;
-        a.store(st, &tiny);
-        b.store(st + SA, &tiny);
+        a.store(st);
+        b.store(st + SA);
     };
     // this lane's octet of each MFMA step in a 32-row block
     int rd[BK / 16];
@@ -251,8 +250,8 @@ gemm_bf16x3_kernel(GemmArgs g) {
 #pragma unroll
             for (int u = r * UNITS / REG; u < (r + 1) * UNITS / REG; ++u) {
                 if constexpr (decltype(next)::value) {
-                    if (u < OpA::OCT) a.store_octet(u, nst, &tiny);
-                    else b.store_octet(u - OpA::OCT, nst + SA, &tiny);
+                    if (u < OpA::OCT) a.store_octet(u, nst);
+                    else b.store_octet(u - OpA::OCT, nst + SA);
                 }
                 if constexpr (decltype(load_more)::value) {
                     if (u < OpA::OCT) a.load_octet(u, k2);
@@ -289,20 +288,18 @@ gemm_bf16x3_kernel(GemmArgs g) {
     }
     step(s, No{}, No{});
 
-    // Out of the pieces' range?  An operand value below 2^-102 (tiny), or a
-    // sum that is not finite (which an infinite or NaN operand, or one that
-    // rounds to infinity in bf16, always gives) or is below 2^-102 itself.
-    bool bad = min(tiny.x, tiny.y) < kTinyKey;
+    // Out of the pieces' range?  An infinite or NaN operand, or one that rounds to
+    // infinity in bf16, always gives a sum that is not finite.
+    bool bad = false;
 #pragma unroll
     for (int i = 0; i < IB; ++i)
 #pragma unroll
         for (int j = 0; j < JB; ++j)
 #pragma unroll
-            for (int e = 0; e < 16; ++e) {
-                const float v = __builtin_fabsf(acc[i][j][e]);
-                bad = bad || !(v < INFINITY) || (v < 0x1p-102f && v != 0.0f);
-            }
+            for (int e = 0; e < 16; ++e) bad = bad || !(__builtin_fabsf(acc[i][j][e]) < INFINITY);
+    float unscale = kSumUnscale;
     if (__builtin_expect(__syncthreads_or(bad), 0)) {
+        unscale = 1.0f;
         // redo: the same tile from the f32 values on v_mfma_f32_32x32x2_f32,
         // one slab in LDS at a time.
         clear();
@@ -354,7 +351,7 @@ gemm_bf16x3_kernel(GemmArgs g) {
                 for (int j = 0; j < JB; ++j) {
                     const int row = m0 + wm0 + 32 * i + 8 * (e / 4) + 4 * h + (e % 4);
                     const int col = n0 + wn0 + 32 * j + l32;
-                    float v = acc[i][j][e];
+                    float v = acc[i][j][e] * unscale;
                     if constexpr (EPI) v = epilogue(g.epi, v, row, col, N, &bc[j]);
                     if (row < M && col < N) g.C[(size_t)row * N + col] = v;
                 }
@@ -368,7 +365,7 @@ gemm_bf16x3_kernel(GemmArgs g) {
 #pragma unroll
             for (int j = 0; j < JB; ++j)
                 part[(wm0 + 32 * i + 8 * (e / 4) + 4 * h + (e % 4)) * BN + wn0 + 32 * j + l32] =
-                    acc[i][j][e];
+                    acc[i][j][e] * unscale;
 }
 
 template <int BM, int BN, int BK, int WM, int WN, int T, int MINW>

@@ -156,3 +156,41 @@ def test_plan_takes_special_values(hip):
     assert np.array_equal(got[inf], want[inf].astype(np.float32))
     ok = np.isfinite(want)
     assert np.max(np.abs(got[ok] - want[ok])) < 1e-3
+
+
+@pytest.mark.parametrize("cfg", TILES)
+def test_small_operands_keep_every_bit(hip, monkeypatch, cfg):
+    """The same down to f32's smallest: every bit of values from 2^-149 on,
+    beside ordinary ones, and products of two small operands."""
+    monkeypatch.setenv("CLOVE_GEMM_CFG", cfg)
+    g = rng(12)
+    a = g.standard_normal((300, 256)).astype(np.float32)
+    a[:, 1::2] *= np.exp2(g.integers(-149, -100, (300, 128))).astype(np.float32)
+    eye = np.eye(256, dtype=np.float32)
+    assert np.array_equal(hip.matmul(hip.tensor(a), hip.tensor(eye)).numpy(), a)
+    b = (eye[g.permutation(256)] * np.exp2(g.integers(-80, 20, 256))).astype(np.float32)
+    want = (a.astype(np.float64) @ b.astype(np.float64)).astype(np.float32)  # rounded once
+    assert np.array_equal(hip.matmul(hip.tensor(a), hip.tensor(b)).numpy(), want)
+
+
+def best_ms(hip, call, reps=10):
+    call()
+    times = []
+    for _ in range(3):
+        e0 = hip.event_record()
+        for _ in range(reps):
+            call()
+        times.append(hip.event_elapsed(e0, hip.event_record()))
+        hip.event_reset()
+    return min(times)
+
+
+def test_small_operands_cost_nothing(hip):
+    """A tiny value per 256 rows, as softmax and loss gradients hold them, does
+    not send its tiles to a second computation (which took 2.6 times as long)."""
+    n = 4096
+    a, b = hip.empty((n, n)).fill_normal(1), hip.empty((n, n)).fill_normal(2)
+    plain = best_ms(hip, lambda: hip.matmul(a, b))
+    for r in range(0, n, 256):
+        a.write(r * n + 5, np.array([1e-33, 1e-40], np.float32))
+    assert best_ms(hip, lambda: hip.matmul(a, b)) <= 1.3 * plain
