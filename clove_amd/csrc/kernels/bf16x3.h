@@ -18,7 +18,6 @@ typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
 typedef float f2 __attribute__((ext_vector_type(2)));
 typedef unsigned u4 __attribute__((ext_vector_type(4)));
-typedef unsigned short us2 __attribute__((ext_vector_type(2)));
 
 // Operands are split as 2^24 x.  A value's lowest bit is 2^-149 or more, so no
 // piece is then a bf16 subnormal, and a product of operands, 2^48 times larger,
@@ -49,25 +48,6 @@ __device__ __forceinline__ void split_pair(float a, float b, unsigned *p1, unsig
     *p1 = h;
     *p2 = m;
     *p3 = bf16_pair(ra - __uint_as_float(m << 16), rb - __uint_as_float(m & 0xffff0000u));
-}
-
-// For operands that are not scaled: the tiny key of 2^-102: a least key below it means that some value
-// was too small for its pieces.
-constexpr unsigned short kTinyKey = 2 * (25 << 7);
-
-// Two floats as one dword of each of the three pieces.  *tiny keeps the least
-// 2 |x1| - 1 seen, as 16-bit integers of the bf16 bits (a zero wraps to the
-// largest): the smallest nonzero magnitude, at one operation per value.
-__device__ __forceinline__ void split_pair(float a, float b, unsigned *p1, unsigned *p2,
-                                           unsigned *p3, us2 *tiny) {
-    const unsigned h = bf16_pair(a, b);
-    const float ra = a - __uint_as_float(h << 16), rb = b - __uint_as_float(h & 0xffff0000u);
-    const unsigned m = bf16_pair(ra, rb);
-    *p1 = h;
-    *p2 = m;
-    *p3 = bf16_pair(ra - __uint_as_float(m << 16), rb - __uint_as_float(m & 0xffff0000u));
-    const us2 key = __builtin_bit_cast(us2, h) * (us2){2, 2} + (us2){0xffff, 0xffff};
-    *tiny = __builtin_elementwise_min(*tiny, key);
 }
 
 // LDS contents are published by a wait for this wave's LDS operations and a

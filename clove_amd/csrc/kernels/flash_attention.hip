@@ -55,11 +55,13 @@ typedef float f16v __attribute__((ext_vector_type(16)));
 // Writes a lane's query: o[j][e] = O[query][32j + 8(e/4) + 4hh + e%4], four
 // consecutive dims per e/4; the output itself, or with the keys split over
 // workgroups the unnormalised sum and (m, lsum) for attention_merge_kernel.
+// unscale: the factor that o is to be brought back by.
 template <int D, int kJ>
 __device__ __forceinline__ void attn_store(const AttnArgs &a, int b, int h, int query, int split,
-                                           int hh, const f16v (&o)[kJ], float m, float lsum) {
+                                           int hh, const f16v (&o)[kJ], float m, float lsum,
+                                           float unscale) {
     const size_t row = (size_t)b * a.S + query;
-    float inv = 1.0f, *orow = a.out + (row * a.H + h) * a.D;
+    float inv = unscale, *orow = a.out + (row * a.H + h) * a.D;
     if (a.splits > 1) {
         const size_t rows = (size_t)a.B * a.S * a.H, at = (size_t)split * rows + row * a.H + h;
         orow = a.part + at * a.D;
@@ -69,7 +71,7 @@ __device__ __forceinline__ void attn_store(const AttnArgs &a, int b, int h, int 
             st[1] = lsum;
         }
     } else {
-        inv = lsum > 0.0f ? 1.0f / lsum : 0.0f;
+        inv = lsum > 0.0f ? unscale / lsum : 0.0f;
     }
 #pragma unroll
     for (int j = 0; j < kJ; ++j)
@@ -310,7 +312,7 @@ __device__ __forceinline__ void attention_f32(const AttnArgs &a, const int q0, c
         __syncthreads();
     }
 
-    if (q_ok) attn_store<D, kJ>(a, b, h, query, split, hh, o, m, lsum);
+    if (q_ok) attn_store<D, kJ>(a, b, h, query, split, hh, o, m, lsum, 1.0f);
 }
 
 // Head dims up to 128 that are multiples of 8, on the bf16 matrix cores, f32
@@ -337,8 +339,11 @@ __device__ __forceinline__ void attention_f32(const AttnArgs &a, const int q0, c
 // block (3.9 us at D = 128 alone on its CU, 1.8 at D = 64), hence the splits.
 // Error against float64 is below that kernel's (2.9e-7 against 3.7e-7 at 377
 // keys, 5.9e-7 at 1031 keys unsplit, less split).
-//  * A workgroup that meets a value under 2^-102 in q, k or v, or ends with a
-//    sum that is not finite, computes its queries again with attention_f32.
+//  * q (times scale * log2(e)), k and v go in as 2^24 x; a score's factor of 2^48
+//    comes off in the exponent's FMA, the output's 2^24 at the end.  A workgroup
+//    that ends with a sum that is not finite (an infinity, a NaN, a value of
+//    2^103, a score of 2^79, a v around 2^65 over many keys) computes its queries
+//    again with attention_f32.
 //    Weights are taken relative to 2^-24 of the largest, so that all that f32
 //    holds relative to the largest (down to 2^-126) keep their pieces whole.
 template <int D, bool CAUSAL, int NW>
@@ -367,16 +372,15 @@ attention_x3_kernel(AttnArgs a) {
     const int qw0 = q0 + wave * 32;
     const int query = qw0 + l32;
     const bool q_ok = query < a.S;
-    us2 tiny = {0xffff, 0xffff};
 
     // this wave's Q^T pieces: step g, slots 0..7 of lane half hh are dims 16g +
-    // 8hh .. +7 of its query, rotated (with RoPE) and times scale * log2(e), in
-    // f32 as in attention_f32, before the split
+    // 8hh .. +7 of its query, rotated (with RoPE) and times 2^24 scale * log2(e),
+    // in f32 as in attention_f32, before the split
     const float *qrow = a.q + ((size_t)b * a.S + (q_ok ? query : 0)) * HD + (size_t)h * DD;
     const float2 *trow = a.rope_tab && q_ok
                              ? a.rope_tab + (size_t)(query + a.q_pos - a.tab_pos0) * (DD / 2)
                              : nullptr;
-    const float qscale = a.scale * 1.44269504088896341f;
+    const float qscale = a.scale * 1.44269504088896341f * kPieceScale;
     bf8 qf[ST][3];
 #pragma unroll
     for (int g = 0; g < ST; ++g) {
@@ -400,7 +404,7 @@ attention_x3_kernel(AttnArgs a) {
 #pragma unroll
             for (int e = 0; e < 2; ++e) {
                 unsigned x, y, z;
-                split_pair(v[2 * e], v[2 * e + 1], &x, &y, &z, &tiny);
+                split_pair<false>(v[2 * e], v[2 * e + 1], &x, &y, &z);
                 p[0][2 * c + e] = x;
                 p[1][2 * c + e] = y;
                 p[2][2 * c + e] = z;
@@ -494,7 +498,7 @@ attention_x3_kernel(AttnArgs a) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             unsigned x1, x2, x3;
-            split_pair(x[2 * e], x[2 * e + 1], &x1, &x2, &x3, &tiny);
+            split_pair<true>(x[2 * e], x[2 * e + 1], &x1, &x2, &x3);
             p[0][e] = x1;
             p[1][e] = x2;
             p[2][e] = x3;
@@ -575,7 +579,7 @@ attention_x3_kernel(AttnArgs a) {
                                                             0);
             if (g == 0) stage_k();
         }
-        // s[i] is the score of key kb + 8(i/4) + 4hh + i%4 (base-2 units)
+        // s[i] is the score of key kb + 8(i/4) + 4hh + i%4 (base-2 units, times 2^48)
         if constexpr (!kSteady) {
             bool full = kb + kBK <= a.Sk && qw0 + 32 <= a.S;
             if (CAUSAL) full = full && kb + kBK - 1 + a.k_pos <= qw0 + a.q_pos;
@@ -589,7 +593,7 @@ attention_x3_kernel(AttnArgs a) {
         float mloc = -INFINITY;
 #pragma unroll
         for (int i = 0; i < 16; ++i) mloc = fmaxf(mloc, s[i]);
-        mloc = fmaxf(mloc, __shfl_xor(mloc, 32, 64));
+        mloc = fmaxf(mloc, __shfl_xor(mloc, 32, 64)) * kSumUnscale;
         // lazy rescale, as in attention_f32, but m stays 24 below the maximum: a
         // weight goes up to 2^(24 + kSlack), and one of 2^-126 of the largest is
         // 2^-102, whose third piece is still no bf16 subnormal
@@ -606,7 +610,6 @@ attention_x3_kernel(AttnArgs a) {
         }
         const float mz = m == -INFINITY ? 0.0f : m;
         float ps = 0.0f;
-        us2 any_size = {0xffff, 0xffff};  // (a weight under 2^-126 of the largest may be tiny)
         // step t's weights, then its products; step 1's exponentials and splits
         // fall between step 0's MFMAs
 #pragma unroll
@@ -615,12 +618,12 @@ attention_x3_kernel(AttnArgs a) {
             u4 pw[3];
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                const float w0 = __builtin_amdgcn_exp2f(s[8 * t + 2 * e] - mz);
-                const float w1 = __builtin_amdgcn_exp2f(s[8 * t + 2 * e + 1] - mz);
+                const float w0 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[8 * t + 2 * e], kSumUnscale, -mz));
+                const float w1 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[8 * t + 2 * e + 1], kSumUnscale, -mz));
                 ps += w0;
                 ps += w1;
                 unsigned x1, x2, x3;
-                split_pair(w0, w1, &x1, &x2, &x3, &any_size);
+                split_pair<false>(w0, w1, &x1, &x2, &x3);
                 pw[0][e] = x1;
                 pw[1][e] = x2;
                 pw[2][e] = x3;
@@ -655,7 +658,7 @@ attention_x3_kernel(AttnArgs a) {
     for (; blk < steady; ++blk) block(blk, Yes{});
     for (; blk < blk1; ++blk) block(blk, No{});
 
-    bool bad = min(tiny.x, tiny.y) < kTinyKey || !(lsum < INFINITY);
+    bool bad = !(lsum < INFINITY);
 #pragma unroll
     for (int j = 0; j < kJ; ++j)
 #pragma unroll
@@ -664,7 +667,7 @@ attention_x3_kernel(AttnArgs a) {
         attention_f32<D, CAUSAL, T>(a, q0, bh, split, blk0, blk1, reinterpret_cast<float *>(smem));
         return;
     }
-    if (q_ok) attn_store<D, kJ>(a, b, h, query, split, hh, o, m, lsum);
+    if (q_ok) attn_store<D, kJ>(a, b, h, query, split, hh, o, m, lsum, kPieceUnscale);
 }
 
 // Adds the key splits of every (row, head): O = sum O_p 2^(m_p - M) / sum l_p

@@ -152,3 +152,39 @@ def test_small_weights_keep_their_bits(hip, D, S, Sk):
     got = hip.flash_attention(hip.tensor(q), hip.tensor(k), hip.tensor(v), 1, flags=0).numpy()
     want = attention64(q, k, v, 1, 0, False)
     assert np.max(np.abs(got - want) / want) <= 2e-5
+
+
+def test_small_operands_cost_nothing(hip):
+    """Tiny values in k or v do not send their heads' queries to a second
+    computation (which took 2.2 times as long)."""
+    S, X = 4096, 2048
+    q, k, v = (hip.empty((1, S, X)).fill_normal(i) for i in (1, 2, 3))
+
+    def best_ms():
+        times = []
+        for _ in range(4):
+            e0 = hip.event_record()
+            for _ in range(10):
+                hip.flash_attention(q, k, v, 16, flags=hip.ATTN_CAUSAL)
+            times.append(hip.event_elapsed(e0, hip.event_record()))
+            hip.event_reset()
+        return min(times)
+
+    plain = best_ms()
+    for h in range(16):
+        k.write(7 * X + 128 * h, np.array([1e-33, 1e-40], np.float32))
+        v.write(9 * X + 128 * h, np.array([1e-33, 1e-40], np.float32))
+    assert best_ms() <= 1.3 * plain
+
+
+@pytest.mark.parametrize("D", [32, 64, 96, 128])
+def test_small_values_keep_their_bits(hip, D):
+    """v down to f32's smallest: a query that attends to one key alone (its
+    score 200 above the others) gets that key's row, every bit of it."""
+    g = rng(D)
+    S = 300
+    q, k = np.ones((1, S, D), np.float32), np.zeros((1, S, D), np.float32)
+    k[0, 77] = 200 / np.sqrt(D)
+    v = (g.standard_normal((1, S, D)) * np.exp2(g.integers(-149, -90, (1, S, D)))).astype(np.float32)
+    got = hip.flash_attention(hip.tensor(q), hip.tensor(k), hip.tensor(v), 1, flags=0).numpy()
+    assert np.array_equal(got[0], np.broadcast_to(v[0, 77], (S, D)))
