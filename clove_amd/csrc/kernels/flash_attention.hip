@@ -10,8 +10,9 @@
 //
 // Head dims up to 128 that are multiples of 8 run attention_x3_kernel below, on
 // the bf16 matrix cores with every f32 value as three bf16 pieces (bf16x3.h);
-// every other head dim runs attention16_kernel (attention_general.hip), 16-query
-// waves on the FP32 MFMA.  Key blocks of 32 are staged through LDS
+// every other head dim, and calls that attention_x3_plan prices as faster there
+// (short ones above all), run attention16_kernel (attention_general.hip),
+// 16-query waves on the FP32 MFMA.  Key blocks of 32 are staged through LDS
 // (double-buffered, one barrier per block).  k is rotated before the kernel,
 // once per element (a rotation inside it would be repeated by every query block
 // that stages the same keys).  The products run in TRANSPOSED form:
@@ -824,8 +825,8 @@ __global__ void __launch_bounds__(256) rope_pairs_kernel(const float *__restrict
 
 bool attention_supported(int head_dim) { return head_dim >= 1 && head_dim <= kAttnMaxHeadDim; }
 
-// Tile size, query blocks and key splits of the bf16x3 kernel; qb = 0: not its
-// head dim.
+// Tile size, query blocks and key splits of the bf16x3 kernel; qb = 0: the FP32
+// MFMA kernel's call.
 //
 // Splitting the keys of a query block over workgroups pays where the blocks
 // alone leave CUs idle or one long block finishes last (64 queries over 2064
@@ -839,6 +840,41 @@ bool attention_supported(int head_dim) { return head_dim >= 1 && head_dim <= kAt
 struct AttnX3Plan {
     int dp, qb, splits;
 };
+
+// 32-key blocks of one head's query blocks of qb queries: their sum, and the
+// longest's.
+struct AttnBlocks {
+    double sum;
+    int most, nqb;
+};
+static AttnBlocks attention_blocks(int S, int Sk, int q_pos, int k_pos, bool causal, int qb) {
+    AttnBlocks r{0.0, 0, (S + qb - 1) / qb};
+    for (int i = 0; i < r.nqb; ++i) {
+        int64_t end = Sk;
+        if (causal)
+            end = std::min<int64_t>(end, std::min<int64_t>((int64_t)(i + 1) * qb, S) + q_pos - k_pos);
+        const int n = end > 0 ? (int)((end + kBK - 1) / kBK) : 0;
+        r.sum += n;
+        r.most = std::max(r.most, n);
+    }
+    return r;
+}
+
+// A whole call's time in us on a kernel that holds per_cu workgroups on a CU: the
+// longer of its longest workgroup (lone us per key block alone on its CU, up to
+// 1 + share times that beside others) and of all of them over the slots (full us
+// per block and slot), pro blocks of prologue each.
+struct AttnPrice {
+    double lone, full, base, pro, share;
+    int per_cu;
+};
+static double attention_us(const AttnPrice &k, double heads, double sum, double wgs, int longest,
+                           int num_cus) {
+    const double beside = std::min(std::max(wgs * heads / num_cus - 1.0, 0.0), k.per_cu - 1.0);
+    return k.base + std::max((longest + k.pro) * k.lone * (1.0 + k.share * beside),
+                             heads * (sum + k.pro * wgs) / (k.per_cu * num_cus) * k.full);
+}
+
 // Up to 64 queries over up to 64 keys, a workgroup to a CU, the split of the
 // operands costs more than the faster products give, and the FP32 MFMA kernel takes the call (with RoPE, FP32 first:
 // 64 queries of 12 heads of 80 13.2 against 15.6 us, of 8 of 64 11.0 against
@@ -855,29 +891,55 @@ static AttnX3Plan attention_x3_plan(int B, int S, int Sk, int H, int D, int q_po
     const int c = (D + 31) / 32 - 1;
     p.dp = 32 * (c + 1);
     p.qb = p.dp == 128 ? 256 : 128;
-    const int nqb = (S + p.qb - 1) / p.qb;
-    double sum = 0.0;  // key blocks of one head's query blocks
-    int most = 0;
-    for (int i = 0; i < nqb; ++i) {
-        int64_t end = Sk;
-        if (causal)
-            end = std::min<int64_t>(end, std::min<int64_t>((int64_t)(i + 1) * p.qb, S) + q_pos - k_pos);
-        const int n = end > 0 ? (int)((end + kBK - 1) / kBK) : 0;
-        sum += n;
-        most = std::max(most, n);
-    }
+    const AttnBlocks n = attention_blocks(S, Sk, q_pos, k_pos, causal, p.qb);
     const double heads = (double)B * H, slots = (double)per_cu[c] * num_cus;
     const double merge = 2.0 * heads * S * D * 4.0 / 5e6;  // us per split
     double best = 0.0;
-    for (int sp = 1; sp <= 64 && (sp == 1 || sp <= most); sp += sp < 8 ? 1 : sp < 16 ? 2 : 8) {
-        const double longest = (double)((most + sp - 1) / sp + 3) * lone[c];
-        const double all = heads * (sum + 3.0 * sp * nqb) / slots * full[c];
+    for (int sp = 1; sp <= 64 && (sp == 1 || sp <= n.most); sp += sp < 8 ? 1 : sp < 16 ? 2 : 8) {
+        const double longest = (double)((n.most + sp - 1) / sp + 3) * lone[c];
+        const double all = heads * (n.sum + 3.0 * sp * n.nqb) / slots * full[c];
         const double t = std::max(longest, all) + (sp > 1 ? 3.0 + merge * sp : 0.0);
         if (sp == 1 || t < best) {
             best = t;
             p.splits = sp;
         }
     }
+
+    // The FP32 MFMA kernel keeps the calls where it is still the faster: short
+    // queries of many heads at D past 96, whose 256-query workgroups have a CU
+    // each (4096 x 32 heads of 128 over one key 2.6 against 4.3 ms, 64 x 32 of 128
+    // queries 136 against 170 us), and D well under a multiple of 32, whose zero
+    // dims cost as much as others here but less than 16 there (64 x 32 heads of 16,
+    // 512 causal queries 197 against 227 us; 128 queries of 48 51 against 62).
+    // Both are priced, by figures fitted to 2976 calls of every D, 32 to 2048
+    // heads, 1 to 512 queries (each model within 10% as a rule): of the 735 that
+    // were slower here than there by 4% and 0.3 us, 33 still are, and 26 became
+    // slower by as much.  Queries under half a workgroup leave waves idle, which
+    // speeds the others up.
+    static const AttnPrice x3[] = {{1.4, 2.9, 3.0, 0.8, 0.15, 4},
+                                   {1.75, 3.05, 3.0, 0.8, 0.15, 2},
+                                   {2.6, 4.6, 3.0, 0.8, 0.15, 2},
+                                   {4.4, 5.1, 3.0, 0.8, 0.15, 1}};
+    static const AttnPrice fp32[] = {
+        {0.73, 1.22, 1.8, 1.2, 0.85, 2}, {1.46, 2.3, 1.8, 0.45, 0.85, 2},
+        {2.05, 3.2, 1.8, 0.45, 0.85, 2}, {2.2, 4.0, 1.8, 1.2, 0.85, 2},
+        {3.2, 5.4, 1.8, 0.45, 0.85, 2},  {3.65, 6.25, 1.8, 0.45, 0.85, 2},
+        {4.2, 7.2, 1.8, 0.45, 0.85, 2},  {4.75, 8.2, 1.8, 0.45, 0.85, 2}};
+    const double used = std::min(1.0, (double)((S + 31) / 32 * 32) / p.qb);
+    const double sp = p.splits, active = 1.0 - 0.22 * (1.0 - used);
+    AttnPrice kx = x3[c];
+    kx.lone *= active;
+    kx.full *= active;
+    const double here = attention_us(kx, heads, n.sum + kx.pro * (sp - 1) * n.nqb, n.nqb,
+                                     (n.most + p.splits - 1) / p.splits, num_cus) +
+                        (p.splits > 1 ? 3.0 + merge * sp : 0.0);
+    const AttnBlocks n16 = attention_blocks(S, Sk, q_pos, k_pos, causal, kBQ);
+    const double there =
+        attention_us(fp32[(D + 15) / 16 - 1], heads, n16.sum, n16.nqb, n16.most, num_cus);
+    // (past 112 dims and up to a head per CU the price of a lone workgroup here is
+    // too high: 256 heads of 128, 100 queries over 200 keys 32 us against 38)
+    const bool lone_heads = D > 112 && heads <= num_cus;
+    if (there < 0.97 * here && !lone_heads) p = AttnX3Plan{0, 0, 1};
     return p;
 }
 
