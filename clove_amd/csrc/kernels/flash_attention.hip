@@ -955,24 +955,37 @@ void attention_prefill(const float *q, const float *k, const float *v, float *ou
                        const float *q_rope_tab, int tab_pos0, float *ws, int num_cus,
                        hipStream_t s) {
     if (B <= 0 || S <= 0 || H <= 0) return;
-    AttnArgs a{q, k, v, out, B, S, Sk, H, q_pos, k_pos, scale, 0,
-               reinterpret_cast<const float2 *>(q_rope_tab), tab_pos0, D, 1, ws};
     const AttnX3Plan p = attention_x3_plan(B, S, Sk, H, D, q_pos, k_pos, causal, num_cus);
-    if (!p.qb) {
-        a.nqb = (S + kBQ - 1) / kBQ;
-        attention_prefill_general(a, causal, (unsigned)(B * H * a.nqb), s);
-        return;
-    }
-    a.nqb = (S + p.qb - 1) / p.qb;
-    a.splits = p.splits;
-    if (p.dp == 32) launch_x3<32, 4>(a, causal, s);
-    else if (p.dp == 64) launch_x3<64, 4>(a, causal, s);
-    else if (p.dp == 96) launch_x3<96, 4>(a, causal, s);
-    else launch_x3<128, 8>(a, causal, s);
-    if (p.splits > 1) {
-        const int64_t rows = (int64_t)B * S * H, blocks = (rows * (D / 4) + 255) / 256;
-        attention_merge_kernel<<<(unsigned)std::min<int64_t>(blocks, 32 * num_cus), 256, 0, s>>>(
-            ws, out, rows, D, p.splits);
+    AttnArgs a{q, k, v, out, B, S, Sk, H, q_pos, k_pos, scale, 0,
+               reinterpret_cast<const float2 *>(q_rope_tab), tab_pos0, D, p.splits, ws};
+    const int qb = p.qb ? p.qb : kBQ, threads = !p.qb ? 512 : p.dp == 128 ? 512 : 256;
+    a.nqb = (S + qb - 1) / qb;
+    // A grid holds under 2^32 threads: more heads than that go in several launches
+    // of whole batch entries (one entry's heads and queries always fit: past 2^23
+    // workgroups of it, q alone would exceed the memory).
+    const int64_t entry = (int64_t)H * a.nqb * p.splits * threads;
+    const int per_launch =
+        (int)std::min<int64_t>(B, std::max<int64_t>(1, ((1ll << 32) - 1) / entry));
+    for (int b0 = 0; b0 < B; b0 += per_launch) {
+        const size_t qo = (size_t)b0 * S * H * D, ko = (size_t)b0 * Sk * H * D;
+        a.B = std::min(per_launch, B - b0);
+        a.q = q + qo;
+        a.k = k + ko;
+        a.v = v + ko;
+        a.out = out + qo;
+        if (!p.qb) {
+            attention_prefill_general(a, causal, (unsigned)((int64_t)a.B * H * a.nqb), s);
+            continue;
+        }
+        if (p.dp == 32) launch_x3<32, 4>(a, causal, s);
+        else if (p.dp == 64) launch_x3<64, 4>(a, causal, s);
+        else if (p.dp == 96) launch_x3<96, 4>(a, causal, s);
+        else launch_x3<128, 8>(a, causal, s);
+        if (p.splits > 1) {
+            const int64_t rows = (int64_t)a.B * S * H, blocks = (rows * (D / 4) + 255) / 256;
+            attention_merge_kernel<<<(unsigned)std::min<int64_t>(blocks, 32 * num_cus), 256, 0, s>>>(
+                ws, a.out, rows, D, p.splits);
+        }
     }
 }
 

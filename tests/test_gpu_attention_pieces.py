@@ -203,3 +203,15 @@ def test_many_short_heads_take_the_faster_kernel(hip, D, below, B, S):
     got = hip.flash_attention(q, k, v, H, flags=hip.ATTN_CAUSAL).read((B - 1) * S * H * D, S * H * D)
     last = [t.read((B - 1) * S * H * D, S * H * D).reshape(1, S, H * D) for t in (q, k, v)]
     check(got.reshape(1, S, H * D), attention64(*last, H, 0, True), f"D={D} {B}x{S}")
+
+
+def test_more_heads_than_one_grid(hip):
+    """Past 2^23 heads (of one query block each) a launch would hold 2^32
+    threads: they go in several.  One key: every output row is its v."""
+    B, H, D = (1 << 18) + 1, 32, 128
+    q, k, v = (hip.empty((B, 1, H * D)).fill_normal(i) for i in (1, 2, 3))
+    out = hip.flash_attention(q, k, v, H, flags=0)
+    for b in (0, 1, (1 << 18) - 2, (1 << 18) - 1, 1 << 18):
+        assert np.array_equal(out.read(b * H * D, H * D), v.read(b * H * D, H * D)), b
+    del q, k, v, out
+    hip.empty_cache()
