@@ -33,6 +33,7 @@
 // wide for the registers (53248 columns) are read more than once.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <type_traits>
 
@@ -974,6 +975,15 @@ int pick_vpt(int cols) {
 
 bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
+// launch(first row, rows) of the row-per-workgroup kernels, whose grid holds
+// under 2^32 threads: 2^23 rows and more go in several launches.
+constexpr size_t kRowsPerLaunch = 1 << 22;
+template <class F>
+void row_runs(size_t rows, F launch) {
+    for (size_t r0 = 0; r0 < rows; r0 += kRowsPerLaunch)
+        launch(r0, (unsigned)std::min(kRowsPerLaunch, rows - r0));
+}
+
 // launch(P, ODD) with the constants the row-per-workgroup kernels are built
 // for.
 template <class F>
@@ -1019,13 +1029,17 @@ void softmax_rows(const float *x, float *y, size_t rows, size_t cols, hipStream_
     const unsigned grid = (unsigned)((rows + kRowsPerBlock - 1) / kRowsPerBlock);
     const int r = (int)rows, c = (int)cols;
     const bool odd = c % 4 != 0 || !aligned16(x) || !aligned16(y);
-    const unsigned nrows = (unsigned)rows;
     const int p = pick_block_p(c);
     if (p < 0)
-        softmax_loop_kernel<<<nrows, kBlockThreads, 0, s>>>(x, y, c);
+        row_runs(rows, [&](size_t r0, unsigned n) {
+            softmax_loop_kernel<<<n, kBlockThreads, 0, s>>>(x + r0 * cols, y + r0 * cols, c);
+        });
     else if (p > 0)
         with_block_p(p, odd, [&](auto P, auto O) {
-            softmax_block_kernel<P(), O()><<<nrows, kBlockThreads, 0, s>>>(x, y, c);
+            row_runs(rows, [&](size_t r0, unsigned n) {
+                softmax_block_kernel<P(), O()>
+                    <<<n, kBlockThreads, 0, s>>>(x + r0 * cols, y + r0 * cols, c);
+            });
         });
     else
         with_vpt<4>(pick_vpt(c), odd, [&](auto V, auto O) {
@@ -1040,7 +1054,6 @@ void layer_norm_rows(const float *x, const float *gamma, const float *beta, floa
     const int r = (int)rows, c = (int)cols;
     const bool odd = c % 4 != 0 || !aligned16(x) || !aligned16(y) || !aligned16(gamma) ||
                      !aligned16(beta);
-    const unsigned nrows = (unsigned)rows;
     const int vpt = pick_vpt(c), p = pick_block_p(c);
     const size_t lds = 2 * (size_t)(c / 4) * sizeof(cl_f4);
     if (vpt > 0)
@@ -1049,11 +1062,16 @@ void layer_norm_rows(const float *x, const float *gamma, const float *beta, floa
         });
     else if (p > 0)
         with_block_p(p, odd, [&](auto P, auto O) {
-            layer_norm_block_kernel<P(), O()><<<nrows, kBlockThreads, 0, s>>>(x, gamma, beta, y, c,
-                                                                             eps);
+            row_runs(rows, [&](size_t r0, unsigned n) {
+                layer_norm_block_kernel<P(), O()><<<n, kBlockThreads, 0, s>>>(
+                    x + r0 * cols, gamma, beta, y + r0 * cols, c, eps);
+            });
         });
     else
-        layer_norm_loop_kernel<<<nrows, kBlockThreads, 0, s>>>(x, gamma, beta, y, c, eps);
+        row_runs(rows, [&](size_t r0, unsigned n) {
+            layer_norm_loop_kernel<<<n, kBlockThreads, 0, s>>>(x + r0 * cols, gamma, beta,
+                                                               y + r0 * cols, c, eps);
+        });
 }
 
 void softmax_backward_rows(const float *y, const float *dy, float *dx, size_t rows, size_t cols,
@@ -1062,13 +1080,18 @@ void softmax_backward_rows(const float *y, const float *dy, float *dx, size_t ro
     const unsigned grid = (unsigned)((rows + kRowsPerBlock - 1) / kRowsPerBlock);
     const int r = (int)rows, c = (int)cols;
     const bool odd = c % 4 != 0 || !aligned16(y) || !aligned16(dy) || !aligned16(dx);
-    const unsigned nrows = (unsigned)rows;
     const int p = pick_block_p(c);
     if (p < 0)
-        softmax_bw_loop_kernel<<<nrows, kBlockThreads, 0, s>>>(y, dy, dx, c);
+        row_runs(rows, [&](size_t r0, unsigned n) {
+            softmax_bw_loop_kernel<<<n, kBlockThreads, 0, s>>>(y + r0 * cols, dy + r0 * cols,
+                                                               dx + r0 * cols, c);
+        });
     else if (p > 0)
         with_block_p(p, odd, [&](auto P, auto O) {
-            softmax_bw_block_kernel<P(), O()><<<nrows, kBlockThreads, 0, s>>>(y, dy, dx, c);
+            row_runs(rows, [&](size_t r0, unsigned n) {
+                softmax_bw_block_kernel<P(), O()><<<n, kBlockThreads, 0, s>>>(
+                    y + r0 * cols, dy + r0 * cols, dx + r0 * cols, c);
+            });
         });
     else
         with_vpt<4>(pick_vpt(c), odd, [&](auto V, auto O) {
@@ -1084,7 +1107,6 @@ static void cross_entropy_launch(const float *logits, const float *targets, size
     const int r = (int)rows, c = (int)cols;
     const long u = (long)used;
     const bool odd = c % 4 != 0 || !aligned16(logits) || (MODE == 1 && !aligned16(out));
-    const unsigned nrows = (unsigned)rows;
     const int p = pick_block_p(c);
     if (MODE == 0 && !odd && (p == 1 || p == 2)) {
         const unsigned pairs = (unsigned)((rows + 1) / 2);
@@ -1094,13 +1116,20 @@ static void cross_entropy_launch(const float *logits, const float *targets, size
             cross_entropy_rows2_kernel<2><<<pairs, kBlockThreads, 0, s>>>(logits, targets, u, r, c, out, err_flag);
         return;
     }
+    const size_t out_row = MODE == 0 ? 1 : cols;  // floats of `out` per row
     if (p < 0)
-        cross_entropy_loop_kernel<MODE><<<nrows, kBlockThreads, 0, s>>>(
-            logits, targets, u, c, (float)r, grad_loss, out, err_flag);
+        row_runs(rows, [&](size_t r0, unsigned n) {
+            cross_entropy_loop_kernel<MODE><<<n, kBlockThreads, 0, s>>>(
+                logits + r0 * cols, targets + r0, u - (long)r0, c, (float)r, grad_loss,
+                out + r0 * out_row, err_flag);
+        });
     else if (p > 0)
         with_block_p(p, odd, [&](auto P, auto O) {
-            cross_entropy_block_kernel<P(), MODE, O()><<<nrows, kBlockThreads, 0, s>>>(
-                logits, targets, u, r, c, grad_loss, out, err_flag);
+            row_runs(rows, [&](size_t r0, unsigned n) {
+                cross_entropy_block_kernel<P(), MODE, O()><<<n, kBlockThreads, 0, s>>>(
+                    logits + r0 * cols, targets + r0, u - (long)r0, r, c, grad_loss,
+                    out + r0 * out_row, err_flag);
+            });
         });
     else
         with_vpt<4>(pick_vpt(c), odd, [&](auto V, auto O) {

@@ -81,3 +81,31 @@ def test_rows_past_2_31_elements(fresh, op):
             want = oracle.layer_norm(xr, gamma, beta)
             rtol, atol = 1e-4, 1e-5
         assert_close(y.read(r * COLS, COLS).reshape(1, COLS), want, rtol, atol, f"{op} row {r}")
+
+
+@pytest.mark.parametrize("op", ["softmax", "softmax_backward", "cross_entropy_backward"])
+def test_odd_rows_past_one_grid(fresh, op):
+    """2^23 rows and more of an odd width: a workgroup of 512 per row would
+    take 2^32 threads, so they go in several launches."""
+    hip = fresh
+    rows, cols = (1 << 23) + 2, 1029
+    x = hip.empty((rows, cols)).fill_normal(71, 0.0, 2.0)
+    targets = np.arange(rows, dtype=np.int64) % cols
+    if op == "softmax":
+        got, want = hip.softmax(x), oracle.softmax
+    elif op == "softmax_backward":
+        got, want = hip.softmax_backward(x, x), lambda a: oracle.softmax_backward(a, a)
+    else:
+        got = hip.cross_entropy_backward(x, hip.tensor(targets.astype(np.float32)),
+                                         hip.tensor(np.array([rows], np.float32)))
+    for r in (0, 1, 2, (1 << 22) - 1, 1 << 22, (1 << 23) - 1, 1 << 23, rows - 1):
+        xr = x.read(r * cols, cols).reshape(1, cols)
+        if op == "cross_entropy_backward":
+            ref = oracle.cross_entropy_backward(xr, targets[r:r + 1].astype(np.float32), 1.0)
+        else:
+            ref = want(xr)
+        # (softmax_backward of y = dy = x: a sum of 1029 squares of deviation 2)
+        scale = np.abs(ref).max()
+        assert_close(got.read(r * cols, cols).reshape(1, cols), ref, 1e-4, 1e-5 * scale,
+                     f"{op} row {r}")
+    del x, got
