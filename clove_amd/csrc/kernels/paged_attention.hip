@@ -755,8 +755,7 @@ __global__ void __launch_bounds__(kMergeThreads) paged_merge_kernel(PagedArgs a,
     __shared__ float wgt[kMergeParts];
     __shared__ float stat[2][kMergeThreads / 64];
     __shared__ float grp[kMergeThreads * V];
-    const int pair = blockIdx.x;
-    const int b = pair / a.num_heads;
+    const int b = blockIdx.y, pair = b * a.num_heads + (int)blockIdx.x;
     const int D = a.head_dim;
     const int ctx = clamp_ctx(a, b, false);
     const int n_parts = (ctx + a.part_tokens - 1) / a.part_tokens;
@@ -1100,7 +1099,8 @@ void paged_attention(const PagedArgs &a, hipStream_t s) {
     }
     if (a.max_parts > 1) {
         // rows of D + 2 floats start 8-byte aligned when D is even
-        const unsigned pairs = (unsigned)(a.num_seqs * a.num_heads);
+        // (a grid holds under 2^32 threads along each side: heads and sequences apart)
+        const dim3 pairs((unsigned)a.num_heads, (unsigned)a.num_seqs);
         const int nv = a.head_dim % 2 == 0 ? a.head_dim / 2 : a.head_dim;
         int lpg = 16;
         while (lpg < kMergeThreads && lpg < nv) lpg *= 2;

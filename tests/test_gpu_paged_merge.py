@@ -5,7 +5,7 @@ import numpy as np
 import pytest
 
 import oracle
-from conftest import assert_close
+from conftest import assert_close, rng
 from test_gpu_paged import ATOL, RTOL, make, run
 
 pytestmark = pytest.mark.gpu
@@ -49,3 +49,26 @@ def test_one_partition_edge(hip, D, blocks):
     q, kn, vn, kv, bt, cl = make(D + blocks, B, H, D, bs, B * blocks + 1, blocks, ctx)
     want = oracle.paged_attention(q, kn, vn, kv, bt, cl).reshape(B, H * D)
     assert_close(run(hip, q, kn, vn, kv, bt, cl), want, RTOL, ATOL, f"D={D} {blocks} blocks")
+
+
+def test_more_pairs_than_one_grid_side(hip):
+    """2^24 (sequence, head) pairs and more, a workgroup of 256 each: long
+    sequences at both ends match a call of their own, the short ones copy v."""
+    B, H, D, bs, blocks = 65535, 257, 4, 16, 129
+    assert B * H * 256 > 2**32
+    g = rng(3)
+    kv = hip.tensor(g.standard_normal((2, blocks, bs, H, D), dtype=np.float32))
+    long = [0, 1, 300, B - 1]
+    ctx = np.ones(B, np.int32)
+    ctx[long] = [2064, 2050, 2063, 2051]  # past one partition of 2048 tokens
+    bt = np.tile(np.arange(blocks, dtype=np.int32), (B, 1))
+    q = hip.empty((B, H * D)).fill_normal(4)
+    got = hip.paged_attention(q, None, None, kv, hip.tensor(bt, np.int32),
+                              hip.tensor(ctx, np.int32), 0.5)
+    rows = np.stack([q.read(i * H * D, H * D) for i in long])
+    want = hip.paged_attention(hip.tensor(rows), None, None, kv, hip.tensor(bt[long], np.int32),
+                               hip.tensor(ctx[long], np.int32), 0.5).numpy()
+    for i, w in zip(long, want):
+        assert np.max(np.abs(got.read(i * H * D, H * D) - w.ravel())) <= 1e-5, i
+    v0 = kv.read(blocks * bs * H * D, H * D)
+    assert np.array_equal(got.read(2 * H * D, H * D), v0)
