@@ -35,15 +35,19 @@ __device__ __forceinline__ unsigned bf16_pair(float a, float b) {
 }
 
 // Two floats, times 2^24 with SCALE, as one dword of each of the three pieces.
-template <bool SCALE>
+// FUSED takes the first remainder as an FMA of the unscaled value, which frees
+// its register earlier but is a longer instruction (the same value).
+template <bool SCALE, bool FUSED = false>
 __device__ __forceinline__ void split_pair(float a, float b, unsigned *p1, unsigned *p2,
                                            unsigned *p3) {
-    if constexpr (SCALE) {
-        a *= kPieceScale;
-        b *= kPieceScale;
-    }
-    const unsigned h = bf16_pair(a, b);
-    const float ra = a - __uint_as_float(h << 16), rb = b - __uint_as_float(h & 0xffff0000u);
+#pragma clang fp contract(off)
+    const float sa = SCALE ? a * kPieceScale : a, sb = SCALE ? b * kPieceScale : b;
+    const unsigned h = bf16_pair(sa, sb);
+    const auto rest = [](float x, float scaled, unsigned bits) {
+        return SCALE && FUSED ? __builtin_fmaf(x, kPieceScale, -__uint_as_float(bits))
+                              : scaled - __uint_as_float(bits);
+    };
+    const float ra = rest(a, sa, h << 16), rb = rest(b, sb, h & 0xffff0000u);
     const unsigned m = bf16_pair(ra, rb);
     *p1 = h;
     *p2 = m;

@@ -40,7 +40,7 @@ constexpr uint32_t kOutside = 0x80000000u;     // past the end of both operands 
 // 4) & 1) at BK = 16, o ^ ((r >> 2) & 3) at BK = 32: a wave's fragment read
 // (lane l: row l % 32, octet 2 step + l / 32) then touches every bank group
 // once per phase, and so do the KC = false stores.
-template <int R, int BK, int T, bool KC>
+template <int R, int BK, int T, bool KC, bool FUSED>
 struct Operand {
     static constexpr int OPR = BK / 8;  // octets per row
     static constexpr int OCT = R * OPR / T;
@@ -122,7 +122,7 @@ struct Operand {
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 unsigned a, b, c;
-                split_pair<true>(x[u][2 * e], x[u][2 * e + 1], &a, &b, &c);
+                split_pair<true, FUSED>(x[u][2 * e], x[u][2 * e + 1], &a, &b, &c);
                 p[0][e] = a;
                 p[1][e] = b;
                 p[2][e] = c;
@@ -163,8 +163,11 @@ struct Operand {
 template <int BM, int BN, int BK, int WM, int WN, int T, int MINW, bool EPI, bool TA, bool TB>
 __global__ void __launch_bounds__(T) __attribute__((amdgpu_waves_per_eu(MINW)))
 gemm_bf16x3_kernel(GemmArgs g) {
-    using OpA = Operand<BM, BK, T, !TA>;
-    using OpB = Operand<BN, BK, T, TB>;
+    // (128-row tiles take the split's remainder as an FMA: 128 x 4096 x 16384 115
+    // against 119 us, 65536 x 1024 x 256 193 against 198; 4096 x 256 x 16384 the
+    // other way, 206 against 194)
+    using OpA = Operand<BM, BK, T, !TA, BM == 128>;
+    using OpB = Operand<BN, BK, T, TB, BM == 128>;
     constexpr int SA = 3 * OpA::kPiece, STAGE = SA + 3 * OpB::kPiece;  // bytes
     constexpr int IB = WM / 32, JB = WN / 32, WNS = BN / WN;
     static_assert((BM / WM) * (BN / WN) * 64 == T, "the waves cover the tile");
@@ -289,14 +292,20 @@ gemm_bf16x3_kernel(GemmArgs g) {
     step(s, No{}, No{});
 
     // Out of the pieces' range?  An infinite or NaN operand, or one that rounds to
-    // infinity in bf16, always gives a sum that is not finite.
-    bool bad = false;
+    // infinity in bf16, always gives a sum that is not finite, and 0 times that is
+    // NaN: one FMA a sum, between the last slab's MFMAs.
+    float zero[IB];
 #pragma unroll
-    for (int i = 0; i < IB; ++i)
+    for (int i = 0; i < IB; ++i) {
+        zero[i] = 0.0f;
 #pragma unroll
         for (int j = 0; j < JB; ++j)
 #pragma unroll
-            for (int e = 0; e < 16; ++e) bad = bad || !(__builtin_fabsf(acc[i][j][e]) < INFINITY);
+            for (int e = 0; e < 16; ++e) zero[i] = __builtin_fmaf(acc[i][j][e], 0.0f, zero[i]);
+    }
+    bool bad = false;
+#pragma unroll
+    for (int i = 0; i < IB; ++i) bad = bad || zero[i] != 0.0f;
     float unscale = kSumUnscale;
     if (__builtin_expect(__syncthreads_or(bad), 0)) {
         unscale = 1.0f;
@@ -336,6 +345,18 @@ gemm_bf16x3_kernel(GemmArgs g) {
 
     // Accumulator element e of block (i, j) is tile element (r, c) with
     // r = wm0 + 32*i + 8*(e/4) + 4*h + e%4 and c = wn0 + 32*j + l%32.
+    // A row of blocks is unscaled in its registers before its first store (a
+    // product next to each store shares one register, which makes the stores wait
+    // on one another).
+    auto unscale_row = [&](int i) {
+#pragma unroll
+        for (int j = 0; j < JB; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                acc[i][j][e] *= unscale;
+                asm volatile("" : "+v"(acc[i][j][e]));
+            }
+    };
     if (g.splits == 1) {
         float bc[JB];  // per-column bias, loaded before any store
 #pragma unroll
@@ -344,28 +365,32 @@ gemm_bf16x3_kernel(GemmArgs g) {
             bc[j] = EPI && g.epi.bias_mode == GEMM_BIAS_COL && col < N ? g.epi.bias[col] : 0.0f;
         }
 #pragma unroll
-        for (int i = 0; i < IB; ++i)
+        for (int i = 0; i < IB; ++i) {
+            unscale_row(i);
 #pragma unroll
             for (int e = 0; e < 16; ++e)
 #pragma unroll
                 for (int j = 0; j < JB; ++j) {
                     const int row = m0 + wm0 + 32 * i + 8 * (e / 4) + 4 * h + (e % 4);
                     const int col = n0 + wn0 + 32 * j + l32;
-                    float v = acc[i][j][e] * unscale;
+                    float v = acc[i][j][e];
                     if constexpr (EPI) v = epilogue(g.epi, v, row, col, N, &bc[j]);
                     if (row < M && col < N) g.C[(size_t)row * N + col] = v;
                 }
+        }
         return;
     }
     float *part = g.ws + ((size_t)split * g.tiles + tile) * (BM * BN);
 #pragma unroll
-    for (int i = 0; i < IB; ++i)
+    for (int i = 0; i < IB; ++i) {
+        unscale_row(i);
 #pragma unroll
         for (int e = 0; e < 16; ++e)
 #pragma unroll
             for (int j = 0; j < JB; ++j)
                 part[(wm0 + 32 * i + 8 * (e / 4) + 4 * h + (e % 4)) * BN + wn0 + 32 * j + l32] =
-                    acc[i][j][e] * unscale;
+                    acc[i][j][e];
+    }
 }
 
 template <int BM, int BN, int BK, int WM, int WN, int T, int MINW>
