@@ -1589,8 +1589,12 @@ static TileChoice choose_tiles(int M, int N, int K, int num_cus, bool only64 = f
 // each: 1554 x 768 x 3072 fused takes 114 us in 256 x 128 tiles, 78 in 128 x
 // 128, where the product alone takes 65 and 60).  The figures are fitted to 45
 // shapes; the picks were within 14% of the best of 15 (shape, split) pairs
-// measured for each, and most within 5%.
-// max_chain: the longest k range one accumulator may sum.
+// measured for each, and most within 5%.  Eight waves with their 32-deep slabs
+// are for a tile per CU only: past that nothing overlaps their epilogue and their
+// partial last slab (8192 x 16 x 4096 45 us against 26 in 128 x 128 x 16, 4096 x
+// 64 x 4096 28 against 24).
+// max_chain: the longest k range one accumulator may sum; GEMM_X3_NONE if up to
+// 64 splits do not keep to it.
 struct X3Choice {
     int shape, splits;
 };
@@ -1612,14 +1616,15 @@ static X3Choice choose_x3(int M, int N, int K, int num_cus, int max_chain) {
     for (int sh = GEMM_X3_256x128; sh <= GEMM_X3_128x128_W8; ++sh) {
         const int BM = kX3BM[sh], BN = kX3BN[sh], BK = kX3BK[sh], slabs = (K + BK - 1) / BK;
         const int tiles = ((M + BM - 1) / BM) * ((N + BN - 1) / BN);
-        for (int sp = 1; sp <= 32 && (sp == 1 || sp <= slabs / 2); ++sp) {
+        for (int sp = 1; sp <= 64 && (sp == 1 || sp <= slabs / 2); ++sp) {
             const int per = (slabs + sp - 1) / sp, made = (slabs + per - 1) / per;
-            if (per * BK > max_chain && sp < 32 && sp < slabs / 2) continue;
+            if (per * BK > max_chain) continue;
             // workgroups of the fullest XCD over its CUs
             const double u = std::ceil((double)((tiles + 7) / 8) * made / (num_cus / 8.0));
+            if (sh == GEMM_X3_128x128_W8 && u > 1.0) continue;
             double t = 5.0 + per * (BK / 16) * std::max(u * thr[sh], std::ceil(u / slots[sh]) * lat[sh]);
             if (made == 1) t += 0.3 * lane_outputs[sh];
-            else t += 4.0 + (2.0 * made + 1.0) * 4.0 * M * N / 5e6;
+            else t += 4.0 + (2.0 * made * tiles * BM * BN + (double)M * N) * 4.0 / 5e6;
             if (best_t == 0.0 || t < best_t) {
                 best_t = t;
                 best = {sh, made};
@@ -1804,14 +1809,25 @@ GemmPlan gemm_plan(int M, int N, int K, int num_cus, int force_cfg, bool a_align
     // FP32 MFMA tiles stay below that, where launches, the reduce pass and a
     // workgroup's first slab are most of the time (917 x 301 x 624, 0.34
     // GFLOP: 14.6 against 16.5 us; 1912 x 136 x 719 10.9 against 13.7; 1747 x
-    // 1171 x 177, 0.72 GFLOP: 23.1 against 20.2; 4096^3 944 against 640).  A
+    // 1171 x 177, 0.72 GFLOP: 23.1 against 20.2; 4096^3 944 against 610).  They
+    // also stay where 128 x 128 tiles are few: up to half the CUs' number at K <=
+    // 256 (64 x 128 tiles then fill the chip unsplit: 512 x 192 x 4096 11.2
+    // against 17.2 us; 160 tiles 16.3 against 14), and up to a CU in 64 (64
+    // splits of their 64-row tiles read a long K with twice the workgroups: 128 x
+    // 65536 x 128 75 against 88 us, 256 x 16384 x 256 29 against 34; eight tiles
+    // 136 against 107).  Of 687 shapes measured on both, 10 then take 4 to 12%
+    // longer than on the FP32 tiles (K <= 48 into 50000 columns and the like).  A
     // K range of one accumulator is kept to 1.25 times what the FP32 plan
     // would sum in one, which keeps the error below that plan's.
-    if (modeled && 2.0 * M * N * K >= 7e8) {
+    const int64_t tiles128 = (int64_t)((M + 127) / 128) * ((N + 127) / 128);
+    const bool few_tiles = tiles128 <= (K <= 256 ? num_cus / 2 : num_cus / 64);
+    if (modeled && 2.0 * M * N * K >= 7e8 && !few_tiles) {
         const int chain = ((K + 15) / 16 + choice.splits - 1) / choice.splits * 16;
         const X3Choice c = choose_x3(M, N, K, num_cus, chain + chain / 4);
-        plan_x3(p, c.shape, c.splits);
-        return p;
+        if (c.shape != GEMM_X3_NONE) {
+            plan_x3(p, c.shape, c.splits);
+            return p;
+        }
     }
     const bool modeled64 = long_k64 && force_cfg < 0;
     if (modeled64) choice = choose_tiles(M, N, K, num_cus, true);

@@ -185,6 +185,25 @@ def best_ms(hip, call, reps=10):
     return min(times)
 
 
+# The smallest K and the fewest tiles that the plan takes, long K whose C cannot
+# fill the chip, thin C whose K splits would park mostly padding.
+@pytest.mark.parametrize("m,k,n", [(4096, 24, 4096), (8192, 16, 4096), (512, 192, 4096),
+                                   (3000, 200, 700), (128, 32768, 128), (256, 16384, 256),
+                                   (1000, 16384, 64), (40000, 256, 64)])
+def test_planned_edges(hip, m, k, n):
+    """Against float64, to the FP32 MFMA kernel's error: 2.3e-8 sqrt(chain) for
+    the K range that one accumulator sums."""
+    g = rng(m + k + n)
+    a = g.standard_normal((m, k), dtype=np.float32)
+    b = g.standard_normal((k, n), dtype=np.float32)
+    got = hip.matmul(hip.tensor(a), hip.tensor(b)).numpy()
+    rows = np.r_[0:min(m, 300), max(0, m - 20):m]
+    want = a[rows].astype(np.float64) @ b.astype(np.float64)
+    err = np.linalg.norm(got[rows] - want) / np.linalg.norm(want)
+    # (64 splits at most; their sum adds one rounding of each)
+    assert err <= 2.3e-8 * np.sqrt(max(k / 64, min(k, 1280))) + 1e-7, err
+
+
 def test_small_operands_cost_nothing(hip):
     """A tiny value per 256 rows, as softmax and loss gradients hold them, does
     not send its tiles to a second computation (which took 2.6 times as long)."""
@@ -194,3 +213,18 @@ def test_small_operands_cost_nothing(hip):
     for r in range(0, n, 256):
         a.write(r * n + 5, np.array([1e-33, 1e-40], np.float32))
     assert best_ms(hip, lambda: hip.matmul(a, b)) <= 1.3 * plain
+
+
+# Shapes on both sides of 0.7 GFLOP, where the plan first weighs the bf16 pieces:
+# (below, above, most that `above` may take of `below`'s time; the work grows by
+# 1.6, 1.2 and 1.6, bound by C's write in the first and last).
+@pytest.mark.parametrize("below,above,most", [((8192, 10, 4096), (8192, 16, 4096), 1.35),
+                                              ((512, 160, 4096), (512, 192, 4096), 1.35),
+                                              ((300000, 10, 100), (300000, 16, 100), 1.4)])
+def test_no_step_where_the_pieces_begin(hip, below, above, most):
+    """Thin K and few tiles took 1.7 to 2 times as long past the line."""
+    ms = {}
+    for m, k, n in (below, above):
+        a, b = hip.empty((m, k)).fill_normal(1), hip.empty((k, n)).fill_normal(2)
+        ms[m, k, n] = best_ms(hip, lambda: hip.matmul(a, b), 50)
+    assert ms[above] <= most * ms[below], ms
