@@ -176,11 +176,11 @@ __global__ void __launch_bounds__(256) softmax_wave_kernel(const float *__restri
     const int lane = threadIdx.x & 63;
     const long row = (long)blockIdx.x * kRowsPerBlock + (threadIdx.x >> 6);
     if (row >= rows) return;
-    const int nvec = cols >> 2;
+    const int nvec = VPT ? cols >> 2 : 0;
     const float *xr = x + row * (long)cols;
     float *yr = y + row * (long)cols;
-    const bool has_tail = ODD && lane < (cols & 3);  // lane holds element 4 nvec + lane too
-    cl_f4 v[VPT];
+    const bool has_tail = ODD && lane < cols - 4 * nvec;  // lane holds element 4 nvec + lane too
+    cl_f4 v[VPT ? VPT : 1];
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
         const int c = lane + 64 * i;
@@ -229,10 +229,10 @@ __global__ void __launch_bounds__(256) layer_norm_wave_kernel(const float *__res
     const int lane = threadIdx.x & 63;
     const long row = (long)blockIdx.x * kRowsPerBlock + (threadIdx.x >> 6);
     const bool live = row < rows;
-    const int nvec = cols >> 2;
+    const int nvec = VPT ? cols >> 2 : 0;
     const float *xr = x + (live ? row : 0) * (long)cols;
-    const bool has_tail = ODD && live && lane < (cols & 3);
-    cl_f4 v[VPT];
+    const bool has_tail = ODD && live && lane < cols - 4 * nvec;
+    cl_f4 v[VPT ? VPT : 1];
     float s = 0.0f;
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
@@ -248,11 +248,13 @@ __global__ void __launch_bounds__(256) layer_norm_wave_kernel(const float *__res
     using gvec = typename std::conditional<ODD, cl_f4u, cl_f4>::type;
     const gvec *g4 = reinterpret_cast<const gvec *>(gamma);
     const gvec *b4 = reinterpret_cast<const gvec *>(beta);
-    for (int c = threadIdx.x; c < nvec; c += 256) {
-        s_gb[c] = g4[c];
-        s_gb[nvec + c] = b4[c];
+    if (VPT) {
+        for (int c = threadIdx.x; c < nvec; c += 256) {
+            s_gb[c] = g4[c];
+            s_gb[nvec + c] = b4[c];
+        }
+        __syncthreads();
     }
-    __syncthreads();
     if (!live) return;
     float *yr = y + row * (long)cols;
 #pragma unroll
@@ -293,11 +295,11 @@ __global__ void __launch_bounds__(256) softmax_bw_wave_kernel(const float *__res
     const int lane = threadIdx.x & 63;
     const long row = (long)blockIdx.x * kRowsPerBlock + (threadIdx.x >> 6);
     if (row >= rows) return;
-    const int nvec = cols >> 2;
+    const int nvec = VPT ? cols >> 2 : 0;
     const float *yr = y + row * (long)cols, *gr = dy + row * (long)cols;
     float *o = dx + row * (long)cols;
-    const bool has_tail = ODD && lane < (cols & 3);
-    cl_f4 vy[VPT], vg[VPT];
+    const bool has_tail = ODD && lane < cols - 4 * nvec;
+    cl_f4 vy[VPT ? VPT : 1], vg[VPT ? VPT : 1];
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
         const int c = lane + 64 * i;
@@ -339,13 +341,13 @@ __global__ void __launch_bounds__(256) cross_entropy_wave_kernel(
     const int lane = threadIdx.x & 63;
     const long row = (long)blockIdx.x * kRowsPerBlock + (threadIdx.x >> 6);
     if (row >= rows) return;
-    const int nvec = cols >> 2;
+    const int nvec = VPT ? cols >> 2 : 0;
     float *go = MODE == 1 ? out + row * (long)cols : nullptr;
-    const bool has_tail = ODD && lane < (cols & 3);
+    const bool has_tail = ODD && lane < cols - 4 * nvec;
     // The row's loads go out first: read after the target (and a branch on
     // it), they would wait one memory latency per row.
     const float *lr = logits + row * (long)cols;
-    cl_f4 v[VPT];
+    cl_f4 v[VPT ? VPT : 1];
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
         const int c = lane + 64 * i;
@@ -1002,7 +1004,13 @@ void with_block_p(int p, bool odd, F launch) {
     }
 }
 
-// The same for the wave-per-row kernels, up to MAXV vectors per lane.
+// Odd rows of at most a wave's lanes move one element a lane (VPT = 0): two
+// loads of a row, its vectors and its tail, cost more than they carry (softmax
+// backward of [1000000, 7] 119 us against 185, of [1000000, 33] 178 against 210).
+bool one_per_lane(int cols, bool odd) { return odd && cols <= 64; }
+
+// The same for the wave-per-row kernels, up to MAXV vectors per lane (0: one
+// element).
 template <int MAXV, class F>
 void with_vpt(int v, bool odd, F launch) {
     auto go = [&](auto V) {
@@ -1010,6 +1018,7 @@ void with_vpt(int v, bool odd, F launch) {
         else launch(V, std::false_type{});
     };
     switch (v) {
+    case 0: launch(std::integral_constant<int, 0>{}, std::true_type{}); return;
     case 1: go(std::integral_constant<int, 1>{}); return;
     case 2: go(std::integral_constant<int, 2>{}); return;
     case 4: go(std::integral_constant<int, 4>{}); return;
@@ -1042,7 +1051,7 @@ void softmax_rows(const float *x, float *y, size_t rows, size_t cols, hipStream_
             });
         });
     else
-        with_vpt<4>(pick_vpt(c), odd, [&](auto V, auto O) {
+        with_vpt<4>(one_per_lane(c, odd) ? 0 : pick_vpt(c), odd, [&](auto V, auto O) {
             softmax_wave_kernel<V(), O()><<<grid, 256, 0, s>>>(x, y, r, c);
         });
 }
@@ -1057,7 +1066,7 @@ void layer_norm_rows(const float *x, const float *gamma, const float *beta, floa
     const int vpt = pick_vpt(c), p = pick_block_p(c);
     const size_t lds = 2 * (size_t)(c / 4) * sizeof(cl_f4);
     if (vpt > 0)
-        with_vpt<32>(vpt, odd, [&](auto V, auto O) {
+        with_vpt<32>(one_per_lane(c, odd) ? 0 : vpt, odd, [&](auto V, auto O) {
             layer_norm_wave_kernel<V(), O()><<<grid, 256, lds, s>>>(x, gamma, beta, y, r, c, eps);
         });
     else if (p > 0)
@@ -1094,7 +1103,7 @@ void softmax_backward_rows(const float *y, const float *dy, float *dx, size_t ro
             });
         });
     else
-        with_vpt<4>(pick_vpt(c), odd, [&](auto V, auto O) {
+        with_vpt<4>(one_per_lane(c, odd) ? 0 : pick_vpt(c), odd, [&](auto V, auto O) {
             softmax_bw_wave_kernel<V(), O()><<<grid, 256, 0, s>>>(y, dy, dx, r, c);
         });
 }
@@ -1116,6 +1125,16 @@ static void cross_entropy_launch(const float *logits, const float *targets, size
             cross_entropy_rows2_kernel<2><<<pairs, kBlockThreads, 0, s>>>(logits, targets, u, r, c, out, err_flag);
         return;
     }
+    if constexpr (MODE == 0) {
+        // Odd rows a little past the other kernels' 1027 columns: half of a
+        // workgroup of 512 would hold no vector (8192 x 1029 9.2 us against 18.7,
+        // 60000 x 1101 45 against 112).
+        if (odd && p > 0 && c <= 1152) {
+            cross_entropy_wave_kernel<8, 0, true><<<grid, 256, 0, s>>>(logits, targets, u, r, c,
+                                                                       grad_loss, out, err_flag);
+            return;
+        }
+    }
     const size_t out_row = MODE == 0 ? 1 : cols;  // floats of `out` per row
     if (p < 0)
         row_runs(rows, [&](size_t r0, unsigned n) {
@@ -1132,7 +1151,7 @@ static void cross_entropy_launch(const float *logits, const float *targets, size
             });
         });
     else
-        with_vpt<4>(pick_vpt(c), odd, [&](auto V, auto O) {
+        with_vpt<4>(one_per_lane(c, odd) ? 0 : pick_vpt(c), odd, [&](auto V, auto O) {
             cross_entropy_wave_kernel<V(), MODE, O()><<<grid, 256, 0, s>>>(
                 logits, targets, u, r, c, grad_loss, out, err_flag);
         });

@@ -134,3 +134,53 @@ def test_close_softmax_subnormal_entries(hip, cols):
     want = y[top][:, None] * np.exp((x - x[top][:, None]).astype(np.float64))
     assert np.any((want > 0) & (want < 2.0**-127))
     assert np.all(np.abs(y - want) <= 2.5 * 2.0**-23 * want + 1.5 * 2.0**-149)
+
+
+# One element a lane up to 64 columns (aligned widths from an odd address too);
+# the loss's wave kernel up to 1152 columns.
+@pytest.mark.parametrize("cols", [4, 31, 33, 60, 63, 64, 65, 68, 1029, 1031, 1151, 1152, 1153])
+@pytest.mark.parametrize("off", [0, 1])
+def test_narrow_and_loss_edges(hip, cols, off):
+    g = rng(cols + off)
+    rows = 6
+    x = g.normal(0, 2, (rows, cols)).astype(np.float32)
+    t = np.array([cols - 1, 0, cols // 3, 4 * (cols // 4) - 1, cols // 2, max(0, cols - 2)],
+                 np.float32)
+    gam = g.uniform(0.5, 1.5, cols).astype(np.float32)
+    bet = g.uniform(-0.1, 0.1, cols).astype(np.float32)
+    keep = []
+
+    def view(a):
+        buf = hip.tensor(np.concatenate([np.full(off, np.nan, np.float32), a.ravel()]))
+        keep.append(buf)
+        return hip.wrap(buf.device_ptr + 4 * off, a.shape)
+
+    check_rows(hip, view, x, t, gam, bet)
+
+
+def best_ms(hip, call, reps=30):
+    call()
+    times = []
+    for _ in range(4):
+        e0 = hip.event_record()
+        for _ in range(reps):
+            call()
+        times.append(hip.event_elapsed(e0, hip.event_record()))
+        hip.event_reset()
+    return min(times)
+
+
+@pytest.mark.parametrize("op,rows,near,cols", [("softmax_backward", 1000000, 8, 7),
+                                               ("cross_entropy", 60000, 1027, 1029)])
+def test_no_step_at_odd_widths(hip, op, rows, near, cols):
+    """Narrow odd rows take about as long as the aligned width beside them, and
+    the loss no longer past the wave kernel's width than at it (they took 1.4
+    and 2.7 times as long)."""
+    ms = {}
+    for c in (near, cols):
+        x = hip.empty((rows, c)).fill_normal(1)
+        t = hip.tensor(np.arange(rows, dtype=np.float32) % c)
+        call = {"softmax_backward": lambda: hip.softmax_backward(x, x),
+                "cross_entropy": lambda: hip.cross_entropy(x, t)}[op]
+        ms[c] = best_ms(hip, call)
+    assert ms[cols] <= 1.25 * ms[near], ms
