@@ -89,9 +89,9 @@ TensorNode HipBackend::softmax_backward(const TensorNode &y_, const TensorNode &
 
 // backend.rs:1314-1360: grad_a = grad_out . b^T (a's shape, m = prod of a's
 // leading dims), grad_b = a^T . grad_out ([k, n]).  Each product is the MFMA
-// GEMM; where its plan allows (the small path, the bf16-piece tiles, and the
-// 128x128, 128x256 and 64x128 FP32 tilings, split over K or not, whose operand
-// rows hold whole 16-byte pieces) the GEMM reads
+// GEMM; where its plan allows (the small path, the bf16-piece tiles, the 64x128
+// FP32 tiling, split over K or not, whose operand rows hold whole 16-byte pieces,
+// and whole 128x128 FP32 tiles of operands past 2 GiB) the GEMM reads
 // the transposed operand directly (k::gemm_f32_transposed), else it runs on a
 // transposed copy with the same plan.  Both give the same bits.
 // CLOVE_GEMM_TRANSPOSED=0 forces the copies (tests).

@@ -1906,17 +1906,22 @@ bool gemm_f32_transposed(const GemmPlan &p, const float *A, const float *B, floa
         reduce_splits(p, kX3BM[p.x3], kX3BN[p.x3], ws, C, GemmEpilogue{}, s);
         return true;
     }
+    // The FP32 MFMA tiles: 64 x 128 below what the bf16 pieces take, and 128 x 128
+    // for operands of 2 GiB and more.
     if (((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(B)) & 15) != 0) return false;
-    if (p.cfg != CFG_128x256 && p.cfg != CFG_128x128 && p.cfg != CFG_64x128) return false;
+    if (p.cfg != CFG_128x128 && p.cfg != CFG_64x128) return false;
     const GemmArgs g{A, B, C, ws, p.M, p.N, p.K, p.tiles_n, p.k_per_split, p.splits,
                      GemmEpilogue{}, p.tiles, (p.tiles + 7) / 8};
     const dim3 grid((unsigned)(g.per_xcd * 8), (unsigned)p.splits);
-    // split K: each split parks its tile in ws, then the splits are summed in
-    // order (gemm_f32's reduce)
-    auto reduce = [&] {
-        reduce_splits(p, kCfgBM[p.cfg], kCfgBN[p.cfg], ws, C, GemmEpilogue{}, s);
-    };
-    if (!p.interior) {
+    constexpr int ST = dma_stages(128);
+    if (p.cfg == CFG_64x128 && p.interior) {
+        // DMA only: the register-staged kernel has no transposed 64x128 form
+        if (!dma_ok(p, 64, 128)) return false;
+        if (ta)
+            gemm_f32_dma_kernel<64, 128, 16, 32, 64, false, true, false, ST><<<grid, 256, 0, s>>>(g);
+        else
+            gemm_f32_dma_kernel<64, 128, 16, 32, 64, false, false, true, ST><<<grid, 256, 0, s>>>(g);
+    } else if (p.cfg == CFG_64x128) {
         // ragged tiles or a K tail: the DMA kernel's edge form, whose 16-byte
         // pieces need whole quads along each stored row (A^T's M and B's N
         // for ta, K for tb); anything else transposes first
@@ -1925,62 +1930,14 @@ bool gemm_f32_transposed(const GemmPlan &p, const float *A, const float *B, floa
         if ((v && *v && std::atoi(v) == 0) || !rows4 ||
             (uint64_t)p.M * p.K * 4 >= (1ull << 31) || (uint64_t)p.K * p.N * 4 >= (1ull << 31))
             return false;
-        constexpr int ST = dma_stages(128);
-        if (p.cfg == CFG_128x256) {
-            if (ta)
-                gemm_f32_dma_kernel<128, 256, 16, 64, 128, false, true, false, kDmaStages, true>
-                    <<<grid, 256, 0, s>>>(g);
-            else
-                gemm_f32_dma_kernel<128, 256, 16, 64, 128, false, false, true, kDmaStages, true>
-                    <<<grid, 256, 0, s>>>(g);
-        } else if (p.cfg == CFG_64x128) {
-            if (ta)
-                gemm_f32_dma_kernel<64, 128, 16, 32, 64, false, true, false, ST, true>
-                    <<<grid, 256, 0, s>>>(g);
-            else
-                gemm_f32_dma_kernel<64, 128, 16, 32, 64, false, false, true, ST, true>
-                    <<<grid, 256, 0, s>>>(g);
-        } else {
-            if (ta)
-                gemm_f32_dma_kernel<128, 128, 16, 64, 64, false, true, false, ST, true>
-                    <<<grid, 256, 0, s>>>(g);
-            else
-                gemm_f32_dma_kernel<128, 128, 16, 64, 64, false, false, true, ST, true>
-                    <<<grid, 256, 0, s>>>(g);
-        }
-        reduce();
-        return true;
-    }
-    if (p.cfg == CFG_64x128) {
-        // DMA only: the register-staged kernel has no transposed 64x128 form
-        if (!dma_ok(p, 64, 128)) return false;
-        constexpr int ST = dma_stages(128);
         if (ta)
-            gemm_f32_dma_kernel<64, 128, 16, 32, 64, false, true, false, ST><<<grid, 256, 0, s>>>(g);
-        else
-            gemm_f32_dma_kernel<64, 128, 16, 32, 64, false, false, true, ST><<<grid, 256, 0, s>>>(g);
-        reduce();
-        return true;
-    }
-    if (p.cfg == CFG_128x256 && dma_ok(p, 128, 256)) {
-        if (ta)
-            gemm_f32_dma_kernel<128, 256, 16, 64, 128, false, true, false><<<grid, 256, 0, s>>>(g);
-        else
-            gemm_f32_dma_kernel<128, 256, 16, 64, 128, false, false, true><<<grid, 256, 0, s>>>(g);
-    } else if (p.cfg == CFG_128x128 && dma_ok(p, 128, 128)) {
-        constexpr int ST = dma_stages(128);
-        if (ta)
-            gemm_f32_dma_kernel<128, 128, 16, 64, 64, false, true, false, ST><<<grid, 256, 0, s>>>(g);
-        else
-            gemm_f32_dma_kernel<128, 128, 16, 64, 64, false, false, true, ST><<<grid, 256, 0, s>>>(g);
-    } else if (p.cfg == CFG_128x256) {
-        if (ta)
-            gemm_f32_mfma_kernel<128, 256, 16, 64, 128, false, true, false, true, false>
+            gemm_f32_dma_kernel<64, 128, 16, 32, 64, false, true, false, ST, true>
                 <<<grid, 256, 0, s>>>(g);
         else
-            gemm_f32_mfma_kernel<128, 256, 16, 64, 128, false, true, false, false, true>
+            gemm_f32_dma_kernel<64, 128, 16, 32, 64, false, false, true, ST, true>
                 <<<grid, 256, 0, s>>>(g);
     } else {
+        if (!p.interior) return false;
         if (ta)
             gemm_f32_mfma_kernel<128, 128, 16, 64, 64, false, true, false, true, false>
                 <<<grid, 256, 0, s>>>(g);
@@ -1988,7 +1945,9 @@ bool gemm_f32_transposed(const GemmPlan &p, const float *A, const float *B, floa
             gemm_f32_mfma_kernel<128, 128, 16, 64, 64, false, true, false, false, true>
                 <<<grid, 256, 0, s>>>(g);
     }
-    reduce();
+    // split K: each split parks its tile in ws, then the splits are summed in
+    // order (gemm_f32's reduce)
+    reduce_splits(p, kCfgBM[p.cfg], kCfgBN[p.cfg], ws, C, GemmEpilogue{}, s);
     return true;
 }
 

@@ -141,8 +141,8 @@ constexpr int kGemmGroupMax = 8;
 void gemm_f32_grouped(const GemmPlan *plans, const float *const *A, const float *const *B,
                       float *const *C, const GemmEpilogue *epi, int count, hipStream_t s);
 // Picks the tile configuration and K split for a shape.  a_aligned / b_aligned:
-// A / B is 16-byte aligned (the small path needs A aligned, the strip and
-// skinny paths both, as they read them in 8- and 16-byte vectors).
+// A / B is 16-byte aligned (the strip and skinny paths need both, as they read
+// them in 8- and 16-byte vectors; the small path takes another form without).
 // force_cfg >= 0 overrides the
 // configuration and turns the skinny path off; force_skinny takes the skinny
 // path wherever it is legal, with force_skinny_nb (1, 2, 4) /
@@ -159,9 +159,10 @@ void gemm_f32(const GemmPlan &p, const float *A, const float *B, float *C, float
 // [N, K] matrix), read transposed inside the tiled kernel's slab loads: the
 // same bits as transposing first.  ws: p.ws_floats floats when p splits K.
 // Launches nothing and returns false unless exactly one of ta, tb is set and
-// p is a 128x128 or 128x256 tiled plan, or a 64x128 one the DMA kernel takes,
-// with 16-byte aligned operands whose transposed rows hold whole 16-byte
-// pieces where its tiles are ragged; the caller then transposes explicitly.
+// p is a small or bf16-piece plan (any alignment), a 64x128 one the DMA kernel
+// takes with 16-byte aligned operands whose transposed rows hold whole 16-byte
+// pieces where its tiles are ragged, or one of whole 128x128 tiles; the caller
+// then transposes explicitly.
 bool gemm_f32_transposed(const GemmPlan &p, const float *A, const float *B, float *C, float *ws,
                          bool ta, bool tb, hipStream_t s);
 

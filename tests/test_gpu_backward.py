@@ -140,18 +140,16 @@ def test_matmul_backward_4096(hip):
 @pytest.mark.parametrize("m,k,n", [(4096, 4096, 4096), (4096, 1024, 2048), (2048, 4096, 4096),
                                    (2048, 2048, 2048), (2048, 2048, 1024),
                                    (3, 5, 7), (1000, 300, 500),
-                                   # ragged tiles and K tails (edge form of the DMA kernel)
+                                   # ragged tiles and K tails
                                    (4100, 4096, 4100), (4100, 2052, 2052), (2052, 4100, 4104),
-                                   # 64x128 tiles: unsplit, split, ragged with a K tail
+                                   # evenly filled and ragged grids of fewer tiles
                                    (768, 4096, 4096), (1536, 1536, 1536), (3000, 3000, 3000),
                                    (2100, 2100, 2100)])
 def test_matmul_backward_transposed_loads_match_copies(hip, monkeypatch, m, k, n):
-    """Where the plan allows, the backward's GEMMs read b^T / a^T straight
-    from b / a, by buffer->LDS DMA (the default; ragged tiles and K tails
-    included) or through registers (CLOVE_GEMM_DMA=0, interior tiles); the
-    result must be the same bits as transposing first
-    (CLOVE_GEMM_TRANSPOSED=0), and shapes the direct path does not take must
-    give the same bits either way too."""
+    """The backward's GEMMs read b^T / a^T straight from b / a: at most of these
+    sizes on the bf16-piece tiles, 3x5x7 on the small path (CLOVE_GEMM_DMA does
+    not change either).  The result must be the same bits as transposing first
+    (CLOVE_GEMM_TRANSPOSED=0)."""
     g = rng(m + 3 * k + 7 * n)
     a = g.normal(0, 1 / np.sqrt(k), (m, k)).astype(np.float32)
     b = g.normal(0, 1 / np.sqrt(k), (k, n)).astype(np.float32)
@@ -165,6 +163,59 @@ def test_matmul_backward_transposed_loads_match_copies(hip, monkeypatch, m, k, n
     monkeypatch.setenv("CLOVE_GEMM_TRANSPOSED", "0")
     da0, db0 = (t.numpy() for t in hip.matmul_backward(ta, tb, tdc))
     assert np.array_equal(da, da0) and np.array_equal(db, db0)
+
+
+# Gradients on the 64x128 FP32 tiles (under 0.7 GFLOP, past the small path), read
+# by buffer->LDS DMA: grad a and grad b of whole and ragged tiles, unsplit and
+# split over K.
+@pytest.mark.parametrize("m,k,n,which", [(768, 384, 128, "a"), (1000, 260, 100, "a"),
+                                         (768, 384, 192, "a"), (130, 68, 2048, "a"),
+                                         (128, 1024, 384, "b"), (100, 1024, 260, "b"),
+                                         (1536, 192, 128, "b"), (2052, 100, 132, "b"),
+                                         # rows of no whole quads: transposed first
+                                         (1000, 260, 101, "a"), (101, 1023, 260, "b"),
+                                         # over 0.7 GFLOP with few tiles, and split 64 ways
+                                         (512, 4096, 192, "a"), (65536, 128, 128, "b")])
+def test_matmul_backward_fp32_tiles_match_copies(hip, monkeypatch, m, k, n, which):
+    g = rng(m + 3 * k + 7 * n)
+    a = g.normal(0, 1, (m, k)).astype(np.float32)
+    b = g.normal(0, 1, (k, n)).astype(np.float32)
+    dc = g.normal(0, 1, (m, n)).astype(np.float32)
+    ta, tb, tdc = hip.tensor(a), hip.tensor(b), hip.tensor(dc)
+    pick = 0 if which == "a" else 1
+
+    def grad():
+        return hip.matmul_backward(ta, tb, tdc, pick == 0, pick == 1)[pick].numpy()
+
+    got = grad()
+    x, y = (dc, b.T) if which == "a" else (a.T, dc)
+    x, y = x.astype(np.float64), y.astype(np.float64)
+    # one f32 rounding per product and sum of K terms, and the splits' sum
+    bound = (x.shape[1] + 65) * 2.0**-24 * (np.abs(x) @ np.abs(y))
+    assert np.all(np.abs(got - x @ y) <= bound)
+    for env in ("CLOVE_GEMM_TRANSPOSED", "CLOVE_GEMM_DMA"):
+        monkeypatch.setenv(env, "0")
+        assert np.array_equal(got, grad()), env
+        monkeypatch.delenv(env)
+
+
+@pytest.mark.parametrize("m,k,n,which", [(524288, 1024, 128, "b"), (128, 131072, 4096, "a")])
+def test_matmul_backward_past_2_gib(hip, monkeypatch, m, k, n, which):
+    """An operand of 2 GiB, past the buffer loads' offsets: whole 128x128 tiles
+    read it transposed through registers, with the copy's bits."""
+    a, b, dc = (hip.empty(s).fill_normal(i) for i, s in enumerate([(m, k), (k, n), (m, n)]))
+    pick = 0 if which == "a" else 1
+    wants = (pick == 0, pick == 1)
+    got = hip.matmul_backward(a, b, dc, *wants)[pick].numpy()
+    monkeypatch.setenv("CLOVE_GEMM_TRANSPOSED", "0")
+    assert np.array_equal(got, hip.matmul_backward(a, b, dc, *wants)[pick].numpy())
+    if which == "a":  # its last columns are products with the last rows of b
+        x = dc.numpy().astype(np.float64)
+        y = b.read((k - 64) * n, 64 * n).reshape(64, n).astype(np.float64).T
+        err = got[:, -64:] - x @ y
+        assert np.max(np.abs(err)) <= n * 2.0**-24 * np.max(np.abs(x) @ np.abs(y))
+    del a, b, dc
+    hip.empty_cache()
 
 
 # ---- broadcast operand gradient (add / sub backward) -----------------------
