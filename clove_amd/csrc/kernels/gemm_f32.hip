@@ -1818,10 +1818,13 @@ GemmPlan gemm_plan(int M, int N, int K, int num_cus, int force_cfg, bool a_align
     // 136 against 107).  Of 687 shapes measured on both, 10 then take 4 to 12%
     // longer than on the FP32 tiles (K <= 48 into 50000 columns and the like).  A
     // K range of one accumulator is kept to 1.25 times what the FP32 plan
-    // would sum in one, which keeps the error below that plan's.
+    // would sum in one, which keeps the error below that plan's.  Below K = 4 the
+    // error of six products is above that of the one or three f32 products (K = 1
+    // 3.4e-8 against 2.5e-8, the rounding of each output; K = 4 3.2e-8 against
+    // 4.0e-8): those stay on the FP32 tiles too.
     const int64_t tiles128 = (int64_t)((M + 127) / 128) * ((N + 127) / 128);
     const bool few_tiles = tiles128 <= (K <= 256 ? num_cus / 2 : num_cus / 64);
-    if (modeled && 2.0 * M * N * K >= 7e8 && !few_tiles) {
+    if (modeled && 2.0 * M * N * K >= 7e8 && K >= 4 && !few_tiles) {
         const int chain = ((K + 15) / 16 + choice.splits - 1) / choice.splits * 16;
         const X3Choice c = choose_x3(M, N, K, num_cus, chain + chain / 4);
         if (c.shape != GEMM_X3_NONE) {

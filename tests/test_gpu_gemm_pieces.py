@@ -173,6 +173,16 @@ def test_small_operands_keep_every_bit(hip, monkeypatch, cfg):
     assert np.array_equal(hip.matmul(hip.tensor(a), hip.tensor(b)).numpy(), want)
 
 
+def test_outer_product_rounds_once(hip):
+    """K = 1 at a size past 0.7 GFLOP: each output is its product, rounded."""
+    n = 18900
+    a, b = hip.empty((n, 1)).fill_normal(1), hip.empty((1, n)).fill_normal(2)
+    got = hip.matmul(a, b)
+    ah, bh = a.numpy(), b.numpy()
+    for r in (0, 1, 127, 128, 9000, n - 1):
+        assert np.array_equal(got.read(r * n, n), ah[r, 0] * bh[0]), r
+
+
 def best_ms(hip, call, reps=10):
     call()
     times = []
