@@ -340,13 +340,13 @@ __device__ __forceinline__ void attention_f32(const AttnArgs &a, const int q0, c
 // block (3.9 us at D = 128 alone on its CU, 1.8 at D = 64), hence the splits.
 // Error against float64 is below that kernel's (2.9e-7 against 3.7e-7 at 377
 // keys, 5.9e-7 at 1031 keys unsplit, less split).
-//  * q (times scale * log2(e)), k and v go in as 2^24 x; a score's factor of 2^48
-//    comes off in the exponent's FMA, the output's 2^24 at the end.  A workgroup
-//    that ends with a sum that is not finite (an infinity, a NaN, a value of
-//    2^103, a score of 2^79, a v around 2^65 over many keys) computes its queries
-//    again with attention_f32.
-//    Weights are taken relative to 2^-24 of the largest, so that all that f32
-//    holds relative to the largest (down to 2^-126) keep their pieces whole.
+//  * q (times scale * log2(e)), k, the weights and v go in as 2^24 x; a score's
+//    factor of 2^48 comes off in the exponent's FMA, the output's at the end.
+//    (The weights' factor has to be a product: taken into the exponent, 24 more
+//    there costs the subtraction before it five bits, an error of 2e-7 against
+//    8e-8.)  A workgroup that ends with a sum that is not finite (an infinity, a
+//    NaN, a value of 2^103, a score of 2^79, a v around 2^65 over many keys)
+//    computes its queries again with attention_f32.
 template <int D, bool CAUSAL, int NW>
 __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)))
 attention_x3_kernel(AttnArgs a) {
@@ -595,12 +595,10 @@ attention_x3_kernel(AttnArgs a) {
 #pragma unroll
         for (int i = 0; i < 16; ++i) mloc = fmaxf(mloc, s[i]);
         mloc = fmaxf(mloc, __shfl_xor(mloc, 32, 64)) * kSumUnscale;
-        // lazy rescale, as in attention_f32, but m stays 24 below the maximum: a
-        // weight goes up to 2^(24 + kSlack), and one of 2^-126 of the largest is
-        // 2^-102, whose third piece is still no bf16 subnormal
-        constexpr float kSlack = 8.0f, kLift = 24.0f;
-        if (__any(mloc - kLift > m + kSlack)) {
-            const float m_new = fmaxf(m, mloc - kLift);
+        // lazy rescale, as in attention_f32
+        constexpr float kSlack = 8.0f;
+        if (__any(mloc > m + kSlack)) {
+            const float m_new = fmaxf(m, mloc);
             const float alpha = m_new == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m - m_new);
             lsum *= alpha;
 #pragma unroll
@@ -624,7 +622,7 @@ attention_x3_kernel(AttnArgs a) {
                 ps += w0;
                 ps += w1;
                 unsigned x1, x2, x3;
-                split_pair<false>(w0, w1, &x1, &x2, &x3);
+                split_pair<true>(w0, w1, &x1, &x2, &x3);
                 pw[0][e] = x1;
                 pw[1][e] = x2;
                 pw[2][e] = x3;
@@ -668,7 +666,7 @@ attention_x3_kernel(AttnArgs a) {
         attention_f32<D, CAUSAL, T>(a, q0, bh, split, blk0, blk1, reinterpret_cast<float *>(smem));
         return;
     }
-    if (q_ok) attn_store<D, kJ>(a, b, h, query, split, hh, o, m, lsum, kPieceUnscale);
+    if (q_ok) attn_store<D, kJ>(a, b, h, query, split, hh, o, m, lsum, kSumUnscale);
 }
 
 // Adds the key splits of every (row, head): O = sum O_p 2^(m_p - M) / sum l_p

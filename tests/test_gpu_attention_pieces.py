@@ -215,3 +215,16 @@ def test_more_heads_than_one_grid(hip):
         assert np.array_equal(out.read(b * H * D, H * D), v.read(b * H * D, H * D)), b
     del q, k, v, out
     hip.empty_cache()
+
+
+@pytest.mark.parametrize("D,S,Sk,H,most", [(32, 8, 8, 600, 1.3e-7), (64, 16, 16, 600, 2.0e-7),
+                                           (96, 70, 70, 512, 3.4e-7), (64, 1024, 1024, 2, 4e-7),
+                                           (128, 1024, 1024, 2, 5e-7), (128, 8, 8000, 1, 6e-7)])
+def test_error_stays_below_the_fp32_kernels(hip, D, S, Sk, H, most):
+    """The relative 2-norm error over normal data, held to what the FP32 MFMA
+    kernel measures there (1.24e-7, 1.94e-7, 3.35e-7, 6.5e-7, 6.9e-7, 16e-7; the
+    pieces 0.9, 1.5, 2.7, 2.6, 3.5 and 4.2e-7)."""
+    q, k, v = inputs(D + S, 1, S, Sk - S, H, D)
+    got = run(hip, q, k, v, H, Sk - S, False)
+    want = attention64(q, k, v, H, Sk - S, False)
+    assert np.linalg.norm(got - want) / np.linalg.norm(want) <= most
