@@ -1,6 +1,7 @@
 // attention16.h -- the 16-query-per-wave attention prefill kernel on
-// v_mfma_f32_16x16x4_f32 for the head dims that the bf16x3 kernel does not take
-// (flash_attention.hip): past 128, or not a multiple of 8.
+// v_mfma_f32_16x16x4_f32 for what the bf16x3 kernel does not take
+// (flash_attention.hip): head dims past 128 or not a multiple of 8, and calls
+// that run faster here, short queries above all (attention_x3_plan).
 //
 // 8 waves = 128 queries per workgroup, the K and V tiles (32 or 64 keys,
 // double buffered through LDS, one barrier per block) shared by all of them.

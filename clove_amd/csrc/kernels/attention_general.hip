@@ -1,5 +1,6 @@
-// attention_general.hip -- the attention prefill at every head dim the bf16x3
-// kernel (flash_attention.hip) does not take: past 128, or not a multiple of 8.
+// attention_general.hip -- the attention prefill where the bf16x3 kernel
+// (flash_attention.hip) does not take it: every head dim past 128 or not a
+// multiple of 8, and the calls of any head dim that its plan prices as faster here.
 //
 // Clove gives head_dim = dim / num_heads with no restriction (nn.rs:519,
 // nn/attention.rs:47), and the lazy FlashAttention step takes it from the

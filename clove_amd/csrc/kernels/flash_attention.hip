@@ -326,17 +326,19 @@ __device__ __forceinline__ void attention_f32(const AttnArgs &a, const int q0, c
 // whose scores the lane already holds, and the order V is stored in.
 //  * K and V tiles of 32 keys are split once per workgroup on their way into
 //    LDS: K as [key][D], V transposed as [dim][32 keys], in 16-byte octets
-//    whose slots are XOR-permuted so that a wave's fragment reads have no bank
-//    conflicts.  Tile n + 1 (in registers) is split while tile n multiplies,
+//    whose slots are XOR-permuted against bank conflicts in a wave's fragment
+//    reads (0.4 conflict cycles per LDS instruction are left, reads and stores
+//    together).  Tile n + 1 (in registers) is split while tile n multiplies,
 //    its octet stores laid between the MFMAs, and tile n + 2 sets out.
 //  * NW waves share a tile: eight (256 queries) at D = 128, where the split of
 //    a tile is a third of the VALU work of four waves; four below.
 //  * The keys of a query block may be split over workgroups (attention_x3_plan);
 //    attention_merge_kernel then adds the parts.
-// What bounds it: at 4096 queries, 32 heads of 128, the card's power limit
-// (non-causal 1190 us, 1386 TFLOP/s of bf16; causal with RoPE 720-750 us with
-// k's pass, against 1066 for the FP32 MFMA kernel; D = 64 391 against 555, D =
-// 96 and 104 two thirds of theirs); below that, one workgroup's chain per key
+// What bounds it: at 4096 queries, 32 heads of 128, the matrix cores at the clock
+// that the load leaves them (2.0 GHz of 2.39 unprofiled, 65% busy under the
+// counters: non-causal 1170-1220 us, 1350-1410 TFLOP/s of bf16; causal with RoPE
+// 670-690 us with k's pass, against 1066 for the FP32 MFMA kernel; D = 64 391
+// against 555, D = 96 and 104 two thirds of theirs); below that, one workgroup's chain per key
 // block (3.9 us at D = 128 alone on its CU, 1.8 at D = 64), hence the splits.
 // Error against float64 is below that kernel's (2.9e-7 against 3.7e-7 at 377
 // keys, 5.9e-7 at 1031 keys unsplit, less split).
@@ -346,7 +348,8 @@ __device__ __forceinline__ void attention_f32(const AttnArgs &a, const int q0, c
 //    there costs the subtraction before it five bits, an error of 2e-7 against
 //    8e-8.)  A workgroup that ends with a sum that is not finite (an infinity, a
 //    NaN, a value of 2^103, a score of 2^79, a v around 2^65 over many keys)
-//    computes its queries again with attention_f32.
+//    computes its queries again with attention_f32 (4096 causal queries with an
+//    infinity in every head's v 1615 us against 644).
 template <int D, bool CAUSAL, int NW>
 __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)))
 attention_x3_kernel(AttnArgs a) {

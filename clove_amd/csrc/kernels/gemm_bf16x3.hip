@@ -14,7 +14,9 @@
 // Operands go in as 2^24 x (bf16x3.h), which holds every value below 2^103.  One
 // past that, an infinity, a NaN or a sum past 2^79 is not for this scheme: the
 // workgroup that meets one computes its tile again from the f32 values on the
-// FP32 MFMA (redo below), so the result is then what f32 arithmetic gives.
+// FP32 MFMA (redo below), so the result is then what f32 arithmetic gives, and
+// the tile takes 2.6 times as long (4096^3 with an infinity in every tile row
+// 1701 us against 645, 948 on the FP32 tiles).
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -152,14 +154,16 @@ struct Operand {
 // slab; 128 x 128 x 32 with eight waves 0.8 against 0.56 per 16 k).
 //
 // What bounds it: large products run at the card's power limit (4096^3 in 256
-// x 128 tiles, two workgroups per CU: 640-690 us by box against 944-1010 for
-// the FP32 MFMA kernel, 200-214 TFLOP/s of f32, 1290 of bf16; MFMA pipe 71%
-// busy at 1.78 GHz; a large bf16 library product reaches 1321 TFLOP/s on the
+// x 128 tiles, two workgroups per CU: 607-645 us by box against 944-1010 for
+// the FP32 MFMA kernel, 213-226 TFLOP/s of f32, 1360 of bf16; the MFMA pipe 78%
+// busy under the counters, the clock 1.74 GHz of 2.39 in an unprofiled run, where
+// the same launch on zeros keeps 2.39 and takes 435; a large bf16 library product
+// reaches 1321 TFLOP/s on the
 // same card).  Waves of 128 x 64 keep LDS reads at half its rate; 64 x 64
 // waves (128 x 128 tiles, three workgroups per CU) take 738 us there but fill
 // the chip from smaller products; eight 64 x 32 waves on one 128 x 128 tile
 // with 32-deep slabs are quickest where a CU gets a single tile (256 x 4096 x
-// 4096: 61 us against 80).
+// 4096: 56 us against 80).
 template <int BM, int BN, int BK, int WM, int WN, int T, int MINW, bool EPI, bool TA, bool TB>
 __global__ void __launch_bounds__(T) __attribute__((amdgpu_waves_per_eu(MINW)))
 gemm_bf16x3_kernel(GemmArgs g) {

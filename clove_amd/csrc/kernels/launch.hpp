@@ -50,7 +50,9 @@ void transpose(const float *in, float *out, size_t R, size_t C, hipStream_t s);
 
 // flash_attention.hip -- attention prefill and RoPE.  q [B, S, H*D], k, v
 // [B, Sk, H*D], out [B, S, H*D]; D in [1, kAttnMaxHeadDim].  Multiples of 8 up
-// to 128 run on the bf16 matrix cores, every other D on the FP32 MFMA; all four
+// to 128 run on the bf16 matrix cores, every other D, and calls that are faster
+// there (up to 64 queries and keys, short queries of many heads), on the FP32
+// MFMA; all four
 // tensors 16-byte aligned when D % 4 == 0, else 4-byte aligned with a null
 // q_rope_tab (the caller rotates q first).
 constexpr int kAttnMaxHeadDim = 256;

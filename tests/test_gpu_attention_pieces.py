@@ -66,7 +66,7 @@ def test_shapes(hip, D, B, S, past, H, causal):
 @pytest.mark.parametrize("scale_q,scale_k,scale_v", [(1e-33, 1e33, 1), (1e33, 1e-33, 1),
                                                      (1, 1, 1e-36), (1, 1, 1e32)])
 def test_far_scales(hip, D, scale_q, scale_k, scale_v):
-    """Values near the ends of f32's range go through the FP32 MFMA."""
+    """Values near the ends of f32's range, as pieces or on the FP32 MFMA."""
     q, k, v = inputs(D, 1, 150, 40, 2, D)
     q, k, v = (x * np.float32(s) for x, s in zip((q, k, v), (scale_q, scale_k, scale_v)))
     check(run(hip, q, k, v, 2, 40, True), attention64(q, k, v, 2, 40, True), f"D={D}")
@@ -97,6 +97,27 @@ def test_special_values(hip, D, S, past):
     check(got[:, keep], want[:, keep], "dims beside the infinity")
 
 
+# Head dims of the smallest tile; and enough heads that no keys are split.
+@pytest.mark.parametrize("D", [8, 24, 32])
+@pytest.mark.parametrize("scale_q,scale_k,scale_v", [(1e-33, 1e33, 1), (1, 1, 1e-36), (1, 1, 1e32)])
+def test_far_scales_small_tile(hip, D, scale_q, scale_k, scale_v):
+    q, k, v = inputs(D, 1, 600, 40, 3, D)
+    q, k, v = (x * np.float32(s) for x, s in zip((q, k, v), (scale_q, scale_k, scale_v)))
+    check(run(hip, q, k, v, 3, 40, True), attention64(q, k, v, 3, 40, True), f"D={D}")
+
+
+@pytest.mark.parametrize("D", [32, 64, 96, 128])
+@pytest.mark.parametrize("causal", [True, False])
+def test_unsplit_launches(hip, D, causal):
+    B, S, H = 32, 600, 16
+    q, k, v = inputs(D, B, S, 0, H, D)
+    got = run(hip, q, k, v, H, 0, causal)
+    for b, h in ((0, 0), (17, 3), (31, 15)):
+        c = slice(h * D, (h + 1) * D)
+        want = attention64(q[b:b + 1, :, c], k[b:b + 1, :, c], v[b:b + 1, :, c], 1, 0, causal)
+        check(got[b:b + 1, :, c], want, f"D={D} b={b} h={h}")
+
+
 def test_no_visible_key(hip):
     """Queries before every key get zeros, in split and unsplit launches."""
     for S, Sk in ((64, 64), (80, 80), (10, 3000)):
@@ -109,8 +130,8 @@ def test_no_visible_key(hip):
         assert np.array_equal(got[0, S - 4], v[0, 0])
 
 
-# Up to 64 queries and keys run on the FP32 MFMA, one more of either on the
-# bf16 pieces.
+# Up to 64 queries and keys run on the FP32 MFMA, one more of either may run on
+# the bf16 pieces (as priced).
 @pytest.mark.parametrize("D", [8, 64, 80, 104, 128])
 @pytest.mark.parametrize("S,past", [(1, 63), (64, 0), (65, 0), (33, 31), (33, 32), (1, 64)])
 def test_short_calls(hip, D, S, past):

@@ -3,11 +3,12 @@ f32 value), against float64.
 
 Every rounding of the kernel is one of f32 on a partial sum: at most four per
 MFMA step of 16 k and product, six products, so 1.5 per k; and the products it
-leaves out are at most 2^-26 |a b|.  The bound per element is therefore (1.5 K
-+ 1) 2^-24 sum |a b|, or half a subnormal step (2^-150) per rounding where sums
-are subnormal; over a whole random matrix the roundings add as a random
-walk, and the 2-norm error stays below 2.5e-8 sqrt(K) (the FP32 MFMA kernel
-measures 1.8e-8 sqrt(K), this one 1.6e-8).
+leaves out are at most 2^-24 |a b| (two pieces of 2^-8 and 2^-17 each way; the
+data that reaches it is in test_same_sign_and_constant_operands).  The bound per
+element is therefore (1.5 K + 1) 2^-24 sum |a b|, or half a subnormal step
+(2^-150) per rounding where sums are subnormal; over a whole random matrix the
+roundings add as a random walk, and the 2-norm error stays below 2.5e-8 sqrt(K)
+(the FP32 MFMA kernel measures 1.8e-8 sqrt(K), this one 1.6e-8).
 """
 import numpy as np
 import pytest
@@ -105,8 +106,8 @@ def test_pieces_hold_every_bit(hip, monkeypatch, cfg):
 @pytest.mark.parametrize("sa,sb", [(1e-36, 1e30), (1e-33, 1e25), (1e-40, 1e36), (1e-25, 1e-20),
                                    (1e30, 1e-35), (1e18, 1e18)])
 def test_far_scales(hip, monkeypatch, cfg, sa, sb):
-    """Operands near the ends of f32's range, where the bf16 pieces would
-    lose bits: the tile is computed on the FP32 MFMA instead."""
+    """Operands near the ends of f32's range: small ones in pieces of 2^24 x, and
+    past 2^103, or for sums past 2^79, on the FP32 MFMA instead."""
     monkeypatch.setenv("CLOVE_GEMM_CFG", cfg)
     g = rng(9)
     a = (g.standard_normal((200, 96)) * sa).astype(np.float32)
@@ -171,6 +172,38 @@ def test_small_operands_keep_every_bit(hip, monkeypatch, cfg):
     b = (eye[g.permutation(256)] * np.exp2(g.integers(-80, 20, 256))).astype(np.float32)
     want = (a.astype(np.float64) @ b.astype(np.float64)).astype(np.float32)  # rounded once
     assert np.array_equal(hip.matmul(hip.tensor(a), hip.tensor(b)).numpy(), want)
+
+
+@pytest.mark.parametrize("k", [64, 1024, 4096, 16384])
+def test_same_sign_and_constant_operands(hip, monkeypatch, k):
+    """Data whose roundings do not cancel: values in [0, 1), held to the error of
+    the FP32 MFMA tiles, and constants, whose every partial sum rounds alike: the
+    one that makes the most of the products left out, and 12 others, whose
+    root mean square is held to those tiles' as well."""
+    g = rng(k)
+
+    def error(a, b, cfg=None):
+        if cfg:
+            monkeypatch.setenv("CLOVE_GEMM_CFG", cfg)
+        got = hip.matmul(hip.tensor(a), hip.tensor(b)).numpy()[:64].astype(np.float64)
+        monkeypatch.delenv("CLOVE_GEMM_CFG", raising=False)
+        want = a[:64].astype(np.float64) @ b.astype(np.float64)
+        return np.linalg.norm(got - want) / np.linalg.norm(want)
+
+    a, b = g.random((512, k), dtype=np.float32), g.random((k, 512), dtype=np.float32)
+    assert error(a, b, "8") <= 1.1 * error(a, b, "2")
+    worst = np.float32(1 + 2.0**-8 - 2.0**-17)
+    # 2^-24 left out, and the roundings of sums that are half the whole on average
+    chain = min(k, 1024) / 16 * 6  # 16 splits, 6 products a step of 16 k
+    assert error(np.full((512, k), worst), np.full((k, 512), worst), "8") <= 2.0**-24 * (2 + chain / 2)
+    pieces, fp32 = [], []
+    for _ in range(12):
+        x, y = (np.float32(1 + g.random()) for _ in range(2))
+        a, b = np.full((512, k), x), np.full((k, 512), y)
+        pieces.append(error(a, b, "8"))
+        fp32.append(error(a, b, "2"))
+    # (the splits differ, so the bound leaves room for a chain twice as long)
+    assert np.linalg.norm(pieces) <= 2 * np.linalg.norm(fp32) + 1e-7, (pieces, fp32)
 
 
 def test_outer_product_rounds_once(hip):
