@@ -249,3 +249,19 @@ def test_error_stays_below_the_fp32_kernels(hip, D, S, Sk, H, most):
     got = run(hip, q, k, v, H, Sk - S, False)
     want = attention64(q, k, v, H, Sk - S, False)
     assert np.linalg.norm(got - want) / np.linalg.norm(want) <= most
+
+
+@pytest.mark.parametrize("D", [8, 16, 104, 120, 128])
+def test_priced_calls_with_rope(hip, D):
+    """Short calls of many heads, which the plan gives to the FP32 MFMA, with RoPE
+    and a past: the result of rotating q and k first, and float64's."""
+    B, S, past, H = 48, 20, 9, 16
+    q, k, v = inputs(D, B, S, past, H, D)
+    tq, tk, tv = (hip.tensor(x) for x in (q, k, v))
+    got = hip.flash_attention(tq, tk, tv, H, q_pos=past,
+                              flags=hip.ATTN_CAUSAL | hip.ATTN_ROPE).numpy()
+    rq, rk = hip.rope(tq, D, past), hip.rope(tk, D, 0)
+    first = hip.flash_attention(rq, rk, tv, H, q_pos=past, flags=hip.ATTN_CAUSAL).numpy()
+    assert np.array_equal(got, first)
+    want = attention64(rq.numpy()[-2:], rk.numpy()[-2:], v[-2:], H, past, True)
+    check(got[-2:], want, f"D={D}")
