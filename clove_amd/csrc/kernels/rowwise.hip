@@ -298,7 +298,8 @@ __global__ void __launch_bounds__(256) softmax_bw_wave_kernel(const float *__res
     const int nvec = VPT ? cols >> 2 : 0;
     const float *yr = y + row * (long)cols, *gr = dy + row * (long)cols;
     float *o = dx + row * (long)cols;
-    const bool has_tail = ODD && lane < cols - 4 * nvec;
+    constexpr int E = VPT ? 1 : 2;  // elements a lane holds past the vectors, 64 apart
+    const int tail = ODD ? cols - 4 * nvec : 0;
     cl_f4 vy[VPT ? VPT : 1], vg[VPT ? VPT : 1];
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
@@ -307,19 +308,30 @@ __global__ void __launch_bounds__(256) softmax_bw_wave_kernel(const float *__res
         vy[i] = in ? row_load<ODD>(yr, c) : (cl_f4){0.f, 0.f, 0.f, 0.f};
         vg[i] = in ? row_load<ODD>(gr, c) : (cl_f4){0.f, 0.f, 0.f, 0.f};
     }
-    const float ey = has_tail ? yr[4 * nvec + lane] : 0.0f;
-    const float eg = has_tail ? gr[4 * nvec + lane] : 0.0f;
+    float ey[E], eg[E];
+#pragma unroll
+    for (int i = 0; i < E; ++i) {
+        const int c = lane + 64 * i;
+        ey[i] = c < tail ? yr[4 * nvec + c] : 0.0f;
+        eg[i] = c < tail ? gr[4 * nvec + c] : 0.0f;
+    }
     float s = 0.0f;
 #pragma unroll
     for (int i = 0; i < VPT; ++i) s += hsum4(vg[i] * vy[i]);
-    if (ODD) s += eg * ey;
+#pragma unroll
+    for (int i = 0; i < E; ++i)
+        if (ODD) s += eg[i] * ey[i];
     s = wave_sum(s);
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
         const int c = lane + 64 * i;
         if (c < nvec) row_store<ODD>(o, c, vy[i] * (vg[i] - s));
     }
-    if (has_tail) o[4 * nvec + lane] = ey * (eg - s);
+#pragma unroll
+    for (int i = 0; i < E; ++i) {
+        const int c = lane + 64 * i;
+        if (c < tail) o[4 * nvec + c] = ey[i] * (eg[i] - s);
+    }
 }
 
 // Rust's `f32 as usize` saturates: NaN and negative targets read class 0.
@@ -1008,6 +1020,10 @@ void with_block_p(int p, bool odd, F launch) {
 // loads of a row, its vectors and its tail, cost more than they carry (softmax
 // backward of [1000000, 7] 119 us against 185, of [1000000, 33] 178 against 210).
 bool one_per_lane(int cols, bool odd) { return odd && cols <= 64; }
+// The softmax backward, which loads two rows, takes two a lane up to here
+// ([300000, 65] 44 us against 69, 61 for a plain walk of the row; 127 columns 85
+// against 90).
+constexpr int kTwoPerLane = 128;
 
 // The same for the wave-per-row kernels, up to MAXV vectors per lane (0: one
 // element).
@@ -1103,7 +1119,7 @@ void softmax_backward_rows(const float *y, const float *dy, float *dx, size_t ro
             });
         });
     else
-        with_vpt<4>(one_per_lane(c, odd) ? 0 : pick_vpt(c), odd, [&](auto V, auto O) {
+        with_vpt<4>(odd && c <= kTwoPerLane ? 0 : pick_vpt(c), odd, [&](auto V, auto O) {
             softmax_bw_wave_kernel<V(), O()><<<grid, 256, 0, s>>>(y, dy, dx, r, c);
         });
 }

@@ -136,9 +136,10 @@ def test_close_softmax_subnormal_entries(hip, cols):
     assert np.all(np.abs(y - want) <= 2.5 * 2.0**-23 * want + 1.5 * 2.0**-149)
 
 
-# One element a lane up to 64 columns (aligned widths from an odd address too);
+# One element a lane up to 64 columns (aligned widths from an odd address too), two
+# up to 128 in the softmax backward;
 # the loss's wave kernel up to 1152 columns.
-@pytest.mark.parametrize("cols", [4, 31, 33, 60, 63, 64, 65, 68, 1029, 1031, 1151, 1152, 1153])
+@pytest.mark.parametrize("cols", [4, 31, 33, 60, 63, 64, 65, 68, 127, 128, 129, 1029, 1031, 1151, 1152, 1153])
 @pytest.mark.parametrize("off", [0, 1])
 def test_narrow_and_loss_edges(hip, cols, off):
     g = rng(cols + off)
@@ -171,6 +172,7 @@ def best_ms(hip, call, reps=30):
 
 
 @pytest.mark.parametrize("op,rows,near,cols", [("softmax_backward", 1000000, 8, 7),
+                                               ("softmax_backward", 300000, 68, 65),
                                                ("cross_entropy", 60000, 1027, 1029)])
 def test_no_step_at_odd_widths(hip, op, rows, near, cols):
     """Narrow odd rows take about as long as the aligned width beside them, and
